@@ -109,6 +109,11 @@ bws_status launch_cluster_stream(const bws_bitmap* A, const int32_t* slot_row,
 bws_status launch_spmm_stream(const uint32_t* S, const int32_t* slot_row, int64_t M, int64_t K,
                               const float* B, int64_t ldb, int64_t N, float* C, int64_t ldc,
                               float alpha, float beta, hipStream_t s);
+// The FP32 0/1 product of small outputs on the matrix cores, B split exactly
+// into three BF16 parts, in one launch without a workspace (spmm_direct.hip).
+bool spmm_direct_ok(const bws_bitmap* A, int64_t ldb, int64_t N);
+bws_status launch_spmm_direct(const bws_bitmap* A, const float* B, int64_t ldb, int64_t N,
+                              float* C, int64_t ldc, float alpha, float beta, hipStream_t s);
 // The subset-sum product for dense masks (16-row sub-stages, 4-row groups):
 // its 32-row mask stream and the product (mask stream pass included).
 size_t subset_stream_bytes(int64_t M, int64_t K);

@@ -1,0 +1,66 @@
+// split3.hpp — the exact three-way BF16 split of FP32 values behind the
+// matrix-core FP32 products of a 0/1 bitmap (spmm_planes.hip, spmm_direct.hip).
+//
+// An FP32 value has 24 significand bits, a BF16 value 8: b = hi + mid + lo
+// with hi the top 8 bits of b, mid the top 8 of what is left and lo the rest,
+// all three BF16 and without any rounding.  A's entries are 0 or 1, so every
+// product is one of the three parts itself, and A·lo + A·mid + A·hi in FP32
+// accumulators is the FP32 sum of the selected B rows in another order.
+//
+// The matrix unit does not round its sums to nearest, so one accumulator must
+// not take all 3 K / 32 steps: chained like that at K = 4096 and 50% density they
+// were 2.6e-7 of |A|·|B| off, against 9.8e-8 for the vector-add kernel.  The
+// kernels keep the chains of the large parts short (see there); both are closer
+// to the 64-bit product than the vector-add kernels over 1% to 100% density.
+//
+// Range: the parts of |b| in [2^-100, 2^128) are normal BF16 numbers.  Of a
+// smaller b bits may be lost, and an Inf or NaN would spread to the rows that
+// do not select it (0 x Inf).  An output that is not finite or is below 2^-80
+// (for zero: only where some b was tiny) is therefore summed again from A's
+// bits and B in FP32, bit by bit, as the vector-add kernels do.
+#pragma once
+
+#include "mfma_common.hpp"
+
+namespace bws {
+namespace {
+
+constexpr int kPlanes = 3;
+constexpr uint32_t kTinyBits = (127u - 100u) << 23;  // 2^-100
+constexpr float kSmallOut = 0x1p-80f;
+
+// FP32 sum of column `col` of B over the set bits of one row of A, ascending k.
+__device__ __forceinline__ float row_sum(const uint32_t* __restrict__ w, int64_t K,
+                                         const float* __restrict__ bcol, int64_t ldb) {
+  float s = 0.0f;
+  for (int64_t i = 0; i * 32 < K; ++i) {
+    uint32_t m = w[i] & valid_bits(i, K);
+    while (m) {
+      const int c = __clz((int)m);
+      m &= ~wbit(c);
+      s += bcol[(32 * i + c) * ldb];
+    }
+  }
+  return s;
+}
+
+// 0/1 A fragment from a bitmap word (bit-reversed): byte q, bit e -> K slot
+// 8q + e; (z & (0x10001 << 2p)) * (ONE >> 2p) puts ONE (BF16 1.0) into the low
+// half iff bit 2p is set and into the high half iff bit 2p + 1 is.
+__device__ __forceinline__ uint4 a_frag01(uint32_t rw, int q) {
+  const uint32_t x = __builtin_amdgcn_ubfe(rw, 8 * q, 8);
+  const uint32_t z = x | (x << 15);
+  return make_uint4((uint32_t)__umul24(z & 0x00010001u, 0x3F80u),
+                    (uint32_t)__umul24(z & 0x00040004u, 0x3F80u >> 2),
+                    (uint32_t)__umul24(z & 0x00100010u, 0x3F80u >> 4),
+                    (uint32_t)__umul24(z & 0x00400040u, 0x3F80u >> 6));
+}
+
+// x is not to be trusted: not finite, or nonzero and below kSmallOut.
+__device__ __forceinline__ bool out_of_range(float x) {
+  const float m = fabsf(x);
+  return !(m < __builtin_inff()) || (m < kSmallOut && m != 0.0f);
+}
+
+}  // namespace
+}  // namespace bws

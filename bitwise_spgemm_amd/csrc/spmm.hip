@@ -212,6 +212,13 @@ bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t
       ws_ok(workspace, workspace_bytes, subset_stream_bytes(A->rows, A->cols)))
     return launch_spmm_subset(A, static_cast<uint32_t*>(workspace), static_cast<const float*>(B),
                               ldb, N, C, ldc, alpha, beta, stream);
+  // FP32 on a 0/1 A, no plan: small outputs in one launch on the matrix cores
+  const bool f32_auto = precision == BWS_PREC_FP32 && !A->values && A->cols > 0 &&
+                        b_dtype == BWS_DTYPE_F32 &&
+                        (!plan || (plan->kernel == 0 && plan->rows_per_wg == 0));
+  if (f32_auto && spmm_direct_ok(A, ldb, N))
+    return launch_spmm_direct(A, static_cast<const float*>(B), ldb, N, C, ldc, alpha, beta,
+                              stream);
   // FP32 on a 0/1 A with the mask stream in the workspace: the streamed
   // kernel (row masks walked on the scalar unit), for problems that fill the
   // chip with 256 x 256 tiles
