@@ -137,6 +137,7 @@ _SIGS = {
     "bws_cluster_stream": ([_BP, _P, _P, _P, _SZ, _P], _I32),
     "bws_spmm_clustered": ([_BP, _P, _P, _P, _I64, _I64, _P, _I64, _F, _F, _P], _I32),
     "bws_spmm_workspace_size": ([_BP, _I64, _I32, C.POINTER(_Plan)], _SZ),
+    "bws_spmm_best_workspace_size": ([_BP, _I64, _I32, C.POINTER(_Plan)], _SZ),
     "bws_spmm": ([_BP, _P, _I32, _I64, _I64, _P, _I64, _F, _F, _I32, C.POINTER(_Plan), _P, _SZ,
                   _P], _I32),
     "bws_spmm_fp32_noalloc_max_bytes": ([], _SZ),
@@ -684,7 +685,7 @@ def spmm(A: Bitmap, B: torch.Tensor, precision: str = "fp32", alpha: float = 1.0
             raise ValueError("beta != 0 needs `out`")
     s = A.struct()
     pl = None if plan is None else C.byref(plan)
-    wsz = lib().bws_spmm_workspace_size(C.byref(s), N, PRECISION[precision], pl)
+    wsz = lib().bws_spmm_best_workspace_size(C.byref(s), N, PRECISION[precision], pl)
     if (precision in ("bf16", "fp16") and A.values is None and B.dtype != torch.float32
             and (plan is None or plan.mfma_min_bits == 0)):
         wsz = 0  # the workspace would hold a rounded FP32 B: not needed for 16-bit B
@@ -726,7 +727,7 @@ def spmm_tA(AT: Bitmap, dC: torch.Tensor, precision: str = "fp32", alpha: float 
         out = torch.empty((AT.rows, N), dtype=torch.float32, device=dev)
     s = AT.struct()
     pl = None if plan is None else C.byref(plan)
-    wsz = lib().bws_spmm_workspace_size(C.byref(s), N, PRECISION[precision], pl)
+    wsz = lib().bws_spmm_best_workspace_size(C.byref(s), N, PRECISION[precision], pl)
     if precision in ("bf16", "fp16") and AT.values is None and dC.dtype != torch.float32:
         wsz = 0  # the workspace would hold a rounded FP32 dC: not needed for 16-bit dC
     ws = _workspace(wsz, dev) if wsz else None

@@ -36,6 +36,7 @@ HIP_FLAGS = [
 FILE_FLAGS = {
     "spmm_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "spmm_direct.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "spmm_planes.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     # 128 x 128 wave tiles: 256 accumulators live in AGPRs
     "spmm_mfma_big.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=0"],
     "sddmm_mfma_big.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=0"],

@@ -109,11 +109,17 @@ bws_status launch_cluster_stream(const bws_bitmap* A, const int32_t* slot_row,
 bws_status launch_spmm_stream(const uint32_t* S, const int32_t* slot_row, int64_t M, int64_t K,
                               const float* B, int64_t ldb, int64_t N, float* C, int64_t ldc,
                               float alpha, float beta, hipStream_t s);
-// The FP32 0/1 product of small outputs on the matrix cores, B split exactly
-// into three BF16 parts, in one launch without a workspace (spmm_direct.hip).
+// The FP32 0/1 product on the matrix cores, B split exactly into three BF16
+// parts: in one launch for small outputs (spmm_direct.hip), and for outputs
+// that fill the chip, where the mask is dense, over planes of B in a workspace
+// of f32_routed_bytes (spmm_planes.hip; sparse masks take the streamed product).
 bool spmm_direct_ok(const bws_bitmap* A, int64_t ldb, int64_t N);
 bws_status launch_spmm_direct(const bws_bitmap* A, const float* B, int64_t ldb, int64_t N,
                               float* C, int64_t ldc, float alpha, float beta, hipStream_t s);
+size_t f32_routed_bytes(int64_t M, int64_t K, int64_t N);
+bws_status launch_spmm_f32_routed(const bws_bitmap* A, void* ws, const float* B, int64_t ldb,
+                                  int64_t N, float* C, int64_t ldc, float alpha, float beta,
+                                  hipStream_t s);
 // The subset-sum product for dense masks (16-row sub-stages, 4-row groups):
 // its 32-row mask stream and the product (mask stream pass included).
 size_t subset_stream_bytes(int64_t M, int64_t K);
@@ -125,6 +131,8 @@ constexpr int32_t kSubsetKStage = 16;
 // Rows and columns of C per workgroup of the streamed product.
 constexpr int64_t kStreamTileRows = 256;
 constexpr int64_t kStreamTileCols = 256;
+// The fewest such tiles it runs for.
+constexpr int64_t kStreamMinTiles = 192;
 
 // MFMA density split (plan mfma_min_bits > 0, 16-bit precision, 0/1 A): the
 // rows in blocks of kSplitRows; the flags pass (per-block bit counts, a byte

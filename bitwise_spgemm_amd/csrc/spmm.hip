@@ -118,7 +118,7 @@ bool stream_ok(const bws_bitmap* A, const void* B, int64_t ldb, int64_t N, const
                int64_t ldc) {
   if (N < 4 || N % 4 != 0 || ldb % 4 != 0 || ldc % 4 != 0) return false;
   if ((reinterpret_cast<uintptr_t>(B) & 15u) || (reinterpret_cast<uintptr_t>(C) & 15u)) return false;
-  return ceil_div(A->rows, kStreamTileRows) * ceil_div(N, kStreamTileCols) >= 192;
+  return ceil_div(A->rows, kStreamTileRows) * ceil_div(N, kStreamTileCols) >= kStreamMinTiles;
 }
 
 }  // namespace
@@ -183,6 +183,17 @@ size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision
   return spmm_vals_workspace(A);
 }
 
+size_t bws_spmm_best_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision,
+                                    const bws_plan* plan) {
+  if (!A || A->rows <= 0 || A->cols <= 0 || N <= 0 || precision != BWS_PREC_FP32 || A->values ||
+      (plan && (plan->kernel != 0 || plan->rows_per_wg != 0)))
+    return bws_spmm_workspace_size(A, N, precision, plan);
+  if (N % 4 == 0 &&
+      ceil_div(A->rows, kStreamTileRows) * ceil_div(N, kStreamTileCols) >= kStreamMinTiles)
+    return f32_routed_bytes(A->rows, A->cols, N);
+  return 0;  // neither the one-launch product nor the vector-add tiles use one
+}
+
 bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb, int64_t N,
                     float* C, int64_t ldc, float alpha, float beta, int32_t precision,
                     const bws_plan* plan, void* workspace, size_t workspace_bytes,
@@ -219,6 +230,12 @@ bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t
   if (f32_auto && spmm_direct_ok(A, ldb, N))
     return launch_spmm_direct(A, static_cast<const float*>(B), ldb, N, C, ldc, alpha, beta,
                               stream);
+  // and outputs that fill the chip with 256 x 256 tiles by the mask's density,
+  // with room for B's planes in the workspace
+  if (f32_auto && stream_ok(A, B, ldb, N, C, ldc) &&
+      ws_ok(workspace, workspace_bytes, f32_routed_bytes(A->rows, A->cols, N)))
+    return launch_spmm_f32_routed(A, workspace, static_cast<const float*>(B), ldb, N, C, ldc,
+                                  alpha, beta, stream);
   // FP32 on a 0/1 A with the mask stream in the workspace: the streamed
   // kernel (row masks walked on the scalar unit), for problems that fill the
   // chip with 256 x 256 tiles

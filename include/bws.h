@@ -399,6 +399,16 @@ typedef struct {
  * 2062-2248) with the operand roles of a bitmap A and a dense B. */
 size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision,
                                const bws_plan* plan);
+/* The workspace with which bws_spmm has every kernel to choose from: at least
+ * bws_spmm_workspace_size, 0 where none helps.  More than that only at FP32 on a
+ * 0/1 A without a plan, for outputs of at least 192 tiles of 256 x 256 (N % 4 ==
+ * 0): room for B split exactly into three BF16 parts (6 bytes per element), so
+ * that masks with more than one bit in eight run on the matrix cores (at 4096³ a
+ * third to a quarter of the vector kernel's time at 50% density).  The density
+ * is estimated from a fixed sample of A's words on the device: the same A always
+ * takes the same kernel. */
+size_t bws_spmm_best_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision,
+                                    const bws_plan* plan);
 bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb,
                     int64_t N, float* C, int64_t ldc, float alpha, float beta,
                     int32_t precision, const bws_plan* plan, void* workspace,

@@ -1,5 +1,6 @@
 """FP32 products of 0/1 masks on the matrix cores (B split exactly into three
-BF16 parts): the one-launch kernel of small outputs.  Sums of 3 K parts in any order, each addition rounded
+BF16 parts): the one-launch kernel of small outputs and the dense side of the
+density-routed product.  Sums of 3 K parts in any order, each addition rounded
 or truncated to 24 bits, are within 3 K 2^-23 of sum |b|; sums of integers that
 fit 24 bits are exact; a value that is not finite or too small for BF16 parts
 acts on the rows that select it and on no other."""
@@ -53,7 +54,39 @@ def test_direct(bws, dev, M, K, N, p):
     assert torch.equal(bws.spmm(A, Bi).double(), D @ Bi.double())
 
 
-@pytest.mark.parametrize("M,K,N", [(200, 150, 70)])
+# 192 and more tiles of 256 x 256: ragged rows, columns and K; the sparse side
+# (5%) and both sides of the line of one bit in eight
+@pytest.mark.parametrize("M,K,N", [(4096, 33, 3072), (4000, 200, 3000), (3841, 1, 3076)])
+@pytest.mark.parametrize("p", [0.05, 0.11, 0.14, 0.5, 1.0])
+def test_routed(bws, dev, M, K, N, p):
+    A, D = _mask(bws, dev, M, K, p, M + K)
+    g = torch.Generator(device=dev).manual_seed(K)
+    B = torch.randn((K, N), device=dev, generator=g)
+    _check(bws.spmm(A, B), D, B, K)
+    C0 = torch.randn((M, N), device=dev, generator=g)
+    _check(bws.spmm(A, B, alpha=2.0, beta=0.5, out=C0.clone()), D, B, K, 2.0, 0.5, C0)
+    Bi = torch.randint(-1000, 1001, (K, N), device=dev, generator=g).float()
+    assert torch.equal(bws.spmm(A, Bi).double(), D @ Bi.double())
+
+
+def test_routed_small_workspace(bws, dev):
+    """With the mask stream's workspace only, a dense mask takes the streamed
+    kernel; both results are sums of the same integers."""
+    M, K, N = 4096, 100, 3072
+    A, D = _mask(bws, dev, M, K, 0.5, 3)
+    B = torch.randint(-1000, 1001, (K, N), device=dev).float()
+    s = A.struct()
+    L = bws.lib()
+    small = L.bws_spmm_workspace_size(bws.C.byref(s), N, 0, None)
+    assert L.bws_spmm_best_workspace_size(bws.C.byref(s), N, 0, None) > small
+    ws = torch.empty(small, dtype=torch.uint8, device=dev)
+    out = torch.empty((M, N), device=dev)
+    assert L.bws_spmm(bws.C.byref(s), B.data_ptr(), 0, N, N, out.data_ptr(), N, 1.0, 0.0, 0, None,
+                      ws.data_ptr(), small, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out, bws.spmm(A, B)) and torch.equal(out.double(), D @ B.double())
+
+
+@pytest.mark.parametrize("M,K,N", [(200, 150, 70), (4096, 90, 3072)])
 def test_special_values(bws, dev, M, K, N):
     """Columns with an infinity, a NaN, sums that overflow, values below the
     range of the parts (FP32 subnormals among them) and a mixture of tiny and
@@ -84,3 +117,28 @@ def test_special_values(bws, dev, M, K, N):
     assert torch.equal(C[~ok & ~torch.isnan(C)], R32[~ok & ~torch.isnan(C)])
     err = (C.double() - R).abs()[ok]
     assert bool((err <= (3 * K + 4) * 2.0 ** -23 * S[ok] + 2.0 ** -149).all())
+
+
+def test_direct_graph(bws, dev):
+    """Captured with the routed product and replayed with eager work between."""
+    A, _ = _mask(bws, dev, 300, 400, 0.1, 5)
+    A2, _ = _mask(bws, dev, 4096, 64, 0.4, 6)
+    B, B2 = torch.randn((400, 200), device=dev), torch.randn((64, 3072), device=dev)
+    ref, ref2 = bws.spmm(A, B), bws.spmm(A2, B2)
+    out, out2 = torch.empty_like(ref), torch.empty_like(ref2)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(g, stream=s):
+            bws.spmm(A, B, out=out)
+            bws.spmm(A2, B2, out=out2)
+    torch.cuda.current_stream().wait_stream(s)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        out2.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref) and torch.equal(out2, ref2)
+        torch.randn(1 << 20, device=dev).cumsum(0)
+        torch.cuda.synchronize()
