@@ -213,6 +213,35 @@ __device__ __forceinline__ T wave_incl_scan(T v) {
   return v;
 }
 
+// Grouped launches: workgroup b runs on XCD b % 8 and takes slot b / 8 of that
+// XCD.  Every problem gives each XCD an eighth of its tiles (a contiguous range
+// of the column-block-major order, so an XCD's L2 holds few panels of B);
+// slot_off[i] is the first slot of problem i, slot_off[i + 1] - slot_off[i] the
+// largest of its eight shares.  A range of equal tile counts over the whole
+// table, as the single-problem kernels use, gave XCDs up to 1.4 times the mean
+// work where the problems' K differ (32 problems, K 256 to 8192).
+__device__ __forceinline__ bool batch_tile(const BatchEntry* __restrict__ entries,
+                                           const int64_t* __restrict__ slot_off, int count,
+                                           int& problem, int64_t& tile) {
+  const int64_t slot = blockIdx.x >> 3;
+  if (slot >= slot_off[count]) return false;
+  int lo = 0, hi = count;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (slot_off[mid] <= slot) lo = mid;
+    else hi = mid;
+  }
+  problem = lo;
+  const int64_t tiles = entries[lo].row_blocks * entries[lo].col_blocks;
+  const int64_t x = (blockIdx.x + lo) & 7;  // the larger shares go round the XCDs
+  tile = tiles * x / 8 + slot - slot_off[lo];
+  return tile < tiles * (x + 1) / 8;
+}
+// Workgroups of such a launch (every share rounded up to the largest).
+inline int64_t batch_grid(int64_t total_tiles, int count) {
+  return 8 * (total_tiles / 8 + count);
+}
+
 __device__ __forceinline__ uint32_t lo32(uint64_t x) { return (uint32_t)x; }
 __device__ __forceinline__ uint32_t hi32(uint64_t x) { return (uint32_t)(x >> 32); }
 

@@ -456,19 +456,14 @@ k_spmm_mfma4(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
 
 template <int PREC, int WM, int WN, int NBUF, int KS>
 __global__ void __launch_bounds__(256, 2)
-k_spmm_mfma4_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ tile_off,
-                   int count, int64_t per_xcd) {
-  const int64_t g = xcd_tile(blockIdx.x, per_xcd);
-  if (g >= tile_off[count]) return;
-  int lo = 0, hi = count;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (tile_off[mid] <= g) lo = mid;
-    else hi = mid;
-  }
+k_spmm_mfma4_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ slot_off,
+                   int count) {
+  int lo;
+  int64_t tile;
+  if (!batch_tile(entries, slot_off, count, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   mfma4_tile<PREC, WM, WN, NBUF, KS>(e.W, e.M, e.K, e.ldw, static_cast<const uint16_t*>(e.B),
-                                     e.ldb, e.N, e.C, e.ldc, 1.0f, 0.0f, g - tile_off[lo],
+                                     e.ldb, e.N, e.C, e.ldc, 1.0f, 0.0f, tile,
                                      e.row_blocks);
 }
 
@@ -486,19 +481,14 @@ k_spmm_mfma3(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
 
 template <int PREC, int TB, int WM, int WN>
 __global__ void __launch_bounds__(256, 2)
-k_spmm_mfma3_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ tile_off,
-                   int count, int64_t per_xcd, int vec) {
-  const int64_t g = xcd_tile(blockIdx.x, per_xcd);
-  if (g >= tile_off[count]) return;
-  int lo = 0, hi = count;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (tile_off[mid] <= g) lo = mid;
-    else hi = mid;
-  }
+k_spmm_mfma3_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ slot_off,
+                   int count, int vec) {
+  int lo;
+  int64_t tile;
+  if (!batch_tile(entries, slot_off, count, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   mfma3_tile<PREC, TB, WM, WN>(e.W, e.M, e.K, e.ldw, e.B, e.ldb, e.N, e.C, e.ldc, 1.0f, 0.0f,
-                               g - tile_off[lo], e.row_blocks, vec);
+                               tile, e.row_blocks, vec);
 }
 
 template <int PREC, int TB>
@@ -510,24 +500,6 @@ k_spmm_mfma(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
   const int64_t tile = xcd_tile(blockIdx.x, per_xcd);
   if (tile >= row_blocks * col_blocks) return;
   mfma_tile<PREC, TB>(W, M, K, ldw, Bv, ldb, N, C, ldc, alpha, beta, tile, row_blocks, vec);
-}
-
-// Grouped launch over a problem table (see BatchEntry); vec applies to all.
-template <int PREC, int TB>
-__global__ void __launch_bounds__(256, 2)
-k_spmm_mfma_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ tile_off,
-                  int count, int64_t per_xcd, int vec) {
-  const int64_t g = xcd_tile(blockIdx.x, per_xcd);
-  if (g >= tile_off[count]) return;
-  int lo = 0, hi = count;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (tile_off[mid] <= g) lo = mid;
-    else hi = mid;
-  }
-  const BatchEntry& e = entries[lo];
-  mfma_tile<PREC, TB>(e.W, e.M, e.K, e.ldw, e.B, e.ldb, e.N, e.C, e.ldc, 1.0f, 0.0f,
-                      g - tile_off[lo], e.row_blocks, vec);
 }
 
 template <int PREC, int TB>
@@ -624,48 +596,47 @@ bws_status launch_mfma_cfg(const MfmaTile& t, const bws_bitmap* A, const void* B
 }
 
 template <int PREC, int TB, int WM, int WN>
-void launch_mfma3_batch(dim3 grid, const BatchEntry* entries, const int64_t* tile_off, int count,
-                        int64_t per_xcd, int vec, hipStream_t s) {
+void launch_mfma3_batch(dim3 grid, const BatchEntry* entries, const int64_t* slot_off, int count,
+                        int vec, hipStream_t s) {
   hipLaunchKernelGGL((k_spmm_mfma3_batch<PREC, TB, WM, WN>), grid, dim3(256), 0, s, entries,
-                     tile_off, count, per_xcd, vec);
+                     slot_off, count, vec);
 }
 
 template <int PREC, int TB>
-bws_status launch_mfma_batch(const BatchEntry* entries, const int64_t* tile_off, int count,
+bws_status launch_mfma_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
                              int64_t total_tiles, const MfmaTile& t, int vec, hipStream_t s) {
-  const int64_t per_xcd = ceil_div(total_tiles, 8);
-  if (8 * per_xcd > kMaxGrid) return BWS_ECAPACITY;
+  if (batch_grid(total_tiles, count) > kMaxGrid) return BWS_ECAPACITY;
   if (total_tiles == 0) return BWS_OK;
   if (!has_tile<PREC, TB>(t.bm, t.bn)) return BWS_EUNSUPPORTED;
-  const dim3 grid((unsigned)(8 * per_xcd));
+  const dim3 grid((unsigned)batch_grid(total_tiles, count));
   bool done = false;
   if constexpr (TB != 0 && PREC != 3) {
     if (t.dma) {
       if (t.bn == 256)
         hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 64, 128, 2, 64>), grid, dim3(256), 0, s,
-                           entries, tile_off, count, per_xcd);
+                           entries, slot_off, count);
       else if (t.bm == 256)
         hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 128, 64, 2, 64>), grid, dim3(256), 0, s,
-                           entries, tile_off, count, per_xcd);
+                           entries, slot_off, count);
       else
         hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 64, 64, 2, 64>), grid, dim3(256), 0, s,
-                           entries, tile_off, count, per_xcd);
+                           entries, slot_off, count);
       return launch_check();
     }
   }
   if constexpr (has_tile<PREC, TB>(128, 256)) {
     if (t.bn == 256) {
-      launch_mfma3_batch<PREC, TB, 64, 128>(grid, entries, tile_off, count, per_xcd, vec, s);
+      launch_mfma3_batch<PREC, TB, 64, 128>(grid, entries, slot_off, count, vec, s);
       done = true;
     }
   }
   if constexpr (has_tile<PREC, TB>(256, 128)) {
     if (!done && t.bm == 256) {
-      launch_mfma3_batch<PREC, TB, 128, 64>(grid, entries, tile_off, count, per_xcd, vec, s);
+      launch_mfma3_batch<PREC, TB, 128, 64>(grid, entries, slot_off, count, vec, s);
       done = true;
     }
   }
-  if (!done) launch_mfma3_batch<PREC, TB, 64, 64>(grid, entries, tile_off, count, per_xcd, vec, s);
+  if (!done) launch_mfma3_batch<PREC, TB, 64, 64>(grid, entries, slot_off, count, vec, s);
   return launch_check();
 }
 
@@ -719,10 +690,10 @@ bool mfma_tile_valid(int bm, int bn) {
   return (bm == 0 || bm == 128 || bm == 256) && (bn == 0 || bn == 128 || bn == 256);
 }
 
-bws_status spmm_mfma_batch(const BatchEntry* entries, const int64_t* tile_off, int count,
+bws_status spmm_mfma_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
                            int64_t total_tiles, const MfmaTile& t, int32_t b_dtype,
                            int32_t precision, int vec, hipStream_t s) {
-#define BWS_MB(P, T) return launch_mfma_batch<P, T>(entries, tile_off, count, total_tiles, t, vec, s)
+#define BWS_MB(P, T) return launch_mfma_batch<P, T>(entries, slot_off, count, total_tiles, t, vec, s)
   if (precision == BWS_PREC_BF16) {
     if (b_dtype == BWS_DTYPE_BF16) BWS_MB(1, 1);
     if (b_dtype == BWS_DTYPE_F32) BWS_MB(1, 0);

@@ -532,24 +532,18 @@ k_spmm_rows2_groups(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_
                                          0.0f, tile, row_blocks, gt);
 }
 
-// Grouped launch: workgroup g takes global tile xcd_tile(g), finds its problem
-// by binary search over the tile offsets and runs that problem's tile.
+// Grouped launch: a workgroup finds its problem and tile with batch_tile.
 template <int WAVES, int RPW, int KS, bool VALS>
 __global__ void __launch_bounds__(WAVES * 64)
-k_spmm_rows2_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ tile_off,
-                   int count, int64_t per_xcd) {
-  const int64_t g = xcd_tile(blockIdx.x, per_xcd);
-  if (g >= tile_off[count]) return;
-  int lo = 0, hi = count;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (tile_off[mid] <= g) lo = mid;
-    else hi = mid;
-  }
+k_spmm_rows2_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ slot_off,
+                   int count) {
+  int lo;
+  int64_t tile;
+  if (!batch_tile(entries, slot_off, count, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   rows2_tile<WAVES, RPW, KS, VALS>(e.W, e.M, e.K, e.ldw, e.row_ptr, e.values,
                                    static_cast<const float*>(e.B), e.ldb, e.N, e.C, e.ldc, 1.0f,
-                                   0.0f, g - tile_off[lo], e.row_blocks);
+                                   0.0f, tile, e.row_blocks);
 }
 
 // Grouped evaluation: one wave per (row, 256-column block), values from the
@@ -707,25 +701,25 @@ inline int grid_for(int64_t items, int64_t per_block) {
 }
 
 template <int WAVES, int RPW, int KS, bool VALS>
-bws_status launch_rows2_batch(const BatchEntry* entries, const int64_t* tile_off, int count,
+bws_status launch_rows2_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
                               int64_t total_tiles, hipStream_t s) {
-  const int64_t per_xcd = ceil_div(total_tiles, 8);
-  if (8 * per_xcd > kMaxGrid) return BWS_ECAPACITY;
+  const int64_t grid = batch_grid(total_tiles, count);
+  if (grid > kMaxGrid) return BWS_ECAPACITY;
   if (total_tiles == 0) return BWS_OK;
-  hipLaunchKernelGGL((k_spmm_rows2_batch<WAVES, RPW, KS, VALS>), dim3((unsigned)(8 * per_xcd)),
-                     dim3(WAVES * 64), 0, s, entries, tile_off, count, per_xcd);
+  hipLaunchKernelGGL((k_spmm_rows2_batch<WAVES, RPW, KS, VALS>), dim3((unsigned)grid),
+                     dim3(WAVES * 64), 0, s, entries, slot_off, count);
   return launch_check();
 }
 
 }  // namespace
 
 // Grouped vector-add launch (FP32 B meeting the direct-staging conditions).
-bws_status spmm_valu_batch(const BatchEntry* entries, const int64_t* tile_off, int count,
+bws_status spmm_valu_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
                            int64_t total_tiles, const ValuCfg& cfg, bool vals, hipStream_t s) {
 #define BWS_VB(WV, RP, KS)                                                                    \
   if (cfg.waves == WV && cfg.rows == WV * RP && cfg.kstage == KS)                             \
-    return vals ? launch_rows2_batch<WV, RP, KS, true>(entries, tile_off, count, total_tiles, s) \
-                : launch_rows2_batch<WV, RP, KS, false>(entries, tile_off, count, total_tiles, s);
+    return vals ? launch_rows2_batch<WV, RP, KS, true>(entries, slot_off, count, total_tiles, s) \
+                : launch_rows2_batch<WV, RP, KS, false>(entries, slot_off, count, total_tiles, s);
   BWS_VB(8, 32, 64)
   BWS_VB(16, 16, 64)
   BWS_VB(16, 16, 32)
