@@ -672,6 +672,12 @@ def make_plan(kernel: int = 0, rows_per_wg: int = 0, waves_per_wg: int = 0, k_st
                  MFMA_STAGING[mfma_staging], 0)
 
 
+def _rows16(B: torch.Tensor) -> bool:
+    """16-bit rows that the kernels copy as they are (16-byte pieces)."""
+    return (B.dtype != torch.float32 and B.shape[1] % 8 == 0 and B.stride(0) % 8 == 0
+            and B.data_ptr() % 16 == 0)
+
+
 def spmm(A: Bitmap, B: torch.Tensor, precision: str = "fp32", alpha: float = 1.0,
          beta: float = 0.0, out: Optional[torch.Tensor] = None, plan=None) -> torch.Tensor:
     """C = alpha * A·B + beta * C (C FP32, M x N)."""
@@ -686,9 +692,9 @@ def spmm(A: Bitmap, B: torch.Tensor, precision: str = "fp32", alpha: float = 1.0
     s = A.struct()
     pl = None if plan is None else C.byref(plan)
     wsz = lib().bws_spmm_best_workspace_size(C.byref(s), N, PRECISION[precision], pl)
-    if (precision in ("bf16", "fp16") and A.values is None and B.dtype != torch.float32
+    if (precision in ("bf16", "fp16") and A.values is None and _rows16(B)
             and (plan is None or plan.mfma_min_bits == 0)):
-        wsz = 0  # the workspace would hold a rounded FP32 B: not needed for 16-bit B
+        wsz = 0  # the workspace would hold a rounded or padded B: not needed for this one
     ws = _workspace(wsz, dev) if wsz else None
     _check(lib().bws_spmm(C.byref(s), _ptr(B), DTYPE[B.dtype], B.stride(0), N, _ptr(out),
                           out.stride(0), alpha, beta, PRECISION[precision], pl, _ptr(ws),
@@ -728,8 +734,8 @@ def spmm_tA(AT: Bitmap, dC: torch.Tensor, precision: str = "fp32", alpha: float 
     s = AT.struct()
     pl = None if plan is None else C.byref(plan)
     wsz = lib().bws_spmm_best_workspace_size(C.byref(s), N, PRECISION[precision], pl)
-    if precision in ("bf16", "fp16") and AT.values is None and dC.dtype != torch.float32:
-        wsz = 0  # the workspace would hold a rounded FP32 dC: not needed for 16-bit dC
+    if precision in ("bf16", "fp16") and AT.values is None and _rows16(dC):
+        wsz = 0  # the workspace would hold a rounded or padded dC: not needed for this one
     ws = _workspace(wsz, dev) if wsz else None
     _check(lib().bws_spmm_tA(C.byref(s), _ptr(dC), DTYPE[dC.dtype], dC.stride(0), N, _ptr(out),
                              out.stride(0), alpha, beta, PRECISION[precision], pl, _ptr(ws),

@@ -81,15 +81,15 @@ struct Choice {
   bool operator==(const Choice& o) const { return !(*this < o) && !(o < *this); }
 };
 
-// big_batch: the batch's problems fill the chip with 128 x 256 tiles by
-// themselves, so every MFMA problem with N >= 256 takes the tile that is
-// fastest per tile (128 x 256: the grouped 32-problem BF16 workload runs in
-// 2.42 ms with it against 2.66 ms with 128 x 128), whatever tile shape a
-// standalone autotuning chose for it (a problem alone prefers smaller tiles
-// that occupy more CUs); the autotuner's kernel choice and an explicit plan
+// together: the MFMA tile for the batch's outputs as one (mfma_auto_tile).  Where
+// they fill the chip with 128 x 256 tiles by themselves, every MFMA problem with
+// N >= 256 takes that tile, the fastest per tile (the grouped 32-problem BF16
+// workload ran in 2.42 ms with it against 2.66 ms with 128 x 128), whatever tile
+// shape a standalone autotuning chose for it (a problem alone prefers smaller
+// tiles that occupy more CUs); the autotuner's kernel choice and an explicit plan
 // are kept.
 Choice classify(const bws_problem& p, int32_t b_dtype, int32_t precision, const bws_plan* plan,
-                bool big_batch) {
+                const MfmaTile& together) {
   Choice c;
   bws_plan eff{};
   const bool explicit_plan = plan && (plan->kernel || plan->rows_per_wg);
@@ -104,15 +104,21 @@ Choice classify(const bws_problem& p, int32_t b_dtype, int32_t precision, const 
   if (kernel == 2 && p.A.values) kernel = 1;
   if (kernel == 2) {
     c.kind = 2;
+    const bool big_batch = together.bn == 256;
     if (big_batch && !explicit_plan && p.N >= 256)
       c.tile = mfma_tile_for(nullptr, precision, b_dtype, int64_t(1) << 40, p.N);
     else
       c.tile = mfma_tile_for(eff.kernel == 2 ? &eff : nullptr, precision, b_dtype, p.A.rows, p.N);
+    if (eff.kernel != 2 && c.tile.bn != 256 && precision != BWS_PREC_BF16X2) {
+      c.tile.bm = together.bm;
+      c.tile.bn = big_batch ? 128 : together.bn;
+    }
     c.tile.legacy = 0;
     c.tile.nbuf = 2;
     const size_t esz = b_dtype == BWS_DTYPE_F32 ? 4 : 2;
     c.vec = (p.ldb % (int64_t)(16 / esz) == 0) && (reinterpret_cast<uintptr_t>(p.B) % 16 == 0);
     c.tile.dma = c.tile.dma && dma_ok(precision, b_dtype, p.B, p.ldb, p.N);
+    if (!c.tile.dma && c.tile.bm < 128) c.tile.bm = c.tile.bn = 128;
     // 256 x 256 runs as 128 x 256 in a grouped launch: with the per-problem
     // lookup the 128 x 128-per-wave tile exceeds its register budget and
     // spills (the result is the same bit for bit: tiles share the K order)
@@ -182,15 +188,17 @@ bws_status bws_batch_prepare(const bws_problem* problems, int32_t count, int32_t
 
   std::vector<Choice> choice((size_t)count);
   std::vector<int> order;
-  int64_t batch_tiles = 0;  // 128 x 256 tiles of the whole batch
+  int64_t t64 = 0, t256 = 0;  // 64 x 64 and 128 x 256 tiles of the whole batch
   for (int32_t i = 0; i < count; ++i) {
     BWS_TRY(validate_problem(problems[i], b_dtype));
-    batch_tiles += ceil_div(problems[i].A.rows, 128) * ceil_div(problems[i].N, 256);
+    t64 += ceil_div(problems[i].A.rows, 64) * ceil_div(problems[i].N, 64);
+    t256 += ceil_div(problems[i].A.rows, 128) * ceil_div(problems[i].N, 256);
   }
-  const bool big_batch = batch_tiles >= 384;
+  MfmaTile together;
+  mfma_auto_tile(together, t64, t256);
   for (int32_t i = 0; i < count; ++i) {
     if (problems[i].A.rows == 0 || problems[i].N == 0) continue;
-    choice[(size_t)i] = classify(problems[i], b_dtype, precision, plan, big_batch);
+    choice[(size_t)i] = classify(problems[i], b_dtype, precision, plan, together);
     order.push_back(i);
   }
   // within a launch the problems with the longest tiles (K) first, so that the
@@ -303,7 +311,7 @@ bws_status bws_batch_run(const bws_batch* batch, bws_stream stream) {
         const bws_problem& pr = batch->problems[p];
         if (pr.A.rows == 0 || pr.N == 0) continue;
         // (the kind does not depend on the batch size, only the MFMA tile does)
-        if (classify(pr, batch->b_dtype, batch->precision, plan, false).kind != 3) continue;
+        if (classify(pr, batch->b_dtype, batch->precision, plan, MfmaTile{}).kind != 3) continue;
         BWS_TRY(spmm_dispatch(&pr.A, pr.B, batch->b_dtype, pr.ldb, pr.N, pr.C, pr.ldc, 1.0f, 0.0f,
                               batch->precision, plan, stream));
       }

@@ -58,7 +58,8 @@ struct ValuCfg {
 };
 bool valu_cfg_valid(const ValuCfg& c);
 
-// MFMA workgroup tile: bm x bn of C (128 or 256 each); legacy selects the
+// MFMA workgroup tile: bm x bn of C (128 or 256 each, or the direct-to-LDS
+// kernel's small tiles 32 x 64, 64 x 64, 64 x 128); legacy selects the
 // 64 x 64-per-wave kernel with table-lookup A fragments.
 struct MfmaTile {
   int32_t bm = 128;
@@ -72,6 +73,7 @@ struct MfmaTile {
 bool dma_ok(int32_t precision, int32_t b_dtype, const void* B, int64_t ldb, int64_t N);
 MfmaTile mfma_tile_for(const bws_plan* plan, int32_t precision, int32_t b_dtype, int64_t M,
                        int64_t N);
+void mfma_auto_tile(MfmaTile& t, int64_t t64, int64_t t256);
 bool mfma_tile_valid(int bm, int bn);
 
 // One problem of a grouped launch, as the kernels read it from the workspace.

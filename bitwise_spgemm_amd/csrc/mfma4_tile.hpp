@@ -26,21 +26,23 @@ __device__ __forceinline__ uint4 a_frag_bits(uint32_t rw, int q) {
 }
 
 // ---------------------------------------------------------------------------
-// Direct-to-LDS variant for 16-bit B (N and ldb multiples of 8, 16-byte
+// Direct-to-LDS variant for 16-bit B (nb and ldb multiples of 8, 16-byte
 // aligned): no register staging at all.
 //  - B stages of 64 K rows are copied row-major into LDS by
 //    global_load_lds_dwordx4 (each wave instruction writes 1 KiB), NBUF stages
 //    in flight.  Within a row, 32-byte unit c is stored at slot c ^ f(k) with
 //    f(k) = (k & 3) | ((k >> 1) & 4), so the transposing reads below hit 8
-//    different slots (all 64 banks) per 32 lanes.
+//    different slots (all 64 banks) per 32 lanes (64-column tiles have four
+//    units a row and use f(k) & 3).
 //  - B fragments come from ds_read_b64_tr_b16: in each group of 16 lanes, lane
 //    i addresses row kb + i/4, columns n + 4(i%4) .. +3, and receives column
 //    n + i of rows kb .. kb+3; two reads give the 8 K values of an MFMA operand
 //    (K slots 8q .. 8q+7 for lane group q, the same slots the A operand uses).
 //  - bitmap words are copied by global_load_lds_dword (4 bytes per lane);
 //    masking of bits beyond K and the bit reversal happen when they are read.
-// Rows beyond K load row K-1 and columns beyond N load columns N-8..N-1: that
-// data meets zero A bits or is never stored.  B must be finite (0 x Inf = NaN
+// B has nb >= N columns, a multiple of 8 (more than N where it was padded).  Rows
+// beyond K load row K-1 and columns beyond nb load columns nb-8..nb-1: that data
+// meets zero A bits or is never stored.  B must be finite (0 x Inf = NaN
 // in a dense contraction, as in any GEMM).
 // ---------------------------------------------------------------------------
 
@@ -51,9 +53,11 @@ struct Cfg4 {
   static constexpr int ROWB = BN * 2;                    // bytes per B row in LDS
   static constexpr int SB = KS * ROWB;                   // bytes per B stage
   static constexpr int NB_W = SB / 1024 / 4;             // B DMA instructions per wave per stage
-  static constexpr int NA_W = BM * KW / 64 / 4;          // word DMA instructions per wave
+  static constexpr int NA_W = (BM * KW + 255) / 256;     // word DMA instructions per wave,
+  static constexpr int A_L = BM * KW / 4 / NA_W;         // of A_L lanes each
   static constexpr int PER_STAGE = NB_W + NA_W;
-  static constexpr int LANES_PER_ROW = ROWB / 16;        // 32 (BN 256) or 16 (BN 128)
+  static constexpr int LANES_PER_ROW = ROWB / 16;        // 32 (BN 256), 16 (BN 128) or 8 (BN 64)
+  static constexpr int UMASK = (ROWB / 32 - 1) & 7;      // swizzle of the row's 32-byte units
 };
 
 template <int PREC, int WM, int WN, int NBUF, int KS_, bool SKIP = true>
@@ -61,11 +65,11 @@ __device__ __forceinline__ void mfma4_tile(const uint32_t* __restrict__ W, int64
                                            int64_t ldw, const uint16_t* __restrict__ B,
                                            int64_t ldb, int64_t N, float* __restrict__ C,
                                            int64_t ldc, float alpha, float beta, int64_t tile,
-                                           int64_t row_blocks) {
+                                           int64_t row_blocks, int64_t nb) {
   using G = Cfg4<WM, WN, NBUF, KS_>;
   constexpr int BM = G::BM, BN = G::BN, KS = G::KS, KW = G::KW, TM = G::TM, TN = G::TN;
   constexpr int ROWB = G::ROWB, SB = G::SB, NB_W = G::NB_W, NA_W = G::NA_W;
-  constexpr int LPR = G::LANES_PER_ROW;
+  constexpr int LPR = G::LANES_PER_ROW, A_L = G::A_L;
   static_assert(NB_W >= 1 && NA_W >= 1, "stage must give every wave DMA work");
   __shared__ __attribute__((aligned(1024))) uint8_t sB[NBUF][SB];
   __shared__ __attribute__((aligned(256))) uint32_t sA[NBUF][BM * KW];
@@ -89,9 +93,9 @@ __device__ __forceinline__ void mfma4_tile(const uint32_t* __restrict__ W, int64
     const int r = g * (1024 / ROWB) + lane / LPR;  // B row within the stage
     const int u = lane % LPR;                      // 16-byte piece of the LDS row
     const int slot = u >> 1, half = u & 1;
-    const int c = slot ^ ((r & 3) | ((r >> 1) & 4));
+    const int c = slot ^ (((r & 3) | ((r >> 1) & 4)) & G::UMASK);
     int64_t col = n0 + 16 * c + 8 * half;
-    if (col + 8 > N) col = N - 8;
+    if (col + 8 > nb) col = nb - 8;
     bsrc[t] = B + col;
     brow[t] = r;
   }
@@ -99,7 +103,7 @@ __device__ __forceinline__ void mfma4_tile(const uint32_t* __restrict__ W, int64
   int aw[NA_W];
 #pragma unroll
   for (int t = 0; t < NA_W; ++t) {
-    const int idx = (wave * NA_W + t) * 64 + lane;
+    const int idx = (wave * NA_W + t) * A_L + (lane < A_L ? lane : 0);
     int64_t row = m0 + idx / KW;
     if (row > M - 1) row = M - 1;
     asrc[t] = W + row * ldw;
@@ -127,7 +131,8 @@ __device__ __forceinline__ void mfma4_tile(const uint32_t* __restrict__ W, int64
         dma16(bp0[t] + boff, sB0 + (uint32_t)(buf * SB + (wave * NB_W + t) * 1024));
 #pragma unroll
       for (int t = 0; t < NA_W; ++t)
-        dma4(ap0[t] + st * KW, sA0 + (uint32_t)(buf * BM * KW * 4 + (wave * NA_W + t) * 256));
+        if (A_L == 64 || lane < A_L)
+          dma4(ap0[t] + st * KW, sA0 + (uint32_t)((buf * BM * KW + (wave * NA_W + t) * A_L) * 4));
       return;
     }
 #pragma unroll
@@ -140,7 +145,8 @@ __device__ __forceinline__ void mfma4_tile(const uint32_t* __restrict__ W, int64
     for (int t = 0; t < NA_W; ++t) {
       int64_t w = st * KW + aw[t];
       if (w > wpr - 1) w = wpr - 1;
-      dma4(asrc[t] + w, sA0 + (uint32_t)(buf * BM * KW * 4 + (wave * NA_W + t) * 256));
+      if (A_L == 64 || lane < A_L)
+        dma4(asrc[t] + w, sA0 + (uint32_t)((buf * BM * KW + (wave * NA_W + t) * A_L) * 4));
     }
   };
 
@@ -157,7 +163,7 @@ __device__ __forceinline__ void mfma4_tile(const uint32_t* __restrict__ W, int64
   // lane constants of the transposing reads: row 8q + i/4 (+ 4h + 32 ks),
   // 8-byte piece i%4 of the slot
   const int i4 = j >> 2;
-  const int fsw = i4 | ((q & 1) << 2);
+  const int fsw = (i4 | ((q & 1) << 2)) & G::UMASK;
   const uint32_t rd_lane = (uint32_t)((8 * q + i4) * ROWB + 8 * (j & 3));
   const int c0 = (WN * wn) / 16;
 

@@ -54,7 +54,11 @@ ValuCfg plan_valu_cfg(const bws_plan* plan, int64_t M, int64_t N, bool vals) {
 }
 bws_status spmm_mfma(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb, int64_t N,
                      float* C, int64_t ldc, float alpha, float beta, int32_t precision,
-                     const bws_plan* plan, hipStream_t s);
+                     const bws_plan* plan, int64_t nb, hipStream_t s);
+size_t spmm_pad_workspace(int64_t K, int64_t N, int32_t precision);
+bws_status spmm_mfma_padded(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb,
+                            int64_t N, float* C, int64_t ldc, float alpha, float beta,
+                            int32_t precision, void* workspace, hipStream_t s);
 size_t spmm_vals_workspace(const bws_bitmap* A);
 size_t spmm_split_workspace(int64_t K, int64_t N);
 size_t spmm_round_workspace(int64_t K, int64_t N);
@@ -145,7 +149,7 @@ bws_status spmm_dispatch(const bws_bitmap* A, const void* B, int32_t b_dtype, in
   }
   if (kernel == 2) {
     if (A->values) return BWS_EUNSUPPORTED;
-    return spmm_mfma(A, B, b_dtype, ldb, N, C, ldc, alpha, beta, precision, plan, s);
+    return spmm_mfma(A, B, b_dtype, ldb, N, C, ldc, alpha, beta, precision, plan, N, s);
   }
   const ValuCfg cfg = plan_valu_cfg(plan, M, N, A->values != nullptr);
   return spmm_valu(A, B, b_dtype, ldb, N, C, ldc, alpha, beta, cfg, s);
@@ -185,8 +189,12 @@ size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision
 
 size_t bws_spmm_best_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision,
                                     const bws_plan* plan) {
-  if (!A || A->rows <= 0 || A->cols <= 0 || N <= 0 || precision != BWS_PREC_FP32 || A->values ||
-      (plan && (plan->kernel != 0 || plan->rows_per_wg != 0)))
+  if (!A || A->rows <= 0 || A->cols <= 0 || N <= 0 || A->values)
+    return bws_spmm_workspace_size(A, N, precision, plan);
+  if (precision != BWS_PREC_FP32)
+    return plan || N % 8 == 0 ? bws_spmm_workspace_size(A, N, precision, plan)
+                              : spmm_pad_workspace(A->cols, N, precision);
+  if (plan && (plan->kernel != 0 || plan->rows_per_wg != 0))
     return bws_spmm_workspace_size(A, N, precision, plan);
   if (N % 4 == 0 &&
       ceil_div(A->rows, kStreamTileRows) * ceil_div(N, kStreamTileCols) >= kStreamMinTiles)
@@ -293,6 +301,13 @@ bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t
       ws_ok(workspace, workspace_bytes, spmm_round_workspace(A->cols, N)))
     return spmm_mfma_round(A, static_cast<const float*>(B), ldb, N, C, ldc, alpha, beta, precision,
                            plan, workspace, stream);
+  // 16-bit precisions without a plan, B's rows not as the direct copies need
+  // them: with room, B once more in 16 bits with padded rows
+  if (!A->values && A->cols > 0 && !plan && precision != BWS_PREC_FP32 &&
+      (b_dtype == BWS_DTYPE_F32 ? N % 8 != 0 : !dma_ok(precision, b_dtype, B, ldb, N)) &&
+      ws_ok(workspace, workspace_bytes, spmm_pad_workspace(A->cols, N, precision)))
+    return spmm_mfma_padded(A, B, b_dtype, ldb, N, C, ldc, alpha, beta, precision, workspace,
+                            stream);
   // Split-BF16 on a 0/1 A: with room for B's two BF16 planes, split B once and
   // run the direct-to-LDS BF16 kernel twice; otherwise split in registers.
   if (!A->values && A->cols > 0 && precision == BWS_PREC_BF16X2 && (!plan || plan->kernel != 1) &&

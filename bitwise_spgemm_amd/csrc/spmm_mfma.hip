@@ -447,11 +447,11 @@ __global__ void __launch_bounds__(256, 2)
 k_spmm_mfma4(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
              const uint16_t* __restrict__ B, int64_t ldb, int64_t N, float* __restrict__ C,
              int64_t ldc, float alpha, float beta, int64_t row_blocks, int64_t col_blocks,
-             int64_t per_xcd) {
+             int64_t per_xcd, int64_t nb) {
   const int64_t tile = xcd_tile(blockIdx.x, per_xcd);
   if (tile >= row_blocks * col_blocks) return;
   mfma4_tile<PREC, WM, WN, NBUF, KS>(W, M, K, ldw, B, ldb, N, C, ldc, alpha, beta, tile,
-                                     row_blocks);
+                                     row_blocks, nb);
 }
 
 template <int PREC, int WM, int WN, int NBUF, int KS>
@@ -464,7 +464,7 @@ k_spmm_mfma4_batch(const BatchEntry* __restrict__ entries, const int64_t* __rest
   const BatchEntry& e = entries[lo];
   mfma4_tile<PREC, WM, WN, NBUF, KS>(e.W, e.M, e.K, e.ldw, static_cast<const uint16_t*>(e.B),
                                      e.ldb, e.N, e.C, e.ldc, 1.0f, 0.0f, tile,
-                                     e.row_blocks);
+                                     e.row_blocks, e.N);
 }
 
 template <int PREC, int TB, int WM, int WN>
@@ -533,13 +533,14 @@ bws_status launch_mfma3(const bws_bitmap* A, const void* B, int64_t ldb, int64_t
 }
 
 // Tiles built per (precision, B type); mfma_tile_for() only returns these.
-//   16-bit B:        128 x 128, 128 x 256, 256 x 128
+//   16-bit B:        128 x 128, 128 x 256, 256 x 128; 32 x 64, 64 x 64 and
+//                    64 x 128 with direct-to-LDS staging
 //   FP32 B (BF16 / FP16): 128 x 128 (twice the staging registers)
 //   BF16X2:          128 x 128, 256 x 128 (two B planes in LDS)
 template <int PREC, int TB>
 constexpr bool has_tile(int bm, int bn) {
   if (bm == 128 && bn == 128) return true;
-  if (bm == 256 && bn == 256) return PREC != 3 && TB != 0;  // direct-to-LDS only
+  if ((bm == 256 && bn == 256) || bm < 128) return PREC != 3 && TB != 0;  // direct-to-LDS only
   if (PREC == 3) return bm == 256 && bn == 128;
   if (TB == 0) return false;
   return (bm == 128 && bn == 256) || (bm == 256 && bn == 128);
@@ -547,20 +548,20 @@ constexpr bool has_tile(int bm, int bn) {
 
 template <int PREC, int WM, int WN, int NBUF, int KS>
 bws_status launch_mfma4(const bws_bitmap* A, const void* B, int64_t ldb, int64_t N, float* C,
-                        int64_t ldc, float alpha, float beta, hipStream_t s) {
+                        int64_t ldc, float alpha, float beta, int64_t nb, hipStream_t s) {
   const int64_t row_blocks = ceil_div(A->rows, 2 * WM);
   const int64_t col_blocks = ceil_div(N, 2 * WN);
   const int64_t per_xcd = ceil_div(row_blocks * col_blocks, 8);
   if (8 * per_xcd > kMaxGrid) return BWS_ECAPACITY;
   hipLaunchKernelGGL((k_spmm_mfma4<PREC, WM, WN, NBUF, KS>), dim3((unsigned)(8 * per_xcd)), dim3(256),
                      0, s, A->words, A->rows, A->cols, A->ldw, static_cast<const uint16_t*>(B),
-                     ldb, N, C, ldc, alpha, beta, row_blocks, col_blocks, per_xcd);
+                     ldb, N, C, ldc, alpha, beta, row_blocks, col_blocks, per_xcd, nb);
   return launch_check();
 }
 
 template <int PREC, int TB>
 bws_status launch_mfma_cfg(const MfmaTile& t, const bws_bitmap* A, const void* B, int64_t ldb,
-                           int64_t N, float* C, int64_t ldc, float alpha, float beta,
+                           int64_t N, float* C, int64_t ldc, float alpha, float beta, int64_t nb,
                            hipStream_t s) {
   if (t.legacy) return launch_mfma<PREC, TB>(A, B, ldb, N, C, ldc, alpha, beta, s);
   if (!has_tile<PREC, TB>(t.bm, t.bn)) return BWS_EUNSUPPORTED;
@@ -569,7 +570,10 @@ bws_status launch_mfma_cfg(const MfmaTile& t, const bws_bitmap* A, const void* B
       return launch_mfma4_big(PREC == 2 ? BWS_PREC_FP16 : BWS_PREC_BF16, A, B, ldb, N, C, ldc,
                               alpha, beta, s);
     if (t.dma) {
-#define BWS_L4(WM, WN, NB, KS) return launch_mfma4<PREC, WM, WN, NB, KS>(A, B, ldb, N, C, ldc, alpha, beta, s)
+#define BWS_L4(WM, WN, NB, KS) return launch_mfma4<PREC, WM, WN, NB, KS>(A, B, ldb, N, C, ldc, alpha, beta, nb, s)
+      if (t.bm == 32) BWS_L4(16, 32, 2, 128);
+      if (t.bm == 64 && t.bn == 64) BWS_L4(32, 32, 2, 128);
+      if (t.bm == 64) BWS_L4(32, 64, 2, 128);
       if (t.nbuf == 3) {
         if (t.bn == 256) BWS_L4(64, 128, 3, 64);
         if (t.bm == 256) BWS_L4(128, 64, 3, 64);
@@ -612,7 +616,16 @@ bws_status launch_mfma_batch(const BatchEntry* entries, const int64_t* slot_off,
   bool done = false;
   if constexpr (TB != 0 && PREC != 3) {
     if (t.dma) {
-      if (t.bn == 256)
+      if (t.bm == 32)
+        hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 16, 32, 2, 128>), grid, dim3(256), 0, s,
+                           entries, slot_off, count);
+      else if (t.bm == 64 && t.bn == 64)
+        hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 32, 32, 2, 128>), grid, dim3(256), 0, s,
+                           entries, slot_off, count);
+      else if (t.bm == 64)
+        hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 32, 64, 2, 128>), grid, dim3(256), 0, s,
+                           entries, slot_off, count);
+      else if (t.bn == 256)
         hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 64, 128, 2, 64>), grid, dim3(256), 0, s,
                            entries, slot_off, count);
       else if (t.bm == 256)
@@ -650,6 +663,34 @@ bool dma_ok(int32_t precision, int32_t b_dtype, const void* B, int64_t ldb, int6
          ldb % 8 == 0 && (reinterpret_cast<uintptr_t>(B) % 16) == 0;
 }
 
+// The direct-to-LDS tile for an output (or a grouped launch's outputs together)
+// of t64 tiles of 64 x 64 and t256 of 128 x 256: the larger tile when it still
+// gives about 1.5 workgroups per CU (two fit on a CU), and below that the one that
+// keeps every CU's waves busy.  A K stage is a barrier and a copy's latency
+// whatever the tile, so small outputs want many small workgroups and 128-row
+// stages.  Measured BF16 times, us, of 32 x 64 | 64 x 64 | 64 x 128 | 128 x 128:
+//   256 x 512 x 192      (t64 12)     5 |   6 |   8 |  11
+//   1024 x 4096 x 512    (t64 128)   21 |  27 |  34 |  53
+//   1024³                (t64 256)  8.5 | 9.6 |  12 |  18
+//   1999 x 3100 x 1000   (t64 512)   38 |  27 |  31 |  43
+//   4096² x 512          (t64 512)   34 |  30 |  35 |  54
+//   2048³                (t64 1024)  36 |  28 |  26 |  32
+//   1024 x 4096²         (t64 1024)  62 |  46 |  42 |  55
+//   3000 x 700 x 2000    (t64 1504)  29 |  22 |  24 |  19
+//   4096² x 2048         (t64 2048) 119 |  88 |  80 |  66
+// All take the K steps in the same order: the results are the same bits.
+void mfma_auto_tile(MfmaTile& t, int64_t t64, int64_t t256) {
+  t.bm = t.bn = 128;
+  t.ks = 64;
+  if (t256 >= 384) {
+    t.bn = 256;
+  } else if (t64 <= 1280) {
+    t.ks = 128;
+    t.bm = t64 <= 256 ? 32 : 64;
+    t.bn = t64 <= 768 ? 64 : 128;
+  }
+}
+
 MfmaTile mfma_tile_for(const bws_plan* plan, int32_t precision, int32_t b_dtype, int64_t M,
                        int64_t N) {
   MfmaTile t;
@@ -667,13 +708,15 @@ MfmaTile mfma_tile_for(const bws_plan* plan, int32_t precision, int32_t b_dtype,
   int bm = plan && plan->kernel == 2 ? plan->rows_per_wg : 0;
   int bn = plan && plan->kernel == 2 ? plan->cols_per_wg : 0;
   if (bm == 0 || bn == 0) {
-    // the larger tile when it still gives about 1.5 workgroups per CU (two fit
-    // on a CU), else 128 x 128
-    auto tiles = [&](int64_t a, int64_t b) { return ceil_div(M, a) * ceil_div(N, b); };
-    if (tiles(128, 256) >= 384) bm = 128, bn = 256;
-    else bm = 128, bn = 128;
+    MfmaTile best;
+    mfma_auto_tile(best, ceil_div(M, 64) * ceil_div(N, 64), ceil_div(M, 128) * ceil_div(N, 256));
+    // the small tiles exist with direct-to-LDS staging in two stages only
+    if (best.bm < 128 && (!t.dma || t.nbuf != 2)) best.bm = best.bn = 128;
+    if (best.bm < 128) t.ks = best.ks;
+    bm = best.bm, bn = best.bn;
   }
   if (precision == BWS_PREC_BF16X2) {
+    bm = bm < 128 ? 128 : bm;
     bn = 128;  // two B planes
     if (!(plan && plan->kernel == 2 && plan->rows_per_wg) &&
         ceil_div(M, 256) * ceil_div(N, 128) >= 384)
@@ -779,7 +822,7 @@ k_spmm_mfma4_list(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t 
   if (g >= total) return;
   const int64_t rb = list[1 + g % nm], cb = g / nm;
   mfma4_tile<PREC, 64, WN, 2, 64>(W, M, K, ldw, B, ldb, N, C, ldc, alpha, beta,
-                                  cb * row_blocks + rb, row_blocks);
+                                  cb * row_blocks + rb, row_blocks, N);
 }
 
 }  // namespace
@@ -830,17 +873,19 @@ bws_status spmm_mfma_split16(const bws_bitmap* A, const void* B, int32_t precisi
   return launch_check();
 }
 
+// nb: the columns of B that may be read, >= N (more where B was padded).
 bws_status spmm_mfma(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb, int64_t N,
                      float* C, int64_t ldc, float alpha, float beta, int32_t precision,
-                     const bws_plan* plan, hipStream_t s) {
+                     const bws_plan* plan, int64_t nb, hipStream_t s) {
   MfmaTile t = mfma_tile_for(plan, precision, b_dtype, A->rows, N);
-  if (!dma_ok(precision, b_dtype, B, ldb, N)) t.dma = 0;
+  if (!dma_ok(precision, b_dtype, B, ldb, nb)) t.dma = 0;
   if (t.sparse && t.dma && !A->values &&
       ((precision == BWS_PREC_BF16 && b_dtype == BWS_DTYPE_BF16) ||
        (precision == BWS_PREC_FP16 && b_dtype == BWS_DTYPE_F16)))
     return launch_smfmac(precision, A, B, ldb, N, C, ldc, alpha, beta, s);
-  if (!t.dma && t.bm == 256 && t.bn == 256) t.bm = 128;  // 256 x 256 needs the direct copy
-#define BWS_M(P, T) return launch_mfma_cfg<P, T>(t, A, B, ldb, N, C, ldc, alpha, beta, s)
+  if (!t.dma && t.bm == 256 && t.bn == 256) t.bm = 128;  // 256 x 256 and the small tiles
+  if (!t.dma && t.bm < 128) t.bm = t.bn = 128;           // need the direct copy
+#define BWS_M(P, T) return launch_mfma_cfg<P, T>(t, A, B, ldb, N, C, ldc, alpha, beta, nb, s)
   if (precision == BWS_PREC_BF16) {
     if (b_dtype == BWS_DTYPE_BF16) BWS_M(1, 1);
     if (b_dtype == BWS_DTYPE_F32) BWS_M(1, 0);
@@ -914,7 +959,69 @@ k_round_b16(const float* __restrict__ B, int64_t K, int64_t N, int64_t ldb,
   }
 }
 
+// B's rows as 16-bit values at a multiple of 8 columns (zeros past N), four
+// columns per thread: MODE 0 copies 16-bit values, 1 and 2 round FP32 to BF16 and
+// FP16 (as k_round_b16), 3 splits FP32 into hi and lo (as k_split_bf16x2).  Any
+// alignment of B's rows.
+template <int MODE>
+__global__ void __launch_bounds__(256)
+k_pad_b16(const void* __restrict__ B, int64_t K, int64_t N, int64_t ldb, int64_t n8,
+          uint2* __restrict__ out, uint2* __restrict__ lo) {
+  const int64_t quads = n8 / 4, total = K * quads;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total;
+       i += (int64_t)gridDim.x * 256) {
+    const int64_t k = i / quads, c = 4 * (i - k * quads);
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int64_t e = k * ldb + (c + x < N ? c + x : N - 1);
+      l[x] = 0u;
+      if (MODE == 0) {
+        h[x] = static_cast<const uint16_t*>(B)[e];
+      } else {
+        const float v = static_cast<const float*>(B)[e];
+        h[x] = MODE == 2 ? f32_to_f16_rne(v) : f32_to_bf16_rne(v);
+        if (MODE == 3) l[x] = f32_to_bf16_rne(v - bf16_to_f32(h[x]));
+      }
+      if (c + x >= N) h[x] = l[x] = 0u;
+    }
+    out[i] = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    if (MODE == 3) lo[i] = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+  }
+}
+
 }  // namespace
+
+size_t spmm_pad_workspace(int64_t K, int64_t N, int32_t precision) {
+  return (precision == BWS_PREC_BF16X2 ? 2 : 1) * split_plane_bytes(K, (N + 7) / 8 * 8);
+}
+
+// The 16-bit precisions for a B whose rows the direct copies cannot take (N or
+// ldb not a multiple of 8, rows off 16 bytes): B once more as 16-bit rows of a
+// multiple of 8 columns, then the direct-to-LDS kernels.  The rounding and the
+// order of K are those of the register-staged kernel, which loads such rows
+// element by element (500 x 2000 x 300 BF16: 136 us, here 16).
+bws_status spmm_mfma_padded(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb,
+                            int64_t N, float* C, int64_t ldc, float alpha, float beta,
+                            int32_t precision, void* workspace, hipStream_t s) {
+  const int64_t K = A->cols, n8 = (N + 7) / 8 * 8;
+  uint2* hi = static_cast<uint2*>(workspace);
+  uint2* lo = reinterpret_cast<uint2*>(static_cast<char*>(workspace) + split_plane_bytes(K, n8));
+  const unsigned grid = (unsigned)std::min<int64_t>(ceil_div(K * (n8 / 4), 256), 16384);
+#define BWS_PAD(MODE) \
+  hipLaunchKernelGGL(k_pad_b16<MODE>, dim3(grid), dim3(256), 0, s, B, K, N, ldb, n8, hi, lo)
+  if (precision == BWS_PREC_BF16X2) BWS_PAD(3);
+  else if (b_dtype != BWS_DTYPE_F32) BWS_PAD(0);
+  else if (precision == BWS_PREC_FP16) BWS_PAD(2);
+  else BWS_PAD(1);
+#undef BWS_PAD
+  BWS_TRY(launch_check());
+  const int32_t d16 = precision == BWS_PREC_FP16 ? BWS_DTYPE_F16 : BWS_DTYPE_BF16;
+  const int32_t p16 = precision == BWS_PREC_FP16 ? BWS_PREC_FP16 : BWS_PREC_BF16;
+  BWS_TRY(spmm_mfma(A, hi, d16, n8, N, C, ldc, alpha, beta, p16, nullptr, n8, s));
+  if (precision != BWS_PREC_BF16X2) return BWS_OK;
+  return spmm_mfma(A, lo, d16, n8, N, C, ldc, alpha, 1.0f, p16, nullptr, n8, s);
+}
 
 size_t spmm_split_workspace(int64_t K, int64_t N) { return 2 * split_plane_bytes(K, N); }
 size_t spmm_round_workspace(int64_t K, int64_t N) { return split_plane_bytes(K, N); }
@@ -958,7 +1065,7 @@ bws_status spmm_mfma_round(const bws_bitmap* A, const float* B, int64_t ldb, int
   }
   BWS_TRY(launch_check());
   return spmm_mfma(A, Bh, precision == BWS_PREC_FP16 ? BWS_DTYPE_F16 : BWS_DTYPE_BF16, N, N, C,
-                   ldc, alpha, beta, precision, plan, s);
+                   ldc, alpha, beta, precision, plan, N, s);
 }
 
 // Split-BF16 through the 16-bit kernels: B's hi and lo planes are written to
@@ -980,8 +1087,8 @@ bws_status spmm_mfma_split(const bws_bitmap* A, const float* B, int64_t ldb, int
     hipLaunchKernelGGL(k_split_bf16x2<false>, dim3(grid), dim3(256), 0, s, B, K, N, ldb,
                        reinterpret_cast<uint2*>(hi), reinterpret_cast<uint2*>(lo));
   BWS_TRY(launch_check());
-  BWS_TRY(spmm_mfma(A, hi, BWS_DTYPE_BF16, N, N, C, ldc, alpha, beta, BWS_PREC_BF16, plan, s));
-  return spmm_mfma(A, lo, BWS_DTYPE_BF16, N, N, C, ldc, alpha, 1.0f, BWS_PREC_BF16, plan, s);
+  BWS_TRY(spmm_mfma(A, hi, BWS_DTYPE_BF16, N, N, C, ldc, alpha, beta, BWS_PREC_BF16, plan, N, s));
+  return spmm_mfma(A, lo, BWS_DTYPE_BF16, N, N, C, ldc, alpha, 1.0f, BWS_PREC_BF16, plan, N, s);
 }
 
 }  // namespace bws

@@ -22,7 +22,7 @@ k_spmm_mfma4_big(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t l
   const int64_t tile = xcd_tile(blockIdx.x, per_xcd);
   if (tile >= row_blocks * col_blocks) return;
   mfma4_tile<PREC, 128, 128, 2, 64, false>(W, M, K, ldw, B, ldb, N, C, ldc, alpha, beta, tile,
-                                           row_blocks);
+                                           row_blocks, N);
 }
 
 }  // namespace

@@ -400,8 +400,11 @@ typedef struct {
 size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision,
                                const bws_plan* plan);
 /* The workspace with which bws_spmm has every kernel to choose from: at least
- * bws_spmm_workspace_size, 0 where none helps.  More than that only at FP32 on a
- * 0/1 A without a plan, for outputs of at least 192 tiles of 256 x 256 (N % 4 ==
+ * bws_spmm_workspace_size, 0 where none helps.  More than that on a 0/1 A without
+ * a plan: for BF16 / FP16 / BF16X2 with N % 8 != 0, room for B in 16 bits with
+ * rows of a multiple of 8 columns (also used for a 16-bit B whose rows are off 16
+ * bytes; the same bits as without it at BF16 / FP16, at BF16X2 as with the split
+ * of N % 8 == 0); at FP32, for outputs of at least 192 tiles of 256 x 256 (N % 4 ==
  * 0): room for B split exactly into three BF16 parts (6 bytes per element), so
  * that masks with more than one bit in eight run on the matrix cores (at 4096³ a
  * third to a quarter of the vector kernel's time at 50% density).  The density
