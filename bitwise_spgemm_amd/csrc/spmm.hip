@@ -235,7 +235,7 @@ bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t
   const bool f32_auto = precision == BWS_PREC_FP32 && !A->values && A->cols > 0 &&
                         b_dtype == BWS_DTYPE_F32 &&
                         (!plan || (plan->kernel == 0 && plan->rows_per_wg == 0));
-  if (f32_auto && spmm_direct_ok(A, ldb, N))
+  if (f32_auto && spmm_direct_ok(A, ldb, N, kDirectTiles))
     return launch_spmm_direct(A, static_cast<const float*>(B), ldb, N, C, ldc, alpha, beta,
                               stream);
   // and outputs that fill the chip with 256 x 256 tiles by the mask's density,

@@ -216,15 +216,15 @@ k_spmm_direct(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
 
 }  // namespace
 
-// Outputs of up to 512 tiles (2^21 elements): within them the product takes
+// bws_spmm: outputs of up to kDirectTiles = 512 tiles (2^21 elements): within them the product takes
 // 0.4 to 0.95 of the vector-add kernels' time at 1% density and less above
 // (those walk K at one workgroup's pace whatever the mask holds): 1024³ 14 us
 // against 26 (1%) to 92 (50%), 4096 x 1024 x 512 23 against 26 to 93, 4096² x 512
 // 58 against 91 to 358.  Beyond, at 2048³, it is 63 against 52 (1%), 62 (5%), 77
 // (10%).
-bool spmm_direct_ok(const bws_bitmap* A, int64_t ldb, int64_t N) {
+bool spmm_direct_ok(const bws_bitmap* A, int64_t ldb, int64_t N, int64_t max_tiles) {
   const int64_t rows = ceil_div(A->rows, kDT), cols = ceil_div(N, kDT);
-  return rows <= 512 && cols <= 512 && rows * cols <= 512 &&
+  return rows <= max_tiles && cols <= max_tiles && rows * cols <= max_tiles &&
          A->cols < ((int64_t)1 << 31) &&                            // 32-bit steps,
          A->rows * A->ldw < ((int64_t)1 << 32) && ldb < (1 << 24);  // and offsets
 }

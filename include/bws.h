@@ -465,7 +465,9 @@ bws_status bws_cluster_stream(const bws_bitmap* A, const int32_t* slot_row,
  * (base & ~row)·B and its base's base·B, summed once per chunk, is added at
  * the end; other rows sum their own bits.  FP32 vector adds; the summation
  * order differs from bws_spmm's, and the result stays within FP32 rounding of
- * A·B relative to |A|·|B| (the subtracted terms are bits of the base).  Needs
+ * A·B relative to |A|·|B| (the subtracted terms are bits of the base).  Outputs
+ * of up to 1024 tiles of 64 x 64 run as bws_spmm's small ones do, on the matrix
+ * cores from A itself.  Needs
  * N, ldb and ldc multiples of 4 and 16-byte aligned B and C
  * (BWS_EUNSUPPORTED otherwise). */
 bws_status bws_spmm_clustered(const bws_bitmap* A, const int32_t* slot_row,

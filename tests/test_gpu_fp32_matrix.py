@@ -142,3 +142,16 @@ def test_direct_graph(bws, dev):
         assert torch.equal(out, ref) and torch.equal(out2, ref2)
         torch.randn(1 << 20, device=dev).cumsum(0)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("M,K,N", [(64, 40, 4), (1000, 300, 1100), (2048, 128, 2048), (2049, 65, 2052)])
+def test_clustered_small_and_streamed(bws, dev, M, K, N):
+    """The row-clustered product on both sides of 1024 tiles of 64 x 64."""
+    A = bws.Bitmap(to_dev(bws.gen_bitmap_clustered(M, M, K, 16, 0.2, 0.02), dev), M, K)
+    D = bws.unpack_bitmap(A).double()
+    plan = bws.cluster_rows(A)
+    B = torch.randn((K, N), device=dev)
+    C0 = torch.randn((M, N), device=dev)
+    _check(bws.spmm_clustered(A, plan, B, alpha=2.0, beta=0.5, out=C0.clone()), D, B, K, 2.0, 0.5, C0)
+    Bi = torch.randint(-1000, 1001, (K, N), device=dev).float()
+    assert torch.equal(bws.spmm_clustered(A, plan, Bi).double(), D @ Bi.double())
