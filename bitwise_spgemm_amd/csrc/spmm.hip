@@ -52,6 +52,8 @@ ValuCfg plan_valu_cfg(const bws_plan* plan, int64_t M, int64_t N, bool vals) {
   }
   return c;
 }
+bool valu_direct_ok(int32_t b_dtype, const void* B, int64_t ldb, int64_t N, const float* C,
+                    int64_t ldc);
 bws_status spmm_mfma(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb, int64_t N,
                      float* C, int64_t ldc, float alpha, float beta, int32_t precision,
                      const bws_plan* plan, int64_t nb, hipStream_t s);
@@ -235,7 +237,12 @@ bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t
   const bool f32_auto = precision == BWS_PREC_FP32 && !A->values && A->cols > 0 &&
                         b_dtype == BWS_DTYPE_F32 &&
                         (!plan || (plan->kernel == 0 && plan->rows_per_wg == 0));
-  if (f32_auto && spmm_direct_ok(A, ldb, N, kDirectTiles))
+  // (larger ones where the rows are not 16-byte pieces, which the vector-add tile
+  // kernels need: the row kernel took 159 to 318 us at 2000 x 2000 x 2001 and 785
+  // to 1297 at 4096² x 2049, 0.5% to 20% density, against 80 and 285; at 4095³ it
+  // is 421 against 500 at 0.5%)
+  if (f32_auto &&
+      spmm_direct_ok(A, ldb, N, valu_direct_ok(b_dtype, B, ldb, N, C, ldc) ? kDirectTiles : 2304))
     return launch_spmm_direct(A, static_cast<const float*>(B), ldb, N, C, ldc, alpha, beta,
                               stream);
   // and outputs that fill the chip with 256 x 256 tiles by the mask's density,

@@ -33,7 +33,8 @@ def _check(C, D, B, K, alpha=1.0, beta=0.0, C0=None):
 # multiple of 4 and below 4, both wave counts (192 tiles and more)
 DIRECT = [(1, 1, 1, 1.0), (64, 32, 64, 0.3), (63, 31, 61, 0.5), (65, 33, 67, 0.2),
           (130, 256, 2, 0.4), (70, 257, 5, 0.1), (128, 1000, 131, 0.05), (100, 40, 130, 0.9),
-          (12300, 70, 64, 0.2), (64, 300, 12290, 0.1), (1500, 129, 1025, 0.02), (64, 5000, 3, 0.01)]
+          (12300, 70, 64, 0.2), (64, 300, 12290, 0.1), (1500, 129, 1025, 0.02), (64, 5000, 3, 0.01),
+          (2300, 100, 2301, 0.1), (4090, 40, 2306, 0.2)]  # rows off 16 bytes: up to 2304 tiles
 
 
 @pytest.mark.parametrize("M,K,N,p", DIRECT)
