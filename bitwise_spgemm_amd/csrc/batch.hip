@@ -25,6 +25,7 @@ bws_status spmm_mfma_batch(const BatchEntry* entries, const int64_t* slot_off, i
 bool valu_direct_ok(int32_t b_dtype, const void* B, int64_t ldb, int64_t N, const float* C,
                     int64_t ldc);
 ValuCfg plan_valu_cfg(const bws_plan* plan, int64_t M, int64_t N, bool vals);
+bool spmm_vals_ok(int64_t K);
 
 namespace {
 
@@ -125,7 +126,8 @@ Choice classify(const bws_problem& p, int32_t b_dtype, int32_t precision, const 
     if (c.tile.bm == 256 && c.tile.bn == 256) c.tile.bm = 128;
     return c;
   }
-  if (p.A.cols > 0 && valu_direct_ok(b_dtype, p.B, p.ldb, p.N, p.C, p.ldc)) {
+  if (p.A.cols > 0 && valu_direct_ok(b_dtype, p.B, p.ldb, p.N, p.C, p.ldc) &&
+      (!p.A.values || spmm_vals_ok(p.A.cols))) {
     c.kind = 1;
     c.vals = p.A.values != nullptr;
     c.cfg = plan_valu_cfg(eff.rows_per_wg ? &eff : nullptr, p.A.rows, p.N, c.vals);

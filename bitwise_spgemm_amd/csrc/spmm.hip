@@ -8,6 +8,8 @@ bws_status spmm_valu(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_
                      float* C, int64_t ldc, float alpha, float beta, const ValuCfg& cfg,
                      hipStream_t s);
 
+int32_t spmm_vals_rows(int64_t M, int64_t N);
+
 bool valu_cfg_valid(const ValuCfg& c) {
   static const int32_t ok[][3] = {{256, 8, 64}, {256, 16, 64}, {256, 16, 32}, {128, 8, 64},
                                   {128, 8, 32},  {64, 8, 32},   {128, 16, 32}, {128, 16, 64},
@@ -23,15 +25,17 @@ bool valu_cfg_valid(const ValuCfg& c) {
 // 8192 x 4096 x 1024 and 16384 x 4096 x 512 with 5% clustered and 10% iid
 // masks: 16 waves beat 8 waves on the same rows by 25-45% (four waves per
 // SIMD hide the LDS and bit-scan latency of the per-row chains).  Value masks
-// stop at 8 rows per wave: with 16 rows the per-row values of two stages
-// exceed the 128-VGPR budget of a 1024-lane workgroup and spill, and 16 x 8
-// measured 1-3% faster than that on 4096³ (2%, 10%), 8192 x 4096 x 2048 and
-// 16384 x 4096 x 1024 value masks.
+// have a tile kernel of their own (spmm_vals.hip; the rows are its row block).
 ValuCfg default_valu_cfg(int64_t M, int64_t N, bool vals) {
   ValuCfg c;
   c.waves = 16;
+  if (vals) {
+    c.rows = spmm_vals_rows(M, N);
+    if (c.rows == 64) c.kstage = 32;
+    return c;
+  }
   const int64_t tiles256 = ceil_div(M, 256) * ceil_div(N, 256);
-  if (tiles256 >= 192 && !vals) return c;  // 16 waves x 16 rows
+  if (tiles256 >= 192) return c;  // 16 waves x 16 rows
   const int64_t tiles128 = ceil_div(M, 128) * ceil_div(N, 256);
   if (tiles128 >= 192) {
     c.rows = 128;

@@ -14,6 +14,14 @@
 #include "bws_internal.hpp"
 
 namespace bws {
+
+// the FP32 product of a value-carrying bitmap (spmm_vals.hip)
+bool spmm_vals_ok(int64_t K);
+bws_status spmm_vals_f32(const bws_bitmap* A, const float* B, int64_t ldb, int64_t N, float* C,
+                         int64_t ldc, float alpha, float beta, int32_t rows, hipStream_t s);
+bws_status spmm_vals_f32_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
+                               int64_t total_tiles, int32_t rows, hipStream_t s);
+
 namespace {
 
 constexpr int kWaves = 8;
@@ -220,7 +228,7 @@ k_spmm_rows(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
 //    The loads are issued from a two-instruction asm block (they write LDS
 //    only, no VGPR results), and the one wait on them (vmcnt(0)) sits right
 //    before each stage's barrier, so nothing waits on the prefetch mid-stage;
-//  - bitmap words are prefetched two stages ahead and values one stage ahead,
+//  - bitmap words are prefetched two stages ahead (grouped values one stage),
 //    so every global load a stage consumes was issued before its barrier;
 //  - set bits are consumed in batches of 4, 2 and 1 independent LDS reads,
 //    keeping several reads in flight per wave; within a row the adds stay in
@@ -248,8 +256,6 @@ __device__ __forceinline__ void take_bit(uint64_t& m, int& k) {
   asm volatile("s_bitset0_b64 %0, %1" : "+s"(m) : "s"(k));
 }
 
-// One output tile ; the
-// tile index is column-block-major within the problem.
 // The grouped form's value tables (bws_group_rows): the value of set bit i of
 // word w of row r is gv[(G * t + g) * 32 + i] with g = gid[r * ldw + w] >= 0
 // and t = (r / T) * wpr + w; a spilled word (g < 0) takes the row's own
@@ -260,7 +266,8 @@ struct GroupTab {
   int T, G;
 };
 
-template <int WAVES, int RPW, int KS, bool VALS, bool GRP = false>
+// One output tile; the tile index is column-block-major within the problem.
+template <int WAVES, int RPW, int KS, bool GRP = false>
 __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64_t M, int64_t K,
                                            int64_t ldw, const int64_t* __restrict__ row_ptr,
                                            const float* __restrict__ values,
@@ -269,7 +276,6 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
                                            float beta, int64_t tile, int64_t row_blocks,
                                            GroupTab gt = GroupTab{nullptr, nullptr, 1, 1}) {
   static_assert(KS == 32 || KS == 64, "stage is one or two bitmap words");
-  static_assert(VALS || !GRP, "grouped values walk like values");
   constexpr int WPS = KS / 32;  // bitmap words per stage
   __shared__ float4 sB0[KS][64];
   __shared__ float4 sB1[KS][64];
@@ -317,10 +323,10 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
     return ((((uint64_t)w_hi) << 32) | w_lo) & smask;
   };
 
-  int64_t e_l = 0;         // VALS: lane l < RPW: value offset of row l at the current stage
-  int cnt_cur = 0;         // VALS: set bits of row l in the current stage
-  float vv[VALS ? RPW : 1];
-  if (VALS && (!GRP || values)) e_l = row_lane ? row_ptr[mw + rl] : 0;
+  int64_t e_l = 0;         // GRP: lane l < RPW: value offset of row l at the current stage
+  int cnt_cur = 0;         // GRP: set bits of row l in the current stage
+  float vv[GRP ? RPW : 1];
+  if (GRP && values) e_l = row_lane ? row_ptr[mw + rl] : 0;
   // GRP: lane p's value is that of stage column p of row r (zero when the bit
   // is clear), so the walk reads it by column, not by rank; tbase[r] is the
   // group-table tile index of row r's word 0
@@ -330,7 +336,7 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
     const int64_t row = mw + r < M ? mw + r : M - 1;
     tbase[r] = GRP ? (row / gt.T) * wpr : 0;
   }
-  auto grp_values = [&](float (&dst)[VALS ? RPW : 1], uint32_t words, int64_t st, int64_t e_row) {
+  auto grp_values = [&](float (&dst)[GRP ? RPW : 1], uint32_t words, int64_t st, int64_t e_row) {
     const uint64_t sm = stage_mask(st);
     const int p = lane;
     const int64_t wp = WPS * st + (p >> 5);
@@ -357,25 +363,16 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
           v = 1.0f;
         }
       }
-      dst[VALS ? r : 0] = v;
+      dst[GRP ? r : 0] = v;
     }
   };
 
   issue(0, base0);
   uint32_t wcur = load_words(0);
   uint32_t wnext = load_words(1);
-  if (VALS) {
+  if (GRP) {
     cnt_cur = __popcll(lane_row_mask(wcur, stage_mask(0)));
-    if (GRP) {
-      grp_values(vv, wcur, 0, e_l);
-    } else {
-#pragma unroll
-      for (int r = 0; r < RPW; ++r) {
-        const int64_t e = readlane_i64(e_l, r);
-        const int c = __builtin_amdgcn_readlane(cnt_cur, r);
-        vv[r] = lane < c ? values[e + lane] : 0.0f;
-      }
-    }
+    grp_values(vv, wcur, 0, e_l);
   }
 
   auto stage = [&](int64_t st, float4 (*cur)[64], uint32_t nxt_base) {
@@ -384,30 +381,21 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
     // re-defining them through an empty asm statement tells the compiler so,
     // which keeps it from waiting (vmcnt(0)) on the prefetch issued next.
     asm volatile("" : "+v"(wcur), "+v"(wnext));
-    if (VALS) {
+    if (GRP) {
 #pragma unroll
-      for (int r = 0; r < RPW; ++r) asm volatile("" : "+v"(vv[VALS ? r : 0]));
+      for (int r = 0; r < RPW; ++r) asm volatile("" : "+v"(vv[GRP ? r : 0]));
     }
     __syncthreads(); // everyone's; the other buffer is no longer being read
     const bool more = st + 1 < nst;
     if (more) issue(st + 1, nxt_base);
     const uint32_t wn2 = load_words(st + 2);
     const uint64_t smask = stage_mask(st);
-    float vn[VALS ? RPW : 1];
+    float vn[GRP ? RPW : 1];
     int cnt_next = 0;
-    if (VALS) {
+    if (GRP) {
       const int64_t e_next = e_l + cnt_cur;
       cnt_next = more ? __popcll(lane_row_mask(wnext, stage_mask(st + 1))) : 0;
-      if (GRP) {
-        grp_values(vn, wnext, st + 1, e_next);
-      } else {
-#pragma unroll
-        for (int r = 0; r < RPW; ++r) {
-          const int64_t e = readlane_i64(e_next, r);
-          const int c = __builtin_amdgcn_readlane(cnt_next, r);
-          vn[r] = lane < c ? values[e + lane] : 0.0f;
-        }
-      }
+      grp_values(vn, wnext, st + 1, e_next);
     }
 
     // every row's stage mask, masked and bit-reversed once in VALU (lane r
@@ -421,7 +409,6 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
       uint64_t m = (((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)rev_hi, r)) << 32) |
                    (uint32_t)__builtin_amdgcn_readlane((int)rev_lo, r);
       int n = __builtin_amdgcn_readlane(cnt_v, r);
-      int j = 0;
       while (n >= 4) {
         int k0, k1, k2, k3;
         take_bit(m, k0);
@@ -430,11 +417,11 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
         take_bit(m, k3);
         const float4 b0 = cur[k0][lane], b1 = cur[k1][lane], b2 = cur[k2][lane],
                      b3 = cur[k3][lane];
-        if (VALS) {
-          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k0 : j), b0);
-          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k1 : j + 1), b1);
-          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k2 : j + 2), b2);
-          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k3 : j + 3), b3);
+        if (GRP) {
+          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k0), b0);
+          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k1), b1);
+          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k2), b2);
+          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k3), b3);
         } else {
           add4(acc[r], b0);
           add4(acc[r], b1);
@@ -442,32 +429,30 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
           add4(acc[r], b3);
         }
         n -= 4;
-        j += 4;
       }
       if (n >= 2) {
         int k0, k1;
         take_bit(m, k0);
         take_bit(m, k1);
         const float4 b0 = cur[k0][lane], b1 = cur[k1][lane];
-        if (VALS) {
-          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k0 : j), b0);
-          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k1 : j + 1), b1);
+        if (GRP) {
+          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k0), b0);
+          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k1), b1);
         } else {
           add4(acc[r], b0);
           add4(acc[r], b1);
         }
         n -= 2;
-        j += 2;
       }
       if (n) {
         int k0;
         take_bit(m, k0);
         const float4 b0 = cur[k0][lane];
-        if (VALS) fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k0 : j), b0);
+        if (GRP) fma4(acc[r], readlane_f(vv[GRP ? r : 0], k0), b0);
         else add4(acc[r], b0);
       }
     }
-    if (VALS) {
+    if (GRP) {
       e_l += cnt_cur;
       cnt_cur = cnt_next;
 #pragma unroll
@@ -505,7 +490,7 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
   }
 }
 
-template <int WAVES, int RPW, int KS, bool VALS>
+template <int WAVES, int RPW, int KS>
 __global__ void __launch_bounds__(WAVES * 64)
 k_spmm_rows2(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
              const int64_t* __restrict__ row_ptr, const float* __restrict__ values,
@@ -514,7 +499,7 @@ k_spmm_rows2(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
              int64_t per_xcd) {
   const int64_t tile = xcd_tile(blockIdx.x, per_xcd);
   if (tile >= row_blocks * col_blocks) return;
-  rows2_tile<WAVES, RPW, KS, VALS>(W, M, K, ldw, row_ptr, values, B, ldb, N, C, ldc, alpha, beta,
+  rows2_tile<WAVES, RPW, KS>(W, M, K, ldw, row_ptr, values, B, ldb, N, C, ldc, alpha, beta,
                                    tile, row_blocks);
 }
 
@@ -528,12 +513,12 @@ k_spmm_rows2_groups(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_
                     int64_t per_xcd) {
   const int64_t tile = xcd_tile(blockIdx.x, per_xcd);
   if (tile >= row_blocks * col_blocks) return;
-  rows2_tile<WAVES, RPW, KS, true, true>(W, M, K, ldw, row_ptr, values, B, ldb, N, C, ldc, 1.0f,
+  rows2_tile<WAVES, RPW, KS, true>(W, M, K, ldw, row_ptr, values, B, ldb, N, C, ldc, 1.0f,
                                          0.0f, tile, row_blocks, gt);
 }
 
 // Grouped launch: a workgroup finds its problem and tile with batch_tile.
-template <int WAVES, int RPW, int KS, bool VALS>
+template <int WAVES, int RPW, int KS>
 __global__ void __launch_bounds__(WAVES * 64)
 k_spmm_rows2_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ slot_off,
                    int count) {
@@ -541,7 +526,7 @@ k_spmm_rows2_batch(const BatchEntry* __restrict__ entries, const int64_t* __rest
   int64_t tile;
   if (!batch_tile(entries, slot_off, count, lo, tile)) return;
   const BatchEntry& e = entries[lo];
-  rows2_tile<WAVES, RPW, KS, VALS>(e.W, e.M, e.K, e.ldw, e.row_ptr, e.values,
+  rows2_tile<WAVES, RPW, KS>(e.W, e.M, e.K, e.ldw, e.row_ptr, e.values,
                                    static_cast<const float*>(e.B), e.ldb, e.N, e.C, e.ldc, 1.0f,
                                    0.0f, tile, e.row_blocks);
 }
@@ -652,7 +637,7 @@ k_sddmm_f32(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
   }
 }
 
-template <int WAVES, int RPW, int KS, bool VALS>
+template <int WAVES, int RPW, int KS>
 bws_status launch_rows2(const bws_bitmap* A, const float* B, int64_t ldb, int64_t N, float* C,
                         int64_t ldc, float alpha, float beta, hipStream_t s) {
   const int64_t row_blocks = ceil_div(A->rows, WAVES * RPW);
@@ -660,7 +645,7 @@ bws_status launch_rows2(const bws_bitmap* A, const float* B, int64_t ldb, int64_
   const int64_t tiles = row_blocks * col_blocks;
   const int64_t per_xcd = ceil_div(tiles, 8);
   if (8 * per_xcd > kMaxGrid) return BWS_ECAPACITY;
-  hipLaunchKernelGGL((k_spmm_rows2<WAVES, RPW, KS, VALS>), dim3((unsigned)(8 * per_xcd)),
+  hipLaunchKernelGGL((k_spmm_rows2<WAVES, RPW, KS>), dim3((unsigned)(8 * per_xcd)),
                      dim3(WAVES * 64), 0, s, A->words, A->rows, A->cols, A->ldw, A->row_ptr,
                      A->values, B, ldb, N, C, ldc, alpha, beta, row_blocks, col_blocks, per_xcd);
   return launch_check();
@@ -700,13 +685,13 @@ inline int grid_for(int64_t items, int64_t per_block) {
   return (int)g;
 }
 
-template <int WAVES, int RPW, int KS, bool VALS>
+template <int WAVES, int RPW, int KS>
 bws_status launch_rows2_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
                               int64_t total_tiles, hipStream_t s) {
   const int64_t grid = batch_grid(total_tiles, count);
   if (grid > kMaxGrid) return BWS_ECAPACITY;
   if (total_tiles == 0) return BWS_OK;
-  hipLaunchKernelGGL((k_spmm_rows2_batch<WAVES, RPW, KS, VALS>), dim3((unsigned)grid),
+  hipLaunchKernelGGL((k_spmm_rows2_batch<WAVES, RPW, KS>), dim3((unsigned)grid),
                      dim3(WAVES * 64), 0, s, entries, slot_off, count);
   return launch_check();
 }
@@ -716,10 +701,10 @@ bws_status launch_rows2_batch(const BatchEntry* entries, const int64_t* slot_off
 // Grouped vector-add launch (FP32 B meeting the direct-staging conditions).
 bws_status spmm_valu_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
                            int64_t total_tiles, const ValuCfg& cfg, bool vals, hipStream_t s) {
-#define BWS_VB(WV, RP, KS)                                                                    \
-  if (cfg.waves == WV && cfg.rows == WV * RP && cfg.kstage == KS)                             \
-    return vals ? launch_rows2_batch<WV, RP, KS, true>(entries, slot_off, count, total_tiles, s) \
-                : launch_rows2_batch<WV, RP, KS, false>(entries, slot_off, count, total_tiles, s);
+  if (vals) return spmm_vals_f32_batch(entries, slot_off, count, total_tiles, cfg.rows, s);
+#define BWS_VB(WV, RP, KS)                                        \
+  if (cfg.waves == WV && cfg.rows == WV * RP && cfg.kstage == KS) \
+    return launch_rows2_batch<WV, RP, KS>(entries, slot_off, count, total_tiles, s);
   BWS_VB(8, 32, 64)
   BWS_VB(16, 16, 64)
   BWS_VB(16, 16, 32)
@@ -748,13 +733,13 @@ bws_status spmm_valu(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_
   const bool vec = (ldb % 4 == 0) && (ldc % 4 == 0) &&
                    (reinterpret_cast<uintptr_t>(B) % (4 * esz) == 0) &&
                    (reinterpret_cast<uintptr_t>(C) % 16 == 0);
-  if (b_dtype == BWS_DTYPE_F32 && vec && N % 4 == 0 && N >= 4) {
-    const float* Bf = static_cast<const float*>(B);
-    const bool vals = A->values != nullptr;
-#define BWS_V2(WV, RP, KS)                                                              \
-  if (cfg.waves == WV && cfg.rows == WV * RP && cfg.kstage == KS)                       \
-    return vals ? launch_rows2<WV, RP, KS, true>(A, Bf, ldb, N, C, ldc, alpha, beta, s) \
-                : launch_rows2<WV, RP, KS, false>(A, Bf, ldb, N, C, ldc, alpha, beta, s);
+  const float* Bf = static_cast<const float*>(B);
+  if (b_dtype == BWS_DTYPE_F32 && A->values && spmm_vals_ok(A->cols))
+    return spmm_vals_f32(A, Bf, ldb, N, C, ldc, alpha, beta, cfg.rows, s);
+  if (b_dtype == BWS_DTYPE_F32 && vec && N % 4 == 0 && N >= 4 && !A->values) {
+#define BWS_V2(WV, RP, KS)                                        \
+  if (cfg.waves == WV && cfg.rows == WV * RP && cfg.kstage == KS) \
+    return launch_rows2<WV, RP, KS>(A, Bf, ldb, N, C, ldc, alpha, beta, s);
     BWS_V2(8, 32, 64)
     BWS_V2(16, 16, 64)
     BWS_V2(16, 16, 32)
