@@ -115,7 +115,6 @@ bws_status launch_spmm_stream(const uint32_t* S, const int32_t* slot_row, int64_
 // parts: in one launch for small outputs (spmm_direct.hip), and for outputs
 // that fill the chip, where the mask is dense, over planes of B in a workspace
 // of f32_routed_bytes (spmm_planes.hip; sparse masks take the streamed product).
-constexpr int64_t kDirectTiles = 512;  // the most 64 x 64 tiles bws_spmm takes it for
 bool spmm_direct_ok(const bws_bitmap* A, int64_t ldb, int64_t N, int64_t max_tiles);
 bws_status launch_spmm_direct(const bws_bitmap* A, const float* B, int64_t ldb, int64_t N,
                               float* C, int64_t ldc, float alpha, float beta, hipStream_t s);

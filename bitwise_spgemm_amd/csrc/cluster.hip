@@ -823,9 +823,8 @@ bws_status bws_spmm_clustered(const bws_bitmap* A, const int32_t* slot_row,
   // Outputs of up to 1024 tiles of 64 x 64: the streamed kernel has few 256 x 256
   // workgroups and walks K at one workgroup's pace, the one-launch product on the
   // matrix cores does not need the plan.  us, streamed at 1% to 50% density
-  // against that: 1024³ 41 to 236 | 15, 4096² x 512 129 to 307 | 64, 2048³ 79 to
-  // 412 | 63, 4096² x 1024 129 to 306 | 114; at 2048 tiles, 4096 x 1024 x 2048, 40 to
-  // 83 | 78.
+  // against that: 1024³ 41 to 236 | 10, 2048³ 79 to 412 | 48, 4096² x 1024 129 to
+  // 306 | 85; at 2048 tiles, 4096 x 1024 x 2048, 40 to 83 | 60 (by the tiles).
   if (spmm_direct_ok(A, ldb, N, 1024))
     return launch_spmm_direct(A, B, ldb, N, C, ldc, alpha, beta, s);
   return launch_spmm_stream(static_cast<const uint32_t*>(plan_stream), slot_row, A->rows, A->cols,

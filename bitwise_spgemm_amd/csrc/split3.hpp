@@ -44,16 +44,17 @@ __device__ __forceinline__ float row_sum(const uint32_t* __restrict__ w, int64_t
   return s;
 }
 
-// 0/1 A fragment from a bitmap word (bit-reversed): byte q, bit e -> K slot
-// 8q + e; (z & (0x10001 << 2p)) * (ONE >> 2p) puts ONE (BF16 1.0) into the low
-// half iff bit 2p is set and into the high half iff bit 2p + 1 is.
-__device__ __forceinline__ uint4 a_frag01(uint32_t rw, int q) {
-  const uint32_t x = __builtin_amdgcn_ubfe(rw, 8 * q, 8);
-  const uint32_t z = x | (x << 15);
-  return make_uint4((uint32_t)__umul24(z & 0x00010001u, 0x3F80u),
-                    (uint32_t)__umul24(z & 0x00040004u, 0x3F80u >> 2),
-                    (uint32_t)__umul24(z & 0x00100010u, 0x3F80u >> 4),
-                    (uint32_t)__umul24(z & 0x00400040u, 0x3F80u >> 6));
+// 0/1 A fragment from a bitmap word (MSB first): K slot 8q + e of the 32-wide
+// step is bit 7 - e of x, the word's byte q from the top.  For z = x | (x << 17),
+// (z & (0x10001 << (7 - 2p))) * (ONE >> (7 - 2p)) puts ONE (BF16 1.0) into the low
+// half iff slot 2p is set and into the high half iff slot 2p + 1 is.
+__device__ __forceinline__ uint4 a_frag01(uint32_t w, int q) {
+  const uint32_t x = __builtin_amdgcn_ubfe(w, 24 - 8 * q, 8);
+  const uint32_t z = x | (x << 17);
+  return make_uint4((uint32_t)__umul24(z & 0x00800080u, 0x3F80u >> 7),
+                    (uint32_t)__umul24(z & 0x00200020u, 0x3F80u >> 5),
+                    (uint32_t)__umul24(z & 0x00080008u, 0x3F80u >> 3),
+                    (uint32_t)__umul24(z & 0x00020002u, 0x3F80u >> 1));
 }
 
 // x is not to be trusted: not finite, or nonzero and below kSmallOut.

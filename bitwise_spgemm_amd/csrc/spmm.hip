@@ -122,6 +122,26 @@ bool combo_ok(int32_t precision, int32_t b_dtype) {
 
 size_t esize(int32_t d) { return d == BWS_DTYPE_F32 ? 4 : 2; }
 
+// The most 64 x 64 tiles of output for which the FP32 product of a 0/1 A runs in
+// one launch on the matrix cores: its workgroups cost about 5 us besides their K
+// steps, so that short products and many of them go to the vector-add kernels,
+// whose time falls with K and with the mask's density.  us, one launch against
+// vector-add at 1% | 5% density:
+//   tiles  256, K   64:  6.0 |  4.5,  4.8     K  128:  6.2 |  5.9,  6.7
+//   tiles  512, K  128:  7.5 |  6.5,  7.3     K  256:  9.1 |  9.4, 10.9
+//   tiles 1024, K  512: 18.6 | 18.3, 20.0     K 1024: 28.0 | 32.3, 34.0
+//                                             K 2048: 48.0 | 57.8, 61.9
+//   tiles 1536, K 1024: 43.4 | 28.7, 39.8
+// Rows that are not 16-byte pieces leave only the row kernel on the other side:
+//   tiles 1056, K   64: 23.6 | 20.1, 19.3     K  256: 28.2 | 44.6 (2%)
+//   tiles 4096, K 4095:  364 |  480,  723 (432 at 0.1%)
+//   tiles 16384, K 256:  312 |  198,  260
+int64_t direct_max_tiles(int64_t K, bool aligned) {
+  if (K < 128) return 0;
+  if (!aligned) return K < 1024 ? 2304 : (int64_t)1 << 28;
+  return K < 256 ? 256 : K < 1024 ? 512 : 1024;
+}
+
 // The streamed FP32 kernel: 16-byte rows of B and C, and enough 256 x 256
 // tiles to occupy the chip (one workgroup per CU).
 bool stream_ok(const bws_bitmap* A, const void* B, int64_t ldb, int64_t N, const float* C,
@@ -241,12 +261,9 @@ bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t
   const bool f32_auto = precision == BWS_PREC_FP32 && !A->values && A->cols > 0 &&
                         b_dtype == BWS_DTYPE_F32 &&
                         (!plan || (plan->kernel == 0 && plan->rows_per_wg == 0));
-  // (larger ones where the rows are not 16-byte pieces, which the vector-add tile
-  // kernels need: the row kernel took 159 to 318 us at 2000 x 2000 x 2001 and 785
-  // to 1297 at 4096² x 2049, 0.5% to 20% density, against 80 and 285; at 4095³ it
-  // is 421 against 500 at 0.5%)
   if (f32_auto &&
-      spmm_direct_ok(A, ldb, N, valu_direct_ok(b_dtype, B, ldb, N, C, ldc) ? kDirectTiles : 2304))
+      spmm_direct_ok(A, ldb, N,
+                     direct_max_tiles(A->cols, valu_direct_ok(b_dtype, B, ldb, N, C, ldc))))
     return launch_spmm_direct(A, static_cast<const float*>(B), ldb, N, C, ldc, alpha, beta,
                               stream);
   // and outputs that fill the chip with 256 x 256 tiles by the mask's density,

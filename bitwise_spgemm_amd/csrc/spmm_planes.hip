@@ -116,7 +116,7 @@ __device__ __forceinline__ void planes_tile(const uint32_t* __restrict__ W, int6
       const uint32_t vb = valid_bits(st * kPK + x, K);
 #pragma unroll
       for (int a = 0; a < kPA; ++a) {
-        wr[x][a] = __brev(sA[buf * kPWords + x * kPM + (wm * kPA + a) * 16 + j] & vb);
+        wr[x][a] = sA[buf * kPWords + x * kPM + (wm * kPA + a) * 16 + j] & vb;
         any |= wr[x][a];
       }
     }

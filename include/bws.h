@@ -369,9 +369,10 @@ typedef struct {
 
 /* C = alpha * (A · B) + beta * C, A M x K bitmap, B K x N dense (dtype b_dtype,
  * leading dimension ldb), C M x N FP32.  beta == 0 never reads C.
- * FP32 with a 0/1 A, an F32 B and no plan: outputs of up to 512 tiles of 64 x 64
- * run on the matrix cores without a workspace, each b split exactly into three
- * BF16 parts and every product and sum in FP32.
+ * FP32 with a 0/1 A, an F32 B and no plan: outputs of up to 256, 512 and 1024 tiles
+ * of 64 x 64 with K of at least 128, 256 and 1024 (larger ones too where rows of B
+ * or C are off 16 bytes) run on the matrix cores without a workspace, each b split
+ * exactly into three BF16 parts and every product and sum in FP32.
  * precision/b_dtype combinations: FP32 with F32 (or exact BF16/F16 input);
  * BF16 with BF16 or F32 (rounded to nearest even); FP16 with F16 or F32;
  * BF16X2 with F32.
