@@ -35,6 +35,7 @@ HIP_FLAGS = [
 # accumulators between register files around the empty-stage branch.
 FILE_FLAGS = {
     "spmm_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "spmm_direct16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "spmm_direct.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "spmm_planes.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     # 128 x 128 wave tiles: 256 accumulators live in AGPRs

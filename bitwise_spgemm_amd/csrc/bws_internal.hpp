@@ -118,6 +118,11 @@ bws_status launch_spmm_stream(const uint32_t* S, const int32_t* slot_row, int64_
 bool spmm_direct_ok(const bws_bitmap* A, int64_t ldb, int64_t N, int64_t max_tiles);
 bws_status launch_spmm_direct(const bws_bitmap* A, const float* B, int64_t ldb, int64_t N,
                               float* C, int64_t ldc, float alpha, float beta, hipStream_t s);
+// 16-bit precisions, small outputs with a long K, in one launch (spmm_direct16.hip).
+bool spmm_direct16_ok(const bws_bitmap* A, int64_t ldb, int64_t N);
+bws_status launch_spmm_direct16(const bws_bitmap* A, const void* B, int32_t b_dtype,
+                                int32_t precision, int64_t ldb, int64_t N, float* C, int64_t ldc,
+                                float alpha, float beta, hipStream_t s);
 size_t f32_routed_bytes(int64_t M, int64_t K, int64_t N);
 bws_status launch_spmm_f32_routed(const bws_bitmap* A, void* ws, const float* B, int64_t ldb,
                                   int64_t N, float* C, int64_t ldc, float alpha, float beta,

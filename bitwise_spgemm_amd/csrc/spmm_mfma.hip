@@ -669,6 +669,8 @@ bool dma_ok(int32_t precision, int32_t b_dtype, const void* B, int64_t ldb, int6
 // keeps every CU's waves busy.  A K stage is a barrier and a copy's latency
 // whatever the tile, so small outputs want many small workgroups and 128-row
 // stages.  Measured BF16 times, us, of 32 x 64 | 64 x 64 | 64 x 128 | 128 x 128:
+// (outputs of up to 512 tiles of 64 x 64 with a long K take spmm_direct16.hip,
+// except in grouped launches)
 //   256 x 512 x 192      (t64 12)     5 |   6 |   8 |  11
 //   1024 x 4096 x 512    (t64 128)   21 |  27 |  34 |  53
 //   1024³                (t64 256)  8.5 | 9.6 |  12 |  18
