@@ -38,31 +38,40 @@ __device__ __forceinline__ void store_set_bits_128(const f32x4 (&acc)[4][4], uin
   uint32_t* eW = reinterpret_cast<uint32_t*>(scratch);          // [128][4] words
   int64_t* eBase = reinterpret_cast<int64_t*>(scratch + 2048);  // [128][4] value indices
   __syncthreads();  // every wave is done with the operand buffers
-  for (int t = threadIdx.x; t < BR * (BK / 32); t += 256) {
+#pragma unroll
+  for (int t0 = 0; t0 < BR * (BK / 32); t0 += 256) {
+    const int t = t0 + threadIdx.x;
     const int64_t r = r0 + (t >> 2), w = k0 / 32 + (t & 3);
-    uint32_t word = 0u;
-    int64_t base = 0;
-    if (r < M && w < wpr) {
-      word = W[r * ldw + w] & valid_bits(w, K);
-      base = row_ptr[r] + woff[r * wpr + w];
-    }
-    eW[t] = word;
-    eBase[t] = base;
+    const int64_t rc = r < M ? r : M - 1, wc = w < wpr ? w : wpr - 1;
+    const uint32_t word = W[rc * ldw + wc];
+    eBase[t] = row_ptr[rc] + woff[rc * wpr + wc];
+    eW[t] = r < M && w < wpr ? word & valid_bits(w, K) : 0u;
   }
   __syncthreads();
+  // the words and bases of a row tile are read before its stores (a read and a
+  // wait per output took longer than the stores)
+  const uint32_t bit[2] = {wbit(j), wbit(16 + j)};
+  const uint32_t before[2] = {~(0xFFFFFFFFu >> j), ~(0xFFFFFFFFu >> (16 + j))};
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int a = 0; a < 4; ++a) {
+    uint2 word[4];
+    longlong2 base[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int rr = 64 * wm + 16 * a + 4 * q + e;
+      const int ew = (64 * wm + 16 * a + 4 * q + e) * (BK / 32) + 2 * wn;
+      word[e] = *reinterpret_cast<const uint2*>(eW + ew);
+      base[e] = *reinterpret_cast<const longlong2*>(eBase + ew);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        const int ew = rr * (BK / 32) + 2 * wn + (b >> 1);
-        const uint32_t word = eW[ew];
-        const int i = 16 * (b & 1) + j;
-        if (word & wbit(i)) dA[eBase[ew] + rank_before(word, i)] = acc[a][b][e];
+        const uint32_t x = b < 2 ? word[e].x : word[e].y;
+        if (x & bit[b & 1])
+          dA[(b < 2 ? base[e].x : base[e].y) + __popc(x & before[b & 1])] = acc[a][b][e];
       }
-    }
+  }
 }
 
 // Load 8 consecutive elements (row, n..n+7) as raw input, zero outside.

@@ -10,10 +10,13 @@
 // per wave).  Per 32-wide K step a wave reads 8 + 8 fragments for 64 MFMAs
 // (the 128 x 128-block kernel: 8 + 8 for 32).  Each output's N steps run in
 // ascending order, 32 at a time, as in the other MFMA SDDMM kernels, so all of
-// them give the same result.  A stage's 32 fragment reads are all issued
-// before its first MFMA (3% faster than reading each row of tiles' A fragment
-// just before its MFMAs); 32-value stages with four in flight measured 3-8%
-// slower.
+// them give the same result.  A K step's 16 fragment reads are issued before
+// the MFMAs of the step before it (83.2 us against 84.2 with a stage's reads
+// before its first MFMA, 4096 x 4096 x 2048); 32-value stages with four in
+// flight measured 3-8% slower.  At that size the kernel and the pass before it
+// take 74 us: about 1.6 us a stage (1.07 of it MFMAs at one wave per SIMD) and
+// 18 us for the first copies and the stores (28 us and more before the stores'
+// words were read a row tile at a time).
 #include "mfma_common.hpp"
 
 namespace bws {
@@ -99,85 +102,100 @@ k_sddmm_mfma_big(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t l
 #pragma unroll
     for (int b = 0; b < 8; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int64_t nst = N / NS;
-#pragma unroll
-  for (int p = 0; p < NBUF - 1; ++p)
-    if (p < nst) issue(p);
+  const int nst = (int)(N / NS);
   // fragment rows 16x + j of the wave's 128 rows (the swizzle depends only on
   // j since 16x is a multiple of 16)
   const uint32_t row_c = (uint32_t)((128 * wm + j) * ROWB);
   const uint32_t row_b = (uint32_t)((128 * wn + j) * ROWB);
+  struct Frags {  // of one K step
+    uint4 a[8], b[8];
+  };
+  auto load = [&](int st, int ks, Frags& f) {
+    const uint32_t chunk = (uint32_t)(st % NBUF) * STAGE + (uint32_t)(16 * slot_of(j, 4 * ks + q));
+    const uint8_t* bufC = &sC[0][0] + row_c + chunk;
+    const uint8_t* bufB = &sB[0][0] + row_b + chunk;
+#pragma unroll
+    for (int a = 0; a < 8; ++a) f.a[a] = *reinterpret_cast<const uint4*>(bufC + a * 16 * ROWB);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) f.b[b] = *reinterpret_cast<const uint4*>(bufB + b * 16 * ROWB);
+  };
+  auto multiply = [&](const Frags& f) {
+#pragma unroll
+    for (int a = 0; a < 8; ++a)
+#pragma unroll
+      for (int b = 0; b < 8; ++b) acc[a][b] = mfma<PREC>(f.a[a], f.b[b], acc[a][b]);
+  };
 
-  for (int64_t st = 0; st < nst; ++st) {
-    // stage st has landed when at most the later stages' copies are out
-    // (up to NBUF - 2 stages were issued after it)
-    {
-      const int64_t later = nst - 1 - st < NBUF - 2 ? nst - 1 - st : NBUF - 2;
-      static_assert(NBUF >= 2 && NBUF <= 5, "two to five stages");
-      if (NBUF >= 5 && later >= 3) wait_vmcnt<(NBUF >= 5 ? 3 : 0) * 2 * NC_W>();
-      else if (NBUF >= 4 && later >= 2) wait_vmcnt<(NBUF >= 4 ? 2 : 0) * 2 * NC_W>();
-      else if (NBUF >= 3 && later >= 1) wait_vmcnt<(NBUF >= 3 ? 1 : 0) * 2 * NC_W>();
-      else wait_vmcnt<0>();
-    }
-    __syncthreads();  // every wave's copies of stage st; stage st-1's buffer is free
-    if (st + NBUF - 1 < nst) issue(st + NBUF - 1);
-    const uint8_t* bufC = &sC[0][0] + (uint32_t)(st % NBUF) * STAGE;
-    const uint8_t* bufB = &sB[0][0] + (uint32_t)(st % NBUF) * STAGE;
-    // every fragment of the stage is requested before its first MFMA: with
-    // one wave per SIMD nothing else hides an LDS read's latency, and left to
-    // itself the compiler reloads one A fragment register per row of tiles
-    uint4 af[KSTEPS][8], bf[KSTEPS][8];
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      const uint32_t chunk = (uint32_t)(16 * slot_of(j, 4 * ks + q));
-#pragma unroll
-      for (int a = 0; a < 8; ++a)
-        af[ks][a] = *reinterpret_cast<const uint4*>(bufC + row_c + chunk + a * 16 * ROWB);
-#pragma unroll
-      for (int b = 0; b < 8; ++b)
-        bf[ks][b] = *reinterpret_cast<const uint4*>(bufB + row_b + chunk + b * 16 * ROWB);
-    }
+  // With one wave per SIMD nothing but the wave's own MFMAs hides an LDS read:
+  // the fragments of a K step are requested before the MFMAs of the step before
+  // it, across the stage's barrier too (past the last stage they see an old
+  // buffer and are not used).
+  static_assert(NBUF == 2 && KSTEPS == 2, "one stage on its way, two K steps a stage");
+  issue(0);
+  wait_vmcnt<0>();
+  __syncthreads();
+  if (nst > 1) issue(1);
+  Frags f0, f1;
+  load(0, 0, f0);
+  for (int st = 0; st < nst; ++st) {
+    load(st, 1, f1);
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks)
-#pragma unroll
-      for (int a = 0; a < 8; ++a)
-#pragma unroll
-        for (int b = 0; b < 8; ++b) acc[a][b] = mfma<PREC>(af[ks][a], bf[ks][b], acc[a][b]);
+    multiply(f0);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<0>();  // stage st + 1, issued a stage ago
+    __syncthreads();  // every wave's copies of it; stage st's fragments are all read
+    if (st + 2 < nst) issue(st + 2);
+    load(st + 1, 0, f0);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(f1);
+    __builtin_amdgcn_sched_barrier(0);
   }
 
   // Epilogue.  The block's bitmap words and the value index of each word's
-  // first bit are staged in LDS (over the operand buffers), so the stores
-  // below only read LDS: lane (j, q) holds rows 4q + e of each 16-row tile
-  // and column j of each 16-column tile; only set bits are stored.
+  // first bit are staged in LDS (over the operand buffers): lane (j, q) holds
+  // rows 4q + e of each 16-row tile and column j of each 16-column tile; only
+  // set bits are stored.  A row's four words and bases of the wave's columns are
+  // read for a whole row tile before its stores: with a read and a wait per
+  // output the epilogue was 28 of 84 us at 4096 x 4096 x 2048.
   __syncthreads();  // every wave is done with the operand buffers
-  uint32_t* eW = reinterpret_cast<uint32_t*>(&sC[0][0]);        // [BT][BT / 32] words
-  int64_t* eBase = reinterpret_cast<int64_t*>(&sC[1][0]);       // [BT][BT / 32] value indices
-  for (int t = tid; t < BT * (BT / 32); t += 256) {
-    const int64_t r = r0 + (t >> 3), w = k0 / 32 + (t & 7);
-    uint32_t word = 0u;
-    int64_t base = 0;
-    if (r < M && w < wpr) {
-      word = W[r * ldw + w] & valid_bits(w, K);
-      base = row_ptr[r] + woff[r * wpr + w];
-    }
-    eW[t] = word;
-    eBase[t] = base;
+  constexpr int WPB = BT / 32;                                  // words per block row
+  uint32_t* eW = reinterpret_cast<uint32_t*>(&sC[0][0]);        // [BT][WPB] words
+  int64_t* eBase = reinterpret_cast<int64_t*>(&sC[1][0]);       // [BT][WPB] value indices
+#pragma unroll
+  for (int t0 = 0; t0 < BT * WPB; t0 += 256) {
+    const int t = t0 + tid;
+    const int64_t r = r0 + t / WPB, w = k0 / 32 + t % WPB;
+    const int64_t rc = r < M ? r : M - 1, wc = w < wpr ? w : wpr - 1;
+    const uint32_t word = W[rc * ldw + wc];
+    eBase[t] = row_ptr[rc] + woff[rc * wpr + wc];
+    eW[t] = r < M && w < wpr ? word & valid_bits(w, K) : 0u;
   }
   __syncthreads();
+  const uint32_t bit[2] = {wbit(j), wbit(16 + j)};
+  const uint32_t before[2] = {~(0xFFFFFFFFu >> j), ~(0xFFFFFFFFu >> (16 + j))};
 #pragma unroll
-  for (int a = 0; a < 8; ++a)
+  for (int a = 0; a < 8; ++a) {
+    uint4 word[4];
+    longlong2 base[4][2];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int rr = 128 * wm + 16 * a + 4 * q + e;
+      const int ew = (128 * wm + 16 * a + 4 * q + e) * WPB + 4 * wn;
+      word[e] = *reinterpret_cast<const uint4*>(eW + ew);
+      base[e][0] = *reinterpret_cast<const longlong2*>(eBase + ew);
+      base[e][1] = *reinterpret_cast<const longlong2*>(eBase + ew + 2);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
-        const int ew = rr * (BT / 32) + 4 * wn + (b >> 1);
-        const uint32_t word = eW[ew];
-        const int i = 16 * (b & 1) + j;
-        if (word & wbit(i)) dA[eBase[ew] + rank_before(word, i)] = acc[a][b][e];
+        const uint32_t x = (b >> 1) == 0 ? word[e].x : (b >> 1) == 1 ? word[e].y
+                           : (b >> 1) == 2 ? word[e].z : word[e].w;
+        const longlong2 p = base[e][b >> 2];
+        const int64_t at = (b >> 1) & 1 ? p.y : p.x;
+        if (x & bit[b & 1]) dA[at + __popc(x & before[b & 1])] = acc[a][b][e];
       }
-    }
+  }
 }
 
 }  // namespace
