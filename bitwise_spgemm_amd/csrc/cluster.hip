@@ -309,18 +309,26 @@ k_assign(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
             srw[i0 + 2 * s][k] = rb * kPassRows + i0 + 2 * s < M ? x[s] & vb : 0u;
         }
         __syncthreads();
+        // a leader's word is read once for the wave's four rows, 8 words at a time
+        // (a row at a time, four words at a time: 13.9 us against 8.8 at 4096², 60
+        // leaders, the reads' latency)
+        const uint32_t(*rw)[kLeadWords] = srw + wave * 4;
+        for (int k = 0; k < n; k += 8) {
+          uint32_t x[8];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t* rw = srw[wave * 4 + q];
-          uint32_t acc = d[q];
-          for (int k = 0; k < n; k += 4) {
-            const uint4 y = *reinterpret_cast<const uint4*>(rw + k);
-            acc += __popc(sl[k * kLeadPitch + lane] ^ y.x) +
-                   __popc(sl[(k + 1) * kLeadPitch + lane] ^ y.y) +
-                   __popc(sl[(k + 2) * kLeadPitch + lane] ^ y.z) +
-                   __popc(sl[(k + 3) * kLeadPitch + lane] ^ y.w);
-          }
-          d[q] = acc;
+          for (int e = 0; e < 8; ++e) x[e] = sl[(k + e) * kLeadPitch + lane];
+          uint4 y[4][2];
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+              y[q][h] = *reinterpret_cast<const uint4*>(rw[q] + k + 4 * h);
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            d[q] += __popc(x[0] ^ y[q][0].x) + __popc(x[1] ^ y[q][0].y) +
+                    __popc(x[2] ^ y[q][0].z) + __popc(x[3] ^ y[q][0].w) +
+                    __popc(x[4] ^ y[q][1].x) + __popc(x[5] ^ y[q][1].y) +
+                    __popc(x[6] ^ y[q][1].z) + __popc(x[7] ^ y[q][1].w);
         }
       }
 #pragma unroll
