@@ -1,13 +1,13 @@
 // group.hip — row grouping by bitmask (first-fit disjoint groups per tile of
 // tile_rows rows x one 32-column word), spilled-row CSR, un-grouping.
 //
-// One wave (its own workgroup, so that the tiles spread over every CU and no
-// two placement chains share a CU's scalar unit) owns one tile and walks its
-// rows 64 at a time (lane l <-> row j0 + l).  Per chunk one vector pass finds
-// the lanes that fit some group against the masks as the chunk starts; the
-// other non-zero lanes must spill (group masks only grow), and the candidates
-// are placed in ascending row order on the scalar unit against the current
-// masks.  The result equals the serial ascending-row first fit exactly.
+// A workgroup of one or four waves (tiles spread over every CU, no two placement
+// chains share a CU's scalar unit) owns one tile: the waves load its words, the first
+// walks its rows 64 at a time (lane l <-> row j0 + l) and places them, the waves
+// store the results.  Per chunk one vector pass finds the lanes that fit some
+// group; the first of them joins, and again from the rows after it, so that the
+// serial chain is one step per row that joins.  The result equals the serial
+// ascending-row first fit exactly.
 #include "bws_internal.hpp"
 
 namespace bws {
@@ -79,8 +79,8 @@ struct GroupMasks<0> {
   __device__ uint32_t lane_value(int) const { return v; }
 };
 
-template <bool HAS_VALUES, int GC>
-__global__ void __launch_bounds__(256)
+template <bool HAS_VALUES, int GC, int NW>
+__global__ void __launch_bounds__(64 * NW)
 k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t wpr,
              int64_t ldw,
              const int64_t* __restrict__ row_ptr, const float* __restrict__ values, int T, int G,
@@ -89,15 +89,13 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
              int32_t* __restrict__ spill_cnt, int32_t* __restrict__ spill_nnz,
              int32_t* __restrict__ spill_table, int32_t* __restrict__ spill_rev,
              unsigned long long* __restrict__ grouped_nnz, int64_t per_xcd) {
-  // A workgroup of four waves per tile: all of them load words and store results,
-  // the first alone places rows (that is sequential, and what bounds the kernel):
-  // 26.4 us with one wave for all of it, 20.9 so, at 4096² (5%, tiles of 2048 rows,
-  // two groups).
+  // All NW waves load words and store results, the first alone places rows (that
+  // is sequential, and what bounds the kernel).
   __shared__ uint32_t s_word[kGroupPF * 64];   // the words of a group of chunks
   __shared__ uint8_t s_gid[kGroupPF * 64];     // group of the rows that joined one
   __shared__ uint64_t s_joined[kGroupPF];      // which rows of a chunk those are
   __shared__ int32_t s_base[kGroupPF + 1];     // spilled rows before a chunk
-  __shared__ int32_t s_nnz[4];
+  __shared__ int32_t s_nnz[NW];
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // XCD-contiguous tile ranges: the tiles of neighbouring words of the same
@@ -114,6 +112,7 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
     // 0/1 masks with a compile-time group count: lane i < 32 holds the member
     // row of bit i of each group, written once per tile
     constexpr bool kRegMembers = !HAS_VALUES && GC > 0;
+    constexpr bool kRefit = NW > 1 && (GC == 1 || GC == 2);
     int32_t mem[GC > 0 ? GC : 1];
 #pragma unroll
     for (int g = 0; g < (GC > 0 ? GC : 1); ++g) mem[g] = -1;
@@ -124,9 +123,9 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
     // word read with v_readlane), and the candidates are taken anew from the
     // later rows.  The group masks only grow, so a row passed over would not
     // have fitted in its turn: this is the serial ascending-row first fit
-    // exactly, in as many steps as rows join (at most 32 G bits a tile; stepping
-    // through all candidates of the chunk's start: 26.9 us against 26.4 at 4096²,
-    // 5%, tiles of 2048 rows, two groups).
+    // exactly, in as many steps as rows join.  With more than two groups, where
+    // testing all rows again costs more than passing over some, and in short
+    // tiles, where most candidates join, it steps through the chunk's candidates.
     auto chunk = [&](int j0, uint32_t m, int u) {
       int32_t gid = 0;
       const uint64_t nz = __ballot(m != 0u);
@@ -135,15 +134,16 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
       while (cand) {
         const int jl = (int)__builtin_ctzll(cand);
         const uint32_t mj = (uint32_t)__builtin_amdgcn_readlane((int)m, jl);
-        const int gj = gms.fit(mj, G);  // < G
-        joined |= 1ull << jl;
-        gid = lane == jl ? gj : gid;
+        const int gj = gms.fit(mj, G);
+        const bool ok = gj < G;
+        joined |= (uint64_t)ok << jl;
+        gid = lane == jl && ok ? gj : gid;
         gms.add(gj, mj, lane);
         if constexpr (kRegMembers) {
           const bool mine = (mj & wbit(lane & 31)) != 0u;
 #pragma unroll
           for (int g = 0; g < (GC > 0 ? GC : 1); ++g) mem[g] = mine && g == gj ? j0 + jl : mem[g];
-        } else {
+        } else if (ok) {
           int64_t vbase = 0;
           if (HAS_VALUES) {
             const int64_t r = row0 + j0 + jl;
@@ -157,34 +157,53 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
             group_vals[idx] = HAS_VALUES ? values[vbase + rank_before(mj, lane)] : 1.0f;
           }
         }
-        cand = __ballot(m != 0u && gms.fit(m, G) < G) & ~((2ull << jl) - 1ull);
+        if constexpr (kRefit) cand = __ballot(m != 0u && gms.fit(m, G) < G) & ~((2ull << jl) - 1ull);
+        else cand &= cand - 1ull;
       }
-      if (joined) s_gid[u * 64 + lane] = (uint8_t)gid;
-      if (lane == 0) {
-        s_joined[u] = joined;
-        s_base[u] = cnt;
+      const uint64_t spillers = nz & ~joined;
+      if constexpr (NW > 1) {
+        if (joined) s_gid[u * 64 + lane] = (uint8_t)gid;
+        if (lane == 0) {
+          s_joined[u] = joined;
+          s_base[u] = cnt;
+        }
+      } else {  // the row's result in place of its word: (slot + 1) << 8 | (group + 1)
+        int32_t slot = -1;
+        if ((spillers >> lane) & 1ull) {
+          slot = cnt + __popcll(spillers & ((1ull << lane) - 1ull));
+          gid = -1;
+          snnz_lane += __popc(m);
+        }
+        s_word[u * 64 + lane] = ((uint32_t)(slot + 1) << 8) | (uint32_t)(gid + 1);
       }
-      cnt += __popcll(nz & ~joined);
+      cnt += __popcll(spillers);
     };
     const uint32_t vb = valid_bits(w, cols);
     for (int b0 = 0; b0 < nrows; b0 += 64 * kGroupPF) {
       const int nch = min(kGroupPF, (nrows - b0 + 63) / 64);
-      // a wave's chunks are wave, wave + 4, ..; loads four chunks at a time under a
-      // wave-uniform test, unconditional within it (rows past the tile read its
-      // last row and are zeroed)
+      // a wave's chunks are wave, wave + NW, ..: their words are all loaded before
+      // the first is placed, four chunks at a time under a wave-uniform test,
+      // unconditional within it (rows past the tile read its last row and are
+      // zeroed)
       if (b0) __syncthreads();  // the words before have been read
+      constexpr int kPer = kGroupPF / NW;
+      uint32_t mm[kPer];
 #pragma unroll
-      for (int q = 0; q < kGroupPF / 4; q += 4) {
-        if (4 * q < nch) {
-          uint32_t mm[4];
+      for (int q = 0; q < kPer; q += 4) {
+        if (NW * q < nch) {
 #pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            const int j = b0 + 64 * (4 * (q + x) + wave) + lane;
+          for (int x = q; x < q + 4; ++x) {
+            const int j = b0 + 64 * (NW * x + wave) + lane;
             mm[x] = W[(row0 + (j < nrows ? j : nrows - 1)) * ldw + w];
           }
+        }
+      }
 #pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            const int u = 4 * (q + x) + wave;
+      for (int q = 0; q < kPer; q += 4) {
+        if (NW * q < nch) {
+#pragma unroll
+          for (int x = q; x < q + 4; ++x) {
+            const int u = NW * x + wave;
             s_word[u * 64 + lane] = b0 + 64 * u + lane < nrows ? mm[x] & vb : 0u;
           }
         }
@@ -202,19 +221,25 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
       }
       __syncthreads();
 #pragma unroll 2
-      for (int u = wave; u < nch; u += 4) {
+      for (int u = wave; u < nch; u += NW) {
         const int j = b0 + 64 * u + lane;
         const uint32_t m = s_word[u * 64 + lane];
-        const bool joined = (s_joined[u] >> lane) & 1ull;
-        const bool spill = m != 0u && !joined;
-        const uint64_t spillers = __ballot(spill);
-        const int32_t slot =
-            spill ? s_base[u] + __popcll(spillers & ((1ull << lane) - 1ull)) : -1;
-        if (spill) snnz_lane += __popc(m);
+        int32_t gid, slot;
+        if constexpr (NW > 1) {
+          const bool joined = (s_joined[u] >> lane) & 1ull;
+          const bool spill = m != 0u && !joined;
+          const uint64_t spillers = __ballot(spill);
+          slot = spill ? s_base[u] + __popcll(spillers & ((1ull << lane) - 1ull)) : -1;
+          gid = joined ? (int32_t)s_gid[u * 64 + lane] : spill ? -1 : 0;
+          if (spill) snnz_lane += __popc(m);
+        } else {
+          slot = (int32_t)(m >> 8) - 1;
+          gid = (int32_t)(m & 0xffu) - 1;
+        }
         if (j < nrows) {
-          group_id[(row0 + j) * ldw + w] = joined ? (int32_t)s_gid[u * 64 + lane] : spill ? -1 : 0;
+          group_id[(row0 + j) * ldw + w] = gid;
           if (spill_rev) spill_rev[t * T + j] = slot;
-          if (spill_table && spill) spill_table[t * T + slot] = j;
+          if (spill_table && slot >= 0) spill_table[t * T + slot] = j;
         }
       }
     }
@@ -223,9 +248,9 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
     if (lane == 0) s_nnz[wave] = snnz_wave;
     __syncthreads();
     if (spill_rev)
-      for (int j = nrows + threadIdx.x; j < T; j += 256) spill_rev[t * T + j] = -1;
+      for (int j = nrows + threadIdx.x; j < T; j += 64 * NW) spill_rev[t * T + j] = -1;
     if (spill_table)
-      for (int s = cnt + threadIdx.x; s < T; s += 256) spill_table[t * T + s] = 0;
+      for (int s = cnt + threadIdx.x; s < T; s += 64 * NW) spill_table[t * T + s] = 0;
     if (wave != 0) continue;
     if constexpr (kRegMembers) {
 #pragma unroll
@@ -249,7 +274,9 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
     }
     const uint32_t gm_lane = gms.lane_value(lane);
     if (lane < G) group_mask[t * G + lane] = gm_lane;
-    const int32_t snnz = s_nnz[0] + s_nnz[1] + s_nnz[2] + s_nnz[3];
+    int32_t snnz = 0;
+#pragma unroll
+    for (int x = 0; x < NW; ++x) snnz += s_nnz[x];
     const int32_t tile_nnz = wave_sum(lane < G ? __popc(gm_lane) : 0);
     if (lane == 0) {
       spill_cnt[t] = cnt;
@@ -359,20 +386,30 @@ bws_status bws_group_rows(const bws_bitmap* A, int32_t tile_rows, int32_t max_gr
   const int64_t per_xcd = ceil_div(tiles, 8);
   // a multiple of 8 (each workgroup keeps to one XCD's range), at most 65536
   const int grid = (int)(8 * per_xcd < 65536 ? 8 * per_xcd : 65536);
-#define BWS_GROUP(HV, GC)                                                                   \
-  hipLaunchKernelGGL((k_group_rows<HV, GC>), dim3(grid), dim3(256), 0, stream,                    \
+#define BWS_GROUP_W(HV, GC, NW)                                                             \
+  hipLaunchKernelGGL((k_group_rows<HV, GC, NW>), dim3(grid), dim3(64 * NW), 0, stream,            \
                      A->words, A->rows, A->cols, wpr, A->ldw, A->row_ptr, A->values,            \
                      (int)tile_rows, (int)max_groups, tiles, out->group_id, out->group_mask,     \
                      out->group_vals, out->member_row, out->spill_cnt, out->spill_nnz,          \
                      out->spill_table, out->spill_rev, gn, per_xcd)
+#define BWS_GROUP(HV, GC)                      \
+  do {                                         \
+    if (wide) BWS_GROUP_W(HV, GC, 4);          \
+    else BWS_GROUP_W(HV, GC, 1);               \
+  } while (0)
 #define BWS_GROUP_G(HV)              \
   switch (max_groups) {              \
     case 1: BWS_GROUP(HV, 1); break; \
     case 2: BWS_GROUP(HV, 2); break; \
     case 3: BWS_GROUP(HV, 3); break; \
     case 4: BWS_GROUP(HV, 4); break; \
-    default: BWS_GROUP(HV, 0);       \
+    default: BWS_GROUP_W(HV, 0, 1);  \
   }
+  // Four waves where the tiles are long and few enough that the waiting ones take
+  // nobody's place (us, one wave | four): 4096², 2048-row tiles, 2 groups 26.0 | 22.8,
+  // 512 rows 28.1 | 25.9; 8192², 2048 rows (1024 tiles) 46.4 | 36.2, 1024 rows, 4
+  // groups (2048 tiles) 57.4 | 62.0; 4096², 256 rows 38.1 | 39.1.
+  const bool wide = tile_rows >= 512 && tiles <= 1024;
   if (A->values) {
     BWS_GROUP_G(true);
   } else {
@@ -380,6 +417,7 @@ bws_status bws_group_rows(const bws_bitmap* A, int32_t tile_rows, int32_t max_gr
   }
 #undef BWS_GROUP_G
 #undef BWS_GROUP
+#undef BWS_GROUP_W
   return launch_check();
 }
 
