@@ -202,11 +202,15 @@ def _check(status: int, where: str):
 
 
 def _stream(device=None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the handle alone: a stream object per call is a microsecond of a call that
+    # takes seven on the GPU
+    index = None if device is None else torch.device(device).index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index)
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _require_gpu(*tensors):
