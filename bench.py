@@ -251,7 +251,7 @@ def main():
         alg_bytes += 4 * M + 4 * 2 * ((M + 15) // 16) * ((K + 31) // 32)
     achieved = alg_bytes / (ms_kernel * 1e-3) / 1e9
     kname = {"fp32_rowclusters": "k_spmm_stream<true>",
-             "fp32": "k_spmm_stream<false>"}.get(path)
+             "fp32": "k_spmm_f32"}.get(path)
     traffic = None
     traffic_note = None
     tfile = PROFILE_TRAFFIC.format(path)
