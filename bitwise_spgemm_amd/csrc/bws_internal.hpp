@@ -119,7 +119,7 @@ bool spmm_direct_ok(const bws_bitmap* A, int64_t ldb, int64_t N, int64_t max_til
 bws_status launch_spmm_direct(const bws_bitmap* A, const float* B, int64_t ldb, int64_t N,
                               float* C, int64_t ldc, float alpha, float beta, hipStream_t s);
 // 16-bit precisions, small outputs with a long K, in one launch (spmm_direct16.hip).
-bool spmm_direct16_ok(const bws_bitmap* A, int64_t ldb, int64_t N);
+bool spmm_direct16_ok(const bws_bitmap* A, int32_t precision, int64_t ldb, int64_t N);
 bws_status launch_spmm_direct16(const bws_bitmap* A, const void* B, int32_t b_dtype,
                                 int32_t precision, int64_t ldb, int64_t N, float* C, int64_t ldc,
                                 float alpha, float beta, hipStream_t s);

@@ -292,9 +292,9 @@ bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t
       workspace_bytes >= spmm_vals_workspace(A) &&
       (reinterpret_cast<uintptr_t>(workspace) & 255u) == 0)
     return spmm_mfma_vals(A, B, precision, ldb, N, C, ldc, alpha, beta, workspace, stream);
-  // BF16 / FP16 on a 0/1 A without a plan: small outputs with a long K
-  if (!A->values && A->cols > 0 && !plan &&
-      (precision == BWS_PREC_BF16 || precision == BWS_PREC_FP16) && spmm_direct16_ok(A, ldb, N))
+  // 16-bit precisions on a 0/1 A without a plan: small outputs with a long K
+  if (!A->values && A->cols > 0 && !plan && precision != BWS_PREC_FP32 &&
+      spmm_direct16_ok(A, precision, ldb, N))
     return launch_spmm_direct16(A, B, b_dtype, precision, ldb, N, C, ldc, alpha, beta, stream);
   // BF16 / FP16 on a 0/1 A with the plan's density split (mfma_min_bits > 0):
   // the 128-row blocks with fewer than mfma_min_bits set bits per 64 K columns

@@ -1,5 +1,5 @@
-// spmm_direct16.hip — 16-bit product of a 0/1 bitmap for small outputs with a
-// long K, in one launch without a workspace (gfx950, v_mfma_f32_16x16x32).
+// spmm_direct16.hip — 16-bit and split-BF16 product of a 0/1 bitmap for small
+// outputs with a long K (split BF16: any K), in one launch without a workspace (gfx950, v_mfma_f32_16x16x32).
 //
 // The staged tiles of spmm_mfma.hip walk all of K in every workgroup, a barrier
 // and an LDS round trip per stage: with few tiles that chain is the time and
@@ -36,8 +36,7 @@ typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint16_t u16x4_u __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 
-// PREC 1 = BF16, 2 = FP16; F32: B is FP32 and rounded to it; kEA: MFMA tiles down
-// (4 or 8).
+// PREC 1 = BF16, 2 = FP16, 3 = BF16X2 (b = hi + lo, two products); F32: B is FP32 and rounded or split; kEA: MFMA tiles down (4 or 8).
 template <int PREC, bool F32, int kEA>
 __global__ void __launch_bounds__(DW * 64, 2)
 k_spmm_direct16(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
@@ -114,11 +113,17 @@ k_spmm_direct16(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ld
     }
   };
 
-  f32x4 acc[kEA][kEB];
+  // BF16X2: the sums of lo apart, so that its products do not lengthen the chain
+  // of the large ones (the matrix unit does not round its sums to nearest)
+  constexpr int NP = PREC == 3 ? 2 : 1;
+  f32x4 acc[kEA][kEB], low[PREC == 3 ? kEA : 1][kEB];
 #pragma unroll
   for (int a = 0; a < kEA; ++a)
 #pragma unroll
-    for (int b = 0; b < kEB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < kEB; ++b) {
+      acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (PREC == 3) low[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 
   auto multiply = [&](int s, Raw& r, auto fresh, auto next) {
     if (fresh.value && partial_quad) {  // the quad that holds column N - 1, loaded from N - 4 on
@@ -131,21 +136,25 @@ k_spmm_direct16(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ld
         r.v[e] = v;
       }
     }
-    uint4 bf[kEB];
+    uint4 bf[NP][kEB];
 #pragma unroll
     for (int b = 0; b < kEB; ++b) {
-      uint32_t d[4];
+      uint32_t d[4], l[4];
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
         if constexpr (F32) {
           const float x0 = r.v[2 * p][b], x1 = r.v[2 * p + 1][b];
           d[p] = PREC == 2 ? f32_to_f16_rne(x0) | f32_to_f16_rne(x1) << 16
                            : f32_to_bf16_rne(x0) | f32_to_bf16_rne(x1) << 16;
+          if constexpr (PREC == 3)
+            l[p] = f32_to_bf16_rne(x0 - __uint_as_float(d[p] << 16)) |
+                   f32_to_bf16_rne(x1 - __uint_as_float(d[p] & 0xFFFF0000u)) << 16;
         } else {
           d[p] = (uint32_t)r.v[2 * p][b] | (uint32_t)r.v[2 * p + 1][b] << 16;
         }
       }
-      bf[b] = make_uint4(d[0], d[1], d[2], d[3]);
+      bf[0][b] = make_uint4(d[0], d[1], d[2], d[3]);
+      if constexpr (PREC == 3) bf[NP - 1][b] = make_uint4(l[0], l[1], l[2], l[3]);
     }
     uint32_t w[kEA];
 #pragma unroll
@@ -160,9 +169,13 @@ k_spmm_direct16(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ld
     for (int a = 0; a < kEA; ++a) {
       const uint4 af = a_frag_bits<PREC>(w[a], q);
 #pragma unroll
-      for (int b = 0; b < kEB; ++b) acc[a][b] = mfma<PREC>(bf[b], af, acc[a][b]);
+      for (int b = 0; b < kEB; ++b) acc[a][b] = mfma<PREC>(bf[0][b], af, acc[a][b]);
+      if constexpr (PREC == 3) {
 #pragma unroll
-      for (int b = 0; b < kEB; ++b) {  // the next row tile's operand between them
+        for (int b = 0; b < kEB; ++b) low[a][b] = mfma<PREC>(bf[NP - 1][b], af, low[a][b]);
+      }
+#pragma unroll
+      for (int b = 0; b < NP * kEB; ++b) {  // the next row tile's operand between them
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
         __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // three VALU
       }
@@ -186,6 +199,12 @@ k_spmm_direct16(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ld
     }
   }
 
+  if constexpr (PREC == 3) {
+#pragma unroll
+    for (int a = 0; a < kEA; ++a)
+#pragma unroll
+      for (int b = 0; b < kEB; ++b) acc[a][b] += low[a][b];
+  }
   // partial tiles: every wave's through LDS, 64 rows at a time, then a pair of waves
   // adds and stores a row tile, each two of the four accumulators e
   constexpr int PER = 2;
@@ -238,7 +257,7 @@ template <int PREC, bool F32>
 bws_status launch_direct16(const bws_bitmap* A, const void* B, int64_t ldb, int64_t N, float* C,
                            int64_t ldc, float alpha, float beta, hipStream_t s) {
   const int64_t tiles64 = ceil_div(A->rows, 64) * ceil_div(N, 64);
-  const int64_t rows = tiles64 <= 256 ? 64 : 128;
+  const int64_t rows = PREC == 3 || tiles64 <= 256 ? 64 : 128;  // (256 accumulators a lane)
   const int64_t row_blocks = ceil_div(A->rows, rows), col_blocks = ceil_div(N, kEN);
   const int64_t per_xcd = ceil_div(row_blocks * col_blocks, 8);
   const int vec = ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
@@ -247,8 +266,13 @@ bws_status launch_direct16(const bws_bitmap* A, const void* B, int64_t ldb, int6
                        A->rows, A->cols, A->ldw, B, ldb, N, C, ldc, alpha, beta, row_blocks,
                        col_blocks, per_xcd, vec);
   };
-  if (rows == 64) launch(k_spmm_direct16<PREC, F32, 4>);
-  else launch(k_spmm_direct16<PREC, F32, 8>);
+  if constexpr (PREC != 3) {
+    if (rows == 128) {
+      launch(k_spmm_direct16<PREC, F32, 8>);
+      return launch_check();
+    }
+  }
+  launch(k_spmm_direct16<PREC, F32, 4>);
   return launch_check();
 }
 
@@ -256,10 +280,15 @@ bws_status launch_direct16(const bws_bitmap* A, const void* B, int64_t ldb, int6
 
 // Outputs of up to 256 tiles of 64 x 64 with K of at least 1280 and of up to 512
 // with 2048 (figures above): the staged tiles' time is K's, this kernel has about
-// 6 and 9 us besides.
-bool spmm_direct16_ok(const bws_bitmap* A, int64_t ldb, int64_t N) {
+// 6 and 9 us besides.  BF16X2 of up to 512: the other side is a pass that splits B
+// and two products; us, that | this: 200 x 16 x 100 10.4 | 5.6, 500 x 1000 x 300 19.8 |
+// 10.5, 1999 x 3100 x 1000 60.6 | 41.1; at 1024 tiles, 2048 x 256 x 2048, 23.0 | 27.2.
+bool spmm_direct16_ok(const bws_bitmap* A, int32_t precision, int64_t ldb, int64_t N) {
   const int64_t rows = ceil_div(A->rows, 64), cols = ceil_div(N, 64);
-  const int64_t most = A->cols < 1280 ? 0 : A->cols < 2048 ? 256 : 512;
+  const int64_t most = precision == BWS_PREC_BF16X2 ? 512
+                       : A->cols < 1280            ? 0
+                       : A->cols < 2048            ? 256
+                                                   : 512;
   return rows <= most && cols <= most && rows * cols <= most &&
          A->cols < ((int64_t)1 << 31) && ldb < (1 << 24);  // 32-bit steps and offsets
 }
@@ -268,6 +297,8 @@ bws_status launch_spmm_direct16(const bws_bitmap* A, const void* B, int32_t b_dt
                                 int32_t precision, int64_t ldb, int64_t N, float* C, int64_t ldc,
                                 float alpha, float beta, hipStream_t s) {
   const bool f32 = b_dtype == BWS_DTYPE_F32;
+  if (precision == BWS_PREC_BF16X2)
+    return launch_direct16<3, true>(A, B, ldb, N, C, ldc, alpha, beta, s);
   if (precision == BWS_PREC_FP16)
     return f32 ? launch_direct16<2, true>(A, B, ldb, N, C, ldc, alpha, beta, s)
                : launch_direct16<2, false>(A, B, ldb, N, C, ldc, alpha, beta, s);

@@ -376,7 +376,8 @@ typedef struct {
  * BF16 / FP16 with a 0/1 A and no plan: outputs of up to 256 tiles of 64 x 64 with K
  * of at least 1280, and of up to 512 with 2048, share K out over the waves of a
  * workgroup (the partial sums are added at the end: another summation order than
- * the other MFMA kernels', which a plan selects) and need no workspace.
+ * the other MFMA kernels', which a plan selects) and need no workspace; so do
+ * BF16X2 outputs of up to 512 such tiles.
  * precision/b_dtype combinations: FP32 with F32 (or exact BF16/F16 input);
  * BF16 with BF16 or F32 (rounded to nearest even); FP16 with F16 or F32;
  * BF16X2 with F32.
