@@ -199,34 +199,38 @@ k_spmm_direct16(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ld
     }
   }
 
-  if constexpr (PREC == 3) {
-#pragma unroll
-    for (int a = 0; a < kEA; ++a)
-#pragma unroll
-      for (int b = 0; b < kEB; ++b) acc[a][b] += low[a][b];
-  }
   // partial tiles: every wave's through LDS, 64 rows at a time, then a pair of waves
-  // adds and stores a row tile, each two of the four accumulators e
+  // adds and stores a row tile, each two of the four accumulators e.  BF16X2 adds
+  // the waves' hi sums and their lo sums apart and meets them in one rounding, as
+  // the product in two passes does: with lo added to each wave's hi sum before,
+  // K = 16384 at 50% with B in [1, 1.125) was 6.2e-8 of its norm off, 4.8e-8 there.
   constexpr int PER = 2;
   const int a = wave / 2, e0 = wave % 2 * PER;
   typedef float part_t __attribute__((ext_vector_type(PER)));
 #pragma unroll
   for (int h = 0; h < kEA / 4; ++h) {
-    __syncthreads();  // the words, or the rows before, have been read
-#pragma unroll
-    for (int i = 0; i < 4 * kEB; ++i) part[wave][i][lane] = acc[4 * h + i / kEB][i % kEB];
-    __syncthreads();
     const int64_t row = m0 + 64 * h + 16 * a + j;
     part_t sum[kEB];
 #pragma unroll
-    for (int b = 0; b < kEB; ++b) {
-      auto at = [&](int w) {
-        return *reinterpret_cast<const part_t*>(
-            reinterpret_cast<const float*>(&part[w][a * kEB + b][lane]) + e0);
-      };
-      sum[b] = at(0);
+    for (int p = 0; p < NP; ++p) {
+      __syncthreads();  // the words, or what was there before, have been read
 #pragma unroll
-      for (int w = 1; w < DW; ++w) sum[b] += at(w);
+      for (int i = 0; i < 4 * kEB; ++i) {
+        if (p == 0) part[wave][i][lane] = acc[4 * h + i / kEB][i % kEB];
+        else part[wave][i][lane] = low[4 * h + i / kEB][i % kEB];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int b = 0; b < kEB; ++b) {
+        auto at = [&](int w) {
+          return *reinterpret_cast<const part_t*>(
+              reinterpret_cast<const float*>(&part[w][a * kEB + b][lane]) + e0);
+        };
+        part_t x = at(0);
+#pragma unroll
+        for (int w = 1; w < DW; ++w) x += at(w);
+        sum[b] = p == 0 ? x : sum[b] + x;
+      }
     }
     if (row >= M) continue;
 #pragma unroll
@@ -281,8 +285,8 @@ bws_status launch_direct16(const bws_bitmap* A, const void* B, int64_t ldb, int6
 // Outputs of up to 256 tiles of 64 x 64 with K of at least 1280 and of up to 512
 // with 2048 (figures above): the staged tiles' time is K's, this kernel has about
 // 6 and 9 us besides.  BF16X2 of up to 512: the other side is a pass that splits B
-// and two products; us, that | this: 200 x 16 x 100 10.4 | 5.6, 500 x 1000 x 300 19.8 |
-// 10.5, 1999 x 3100 x 1000 60.6 | 41.1; at 1024 tiles, 2048 x 256 x 2048, 23.0 | 27.2.
+// and two products; us, that | this: 200 x 16 x 100 10.4 | 6.6, 500 x 1000 x 300 19.8 |
+// 11.5, 1999 x 3100 x 1000 60.6 | 42.1; at 1024 tiles, 2048 x 256 x 2048, 23.0 | 28.2.
 bool spmm_direct16_ok(const bws_bitmap* A, int32_t precision, int64_t ldb, int64_t N) {
   const int64_t rows = ceil_div(A->rows, 64), cols = ceil_div(N, 64);
   const int64_t most = precision == BWS_PREC_BF16X2 ? 512
