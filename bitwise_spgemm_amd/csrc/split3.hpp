@@ -15,9 +15,11 @@
 //
 // Range: the parts of |b| in [2^-100, 2^128) are normal BF16 numbers.  Of a
 // smaller b bits may be lost, and an Inf or NaN would spread to the rows that
-// do not select it (0 x Inf).  An output that is not finite or is below 2^-80
-// (for zero: only where some b was tiny) is therefore summed again from A's
-// bits and B in FP32, bit by bit, as the vector-add kernels do.
+// do not select it (0 x Inf).  The product over planes leaves columns that hold
+// such values to the vector adds (spmm_planes.hip); the one-launch product, which
+// meets them on the way, sums an output that is not finite or is below 2^-80 (for
+// zero: only where some b was tiny) again from A's bits and B in FP32, bit by bit,
+// as the vector-add kernels do.
 #pragma once
 
 #include "mfma_common.hpp"
@@ -27,6 +29,7 @@ namespace {
 
 constexpr int kPlanes = 3;
 constexpr uint32_t kTinyBits = (127u - 100u) << 23;  // 2^-100
+constexpr uint32_t kHugeBits = (127u + 96u) << 23;   // 2^96
 constexpr float kSmallOut = 0x1p-80f;
 
 // FP32 sum of column `col` of B over the set bits of one row of A, ascending k.

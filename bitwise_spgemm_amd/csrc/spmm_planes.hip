@@ -20,15 +20,20 @@
 // The planes' unit is a block of 32 K rows x 16 columns, 1 KiB, in which lane l
 // of a wave finds its 8 K values (rows 8(l/16) .. +7 of column l % 16) as 16
 // contiguous bytes: copies into LDS and fragment reads are linear, without
-// swizzle or transpose.  A tiny nonzero b is written as +2^-120: no sum that
-// holds it is exactly zero, so its outputs are noticed.
+// swizzle or transpose.
+//
+// B out of the planes' range (infinities, NaN, values from 2^96 on, whose sums may
+// overflow, and nonzero ones below 2^-100, whose parts lose bits): the split marks
+// its 64 columns, and every 256 x 256 output over marked columns takes the
+// streamed tile, which adds B itself.  A dense mask then costs what it does there
+// and the 22 us of the split (4096³, 50%: 1.2 ms for such columns); summed again
+// output by output after the product, one NaN in B took 1.9 ms and a B of 1e-35
+// 53 ms.
 #include "split3.hpp"
 #include "stream_tile.hpp"
 
 namespace bws {
 namespace {
-
-constexpr uint32_t kTinyMark = (127u - 120u) << 23;  // 2^-120, exact in BF16
 
 // The matrix tile: 256 x 128 outputs, 4 x 4 waves of 64 x 32 each, two 32-row K
 // steps per LDS stage and three stages (150 KiB: one workgroup per CU, four waves
@@ -58,9 +63,9 @@ __device__ __forceinline__ void dma16_lin(uint32_t lane_off, const void* base, u
 // Rows m0 .. +255 and columns n0 .. +127 of C.
 __device__ __forceinline__ void planes_tile(const uint32_t* __restrict__ W, int64_t M, int64_t K,
                                             int64_t ldw, const uint8_t* __restrict__ planes,
-                                            const float* __restrict__ B, int64_t ldb, int64_t N,
-                                            float* __restrict__ C, int64_t ldc, float alpha,
-                                            float beta, int64_t m0, int64_t n0, uint8_t* smem) {
+                                            int64_t N, float* __restrict__ C, int64_t ldc,
+                                            float alpha, float beta, int64_t m0, int64_t n0,
+                                            uint8_t* smem) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / kPWaves, wn = wave % kPWaves;
@@ -157,7 +162,6 @@ __device__ __forceinline__ void planes_tile(const uint32_t* __restrict__ W, int6
 
   // lane (j, q) holds row 16a + j, columns 16b + 4q .. +3 of the wave's tile
   // (N a multiple of 4 and 16-byte rows of C, as the streamed tile needs)
-  uint32_t redo = 0;
 #pragma unroll
   for (int a = 0; a < kPA; ++a) {
     const int64_t row = m0 + (wm * kPA + a) * 16 + j;
@@ -165,58 +169,44 @@ __device__ __forceinline__ void planes_tile(const uint32_t* __restrict__ W, int6
     for (int b = 0; b < kPB; ++b) {
       const int64_t col = n0 + (wn * kPB + b) * 16 + 4 * q;
       if (row >= M || col >= N) continue;
-      float* c = C + row * ldc + col;
-      uint32_t bad = 0;
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float x = acc[a][b][e];
-        if (out_of_range(x)) bad |= 1u << e;
-        v[e] = alpha * x;
+      float4* c = reinterpret_cast<float4*>(C + row * ldc + col);
+      f32x4 v = acc[a][b] * alpha;
+      if (beta != 0.0f) {
+        const float4 o = *c;
+        v.x = fmaf(beta, o.x, v.x);
+        v.y = fmaf(beta, o.y, v.y);
+        v.z = fmaf(beta, o.z, v.z);
+        v.w = fmaf(beta, o.w, v.w);
       }
-      redo |= bad << (4 * (a * kPB + b));
-      if (bad == 0) {
-        if (beta != 0.0f) {
-          const float4 o = *reinterpret_cast<const float4*>(c);
-          v[0] = fmaf(beta, o.x, v[0]);
-          v[1] = fmaf(beta, o.y, v[1]);
-          v[2] = fmaf(beta, o.z, v[2]);
-          v[3] = fmaf(beta, o.w, v[3]);
-        }
-        *reinterpret_cast<float4*>(c) = make_float4(v[0], v[1], v[2], v[3]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (!((bad >> e) & 1u)) c[e] = beta != 0.0f ? fmaf(beta, c[e], v[e]) : v[e];
-      }
+      *c = make_float4(v.x, v.y, v.z, v.w);
     }
   }
-  static_assert(kPA * kPB * 4 <= 32, "one bit per output of a lane");
-  // outputs out of the planes' range, from A's bits and B themselves
-  while (redo) {
-    const int i = __builtin_ctz(redo);
-    redo &= redo - 1;
-    const int64_t row = m0 + (wm * kPA + (i >> 2) / kPB) * 16 + j;
-    const int64_t col = n0 + (wn * kPB + (i >> 2) % kPB) * 16 + 4 * q + (i & 3);
-    const float x = alpha * row_sum(W + row * ldw, K, B + col, ldb);
-    float* c = C + row * ldc + col;
-    *c = beta != 0.0f ? fmaf(beta, *c, x) : x;
-  }
+}
+
+// Whether columns n0 .. n0 + 255 hold a marked value (marks: planes_block).
+__device__ __forceinline__ bool cols_marked(const uint32_t* __restrict__ marks, int64_t nks,
+                                            int64_t n0, int64_t N) {
+  const int64_t first = n0 / 64 * nks;
+  const int64_t last = (n0 + kQBN < N ? (n0 + kQBN) / 64 : ceil_div(N, 64)) * nks;
+  uint32_t any = 0u;
+  for (int64_t i = first + threadIdx.x; i < last; i += kQW * 64) any |= marks[i];
+  return __syncthreads_or(any != 0u) != 0;
 }
 
 __global__ void __launch_bounds__(kQW * 64)
 k_spmm_f32(const uint32_t* __restrict__ dense, const uint32_t* __restrict__ S,
-           const uint8_t* __restrict__ planes, const uint32_t* __restrict__ W, int64_t M,
-           int64_t K, int64_t ldw, const float* __restrict__ B, int64_t ldb, int64_t N,
-           float* __restrict__ C, int64_t ldc, float alpha, float beta, int64_t row_blocks,
-           int64_t col_blocks, int64_t per_xcd) {
+           const uint8_t* __restrict__ planes, const uint32_t* __restrict__ marks,
+           const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
+           const float* __restrict__ B, int64_t ldb, int64_t N, float* __restrict__ C,
+           int64_t ldc, float alpha, float beta, int64_t row_blocks, int64_t col_blocks,
+           int64_t per_xcd) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kPLds > kStreamLds ? kPLds : kStreamLds];
   const int64_t tile = xcd_tile(blockIdx.x, per_xcd);
   if (tile >= row_blocks * col_blocks) return;
-  if (dense[0] != 0u) {
-    const int64_t m0 = (tile % row_blocks) * kQRows, n0 = (tile / row_blocks) * kQBN;
+  const int64_t m0 = (tile % row_blocks) * kQRows, n0 = (tile / row_blocks) * kQBN;
+  if (dense[0] != 0u && !cols_marked(marks, ceil_div(K, 32), n0, N)) {
     for (int64_t n = n0; n < n0 + kQBN && n < N; n += kPN) {
-      planes_tile(W, M, K, ldw, planes, B, ldb, N, C, ldc, alpha, beta, m0, n, smem);
+      planes_tile(W, M, K, ldw, planes, N, C, ldc, alpha, beta, m0, n, smem);
       __syncthreads();  // the next half writes the stages
     }
   } else
@@ -226,14 +216,10 @@ k_spmm_f32(const uint32_t* __restrict__ dense, const uint32_t* __restrict__ S,
 
 // hi, mid and lo of b, each in the low 16 bits.
 __device__ __forceinline__ void split3(float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  uint32_t u = __float_as_uint(b);
-  const uint32_t mag = u & 0x7FFFFFFFu;
-  if (mag - 1u < kTinyBits - 1u) u = kTinyMark;
-  const uint32_t h = u & 0xFFFF0000u;
-  const float r = __uint_as_float(u) - __uint_as_float(h);  // exact
+  const uint32_t h = __float_as_uint(b) & 0xFFFF0000u;
+  const float r = b - __uint_as_float(h);  // exact
   const uint32_t m = __float_as_uint(r) & 0xFFFF0000u;
-  const float l = r - __uint_as_float(m);                   // exact, 8 bits
-  // an Inf or a NaN stays not finite in hi, which is all that is used of it
+  const float l = r - __uint_as_float(m);  // exact, 8 bits
   hi = h >> 16;
   mid = m >> 16;
   lo = __float_as_uint(l) >> 16;
@@ -241,10 +227,12 @@ __device__ __forceinline__ void split3(float b, uint32_t& hi, uint32_t& mid, uin
 
 // The planes of B over 32 K rows (step s) x 64 columns (group cg): wave q takes
 // K rows 8q .. 8q+7, a lane one column (each load instruction 256 contiguous
-// bytes).  Rows past K and columns past N are zero.
+// bytes).  Rows past K and columns past N are zero.  mark: a byte per wave, whether
+// any of its values is out of the planes' range.
 __device__ __forceinline__ void planes_block(const float* __restrict__ B, int64_t ldb, int64_t K,
                                              int64_t N, int64_t nks, int64_t ncb, int64_t s,
-                                             int64_t cg, uint8_t* __restrict__ planes) {
+                                             int64_t cg, uint8_t* __restrict__ planes,
+                                             uint8_t* __restrict__ mark) {
   const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
   const int64_t col = cg * 64 + lane, k0 = s * 32 + 8 * q;
   const int64_t cblk = col >> 4;
@@ -253,11 +241,20 @@ __device__ __forceinline__ void planes_block(const float* __restrict__ B, int64_
 #pragma unroll
   for (int e = 0; e < 8; ++e) v[e] = p[(k0 + e < K ? k0 + e : K - 1) * ldb];
   uint32_t o[kPlanes][4];
+  bool out = false;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    if (k0 + e >= K || col >= N) v[e] = 0.0f;
+    const uint32_t mag = __float_as_uint(v[e]) & 0x7FFFFFFFu;
+    out |= mag != 0u && mag - kTinyBits >= kHugeBits - kTinyBits;  // wraps below the range
+  }
+  const uint64_t outs = __ballot(out);
+  if (lane == 0) mark[q] = outs != 0ull ? 1 : 0;
 #pragma unroll
   for (int e = 0; e < 8; e += 2) {
     uint32_t h0, m0, l0, h1, m1, l1;
-    split3(k0 + e < K && col < N ? v[e] : 0.0f, h0, m0, l0);
-    split3(k0 + e + 1 < K && col < N ? v[e + 1] : 0.0f, h1, m1, l1);
+    split3(v[e], h0, m0, l0);
+    split3(v[e + 1], h1, m1, l1);
     o[0][e / 2] = h0 | (h1 << 16);
     o[1][e / 2] = m0 | (m1 << 16);
     o[2][e / 2] = l0 | (l1 << 16);
@@ -300,7 +297,7 @@ __global__ void __launch_bounds__(256)
 k_f32_prep(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
            const float* __restrict__ B, int64_t ldb, int64_t N, int64_t mask_wgs,
            int64_t mask_cols, uint32_t* __restrict__ S, uint8_t* __restrict__ planes,
-           uint32_t* __restrict__ dense) {
+           uint32_t* __restrict__ marks, uint32_t* __restrict__ dense) {
   const int64_t g = blockIdx.x;
   if (g < mask_wgs) {
     mask_stream_block<2>(W, M, K, ldw, ceil_div(K, 64), g % mask_cols, g / mask_cols, S);
@@ -311,18 +308,24 @@ k_f32_prep(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
   if (!d) return;
   const int64_t nks = ceil_div(K, 32), ncb = ceil_div(N, 16), units = nks * ceil_div(N, 64);
   for (int64_t u = g - mask_wgs; u < units; u += gridDim.x - mask_wgs)
-    planes_block(B, ldb, K, N, nks, ncb, u % nks, u / nks, planes);
+    planes_block(B, ldb, K, N, nks, ncb, u % nks, u / nks, planes,
+                 reinterpret_cast<uint8_t*>(marks + u));
 }
 
+// A byte per wave of planes_block, a word per unit: units of one column group together.
+size_t marks_bytes(int64_t K, int64_t N) {
+  return (size_t)ceil_div(K, 32) * ceil_div(N, 64) * sizeof(uint32_t);
+}
 size_t planes_bytes(int64_t K, int64_t N) {
   return (size_t)ceil_div(K, 32) * ceil_div(N, 16) * kPlanes * 1024;
 }
 
 }  // namespace
 
-// [decision, 256 bytes][mask stream][planes]
+// [decision, 256 bytes][mask stream][marks][planes]
 size_t f32_routed_bytes(int64_t M, int64_t K, int64_t N) {
-  return 256 + align_up(mask_stream_bytes(M, K), 256) + planes_bytes(K, N);
+  return 256 + align_up(mask_stream_bytes(M, K), 256) + align_up(marks_bytes(K, N), 256) +
+         planes_bytes(K, N);
 }
 
 bws_status launch_spmm_f32_routed(const bws_bitmap* A, void* ws, const float* B, int64_t ldb,
@@ -332,6 +335,7 @@ bws_status launch_spmm_f32_routed(const bws_bitmap* A, void* ws, const float* B,
   Carve cv(ws);
   uint32_t* dense = cv.take<uint32_t>(1);
   uint32_t* S = cv.take<uint32_t>(mask_stream_bytes(M, K) / 4);
+  uint32_t* marks = cv.take<uint32_t>(marks_bytes(K, N) / 4);
   uint8_t* planes = cv.take<uint8_t>(planes_bytes(K, N));
   const int64_t mask_cols = ceil_div(ceil_div(K, 64), kMaskStages);
   const int64_t row_blocks = ceil_div(M, kQRows), col_blocks = ceil_div(N, kQBN);
@@ -341,10 +345,10 @@ bws_status launch_spmm_f32_routed(const bws_bitmap* A, void* ws, const float* B,
   const int64_t per_xcd = ceil_div(row_blocks * col_blocks, 8);
   if (mask_wgs + split_wgs > kMaxGrid || 8 * per_xcd > kMaxGrid) return BWS_ECAPACITY;
   hipLaunchKernelGGL(k_f32_prep, dim3((unsigned)(mask_wgs + split_wgs)), dim3(256), 0, s, A->words,
-                     M, K, A->ldw, B, ldb, N, mask_wgs, mask_cols, S, planes, dense);
+                     M, K, A->ldw, B, ldb, N, mask_wgs, mask_cols, S, planes, marks, dense);
   BWS_TRY(launch_check());
   hipLaunchKernelGGL(k_spmm_f32, dim3((unsigned)(8 * per_xcd)), dim3(kQW * 64), 0, s, dense, S,
-                     planes, A->words, M, K, A->ldw, B, ldb, N, C, ldc, alpha, beta, row_blocks,
+                     planes, marks, A->words, M, K, A->ldw, B, ldb, N, C, ldc, alpha, beta, row_blocks,
                      col_blocks, per_xcd);
   return launch_check();
 }

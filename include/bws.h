@@ -415,7 +415,9 @@ size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision
  * that masks with more than one bit in eight run on the matrix cores (at 4096³ a
  * third to a quarter of the vector kernel's time at 50% density).  The density
  * is estimated from a fixed sample of A's words on the device: the same A always
- * takes the same kernel. */
+ * takes the same kernel.  256-column blocks of B that hold an infinity, a NaN, a
+ * value of 2^96 and more or a nonzero one below 2^-100 stay with the vector
+ * kernel (their time is the vector kernel's). */
 size_t bws_spmm_best_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision,
                                     const bws_plan* plan);
 bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb,
