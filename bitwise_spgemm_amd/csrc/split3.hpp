@@ -17,9 +17,9 @@
 // smaller b bits may be lost, and an Inf or NaN would spread to the rows that
 // do not select it (0 x Inf).  The product over planes leaves columns that hold
 // such values to the vector adds (spmm_planes.hip); the one-launch product, which
-// meets them on the way, sums an output that is not finite or is below 2^-80 (for
-// zero: only where some b was tiny) again from A's bits and B in FP32, bit by bit,
-// as the vector-add kernels do.
+// meets them on the way, sums an output that is not finite, or is below 2^-80 where
+// some b was tiny, again from A's bits and B in FP32 in ascending k, as the
+// vector-add kernels do.
 #pragma once
 
 #include "mfma_common.hpp"
@@ -32,21 +32,6 @@ constexpr uint32_t kTinyBits = (127u - 100u) << 23;  // 2^-100
 constexpr uint32_t kHugeBits = (127u + 96u) << 23;   // 2^96
 constexpr float kSmallOut = 0x1p-80f;
 
-// FP32 sum of column `col` of B over the set bits of one row of A, ascending k.
-__device__ __forceinline__ float row_sum(const uint32_t* __restrict__ w, int64_t K,
-                                         const float* __restrict__ bcol, int64_t ldb) {
-  float s = 0.0f;
-  for (int64_t i = 0; i * 32 < K; ++i) {
-    uint32_t m = w[i] & valid_bits(i, K);
-    while (m) {
-      const int c = __clz((int)m);
-      m &= ~wbit(c);
-      s += bcol[(32 * i + c) * ldb];
-    }
-  }
-  return s;
-}
-
 // 0/1 A fragment from a bitmap word (MSB first): K slot 8q + e of the 32-wide
 // step is bit 7 - e of x, the word's byte q from the top.  For z = x | (x << 17),
 // (z & (0x10001 << (7 - 2p))) * (ONE >> (7 - 2p)) puts ONE (BF16 1.0) into the low
@@ -58,12 +43,6 @@ __device__ __forceinline__ uint4 a_frag01(uint32_t w, int q) {
                     (uint32_t)__umul24(z & 0x00200020u, 0x3F80u >> 5),
                     (uint32_t)__umul24(z & 0x00080008u, 0x3F80u >> 3),
                     (uint32_t)__umul24(z & 0x00020002u, 0x3F80u >> 1));
-}
-
-// x is not to be trusted: not finite, or nonzero and below kSmallOut.
-__device__ __forceinline__ bool out_of_range(float x) {
-  const float m = fabsf(x);
-  return !(m < __builtin_inff()) || (m < kSmallOut && m != 0.0f);
 }
 
 }  // namespace

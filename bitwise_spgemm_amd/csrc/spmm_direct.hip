@@ -36,6 +36,7 @@ constexpr int kDM = 128, kDN = 32;            // tile rows and columns
 constexpr int kDA = kDM / 16, kDB = kDN / 16;  // MFMA tiles down and across
 typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 
 // hi, mid and lo of column c of eight K rows, and the smallest 2|b| - 1 seen
 // (unsigned, so that zero is the largest).
@@ -58,6 +59,100 @@ __device__ __forceinline__ void split8(const f32x2_u (&v)[8], int c, uint4& hi, 
   lo = make_uint4(up(l[0], l[1]), up(l[2], l[3]), up(l[4], l[5]), up(l[6], l[7]));
 }
 
+// x is not to be trusted: not finite, or below kSmallOut where some b was tiny.
+__device__ __forceinline__ bool not_exact(float x, bool any_tiny) {
+  const float m = fabsf(x);
+  return !(m < __builtin_inff()) || (any_tiny && m < kSmallOut);
+}
+
+// The tile's outputs once more as FP32 sums over the set bits, ascending k, as the
+// vector-add kernels form them: sums[x][i] of row 16a + j, a the wave's x-th row
+// tile, column n0 + 8q + i.  112 DW rows of B at a time go through lds (room for
+// 16 KiB DW), a lane walks its row's bits, four in flight.  us with ordinary values
+// in B | an infinity in every column | the vector-add kernels: 1024³, 10%
+// 12 | 41 | 41, 50% 12 | 78 | 94; 2048 x 1024 x 2048, 5% 30 | 104 | 36, 50%
+// 31 | 262 | 96 (two waves for four row tiles each); 3001 x 2053 x 516, 5%
+// 29 | 96 | 63.  Output by output and bit by bit from global memory the second
+// column was 305, 885, 780 and, in the last row, 735.
+template <int DW>
+__device__ __forceinline__ void vector_sums(const uint32_t* __restrict__ W, int64_t M, int64_t K,
+                                            int64_t ldw, const float* __restrict__ B, int64_t ldb,
+                                            int64_t N, int64_t m0, int64_t n0, float* lds,
+                                            float (&sums)[kDA / DW][8]) {
+  constexpr int kRW = 7 * DW / 2;  // bitmap words of a row at once
+  constexpr int kPitch = kDN + 4;  // floats: B rows start in different banks
+  static_assert(kRW * 32 * kPitch * 4 <= DW * 16384 && kRW * 32 * (kDN / 4) == 14 * DW * 64, "");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int j = lane & 15, q = lane >> 4;
+  const int64_t nks = ceil_div(K, 32);
+#pragma unroll
+  for (int x = 0; x < kDA / DW; ++x)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sums[x][i] = 0.0f;
+  for (int64_t w0 = 0; w0 < nks; w0 += kRW) {
+    __syncthreads();  // what was there has been read
+    for (int u0 = 0; u0 < 14; u0 += 7) {  // a thread's pieces, seven loads in flight
+      f32x4 v[7];
+#pragma unroll
+      for (int u = 0; u < 7; ++u) {
+        const int i = (u0 + u) * (DW * 64) + threadIdx.x;
+        const int64_t k = 32 * w0 + i / (kDN / 4), c = n0 + i % (kDN / 4) * 4;
+        const float* p = B + (k < K ? k : K - 1) * ldb;
+        if (c + 4 <= N) {
+          v[u] = *reinterpret_cast<const f32x4_u*>(p + c);
+        } else {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) v[u][t] = p[c + t < N ? c + t : N - 1];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 7; ++u) {
+        const int i = (u0 + u) * (DW * 64) + threadIdx.x;
+        *reinterpret_cast<f32x4*>(lds + i / (kDN / 4) * kPitch + i % (kDN / 4) * 4) = v[u];
+      }
+    }
+    __syncthreads();
+    const int nw = (int)(nks - w0 < kRW ? nks - w0 : kRW);
+#pragma unroll
+    for (int x = 0; x < kDA / DW; ++x) {
+      const int64_t row = m0 + 16 * (wave * (kDA / DW) + x) + j;
+      const uint32_t* wp = W + (row < M ? row : M - 1) * ldw + w0;
+      for (int i0 = 0; i0 < nw; i0 += 8) {
+        uint32_t wd[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+          wd[t] = i0 + t < nw ? wp[i0 + t] & valid_bits(w0 + i0 + t, K) : 0u;
+#pragma unroll
+        for (int t = 0; t < 8; t += 2) {
+          uint64_t m = ((uint64_t)wd[t] << 32) | wd[t + 1];
+          const float* b = lds + 32 * (i0 + t) * kPitch + 8 * q;
+          while (m) {
+            f32x4 v[4][2];
+            bool on[4];
+            int k = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {  // past the last bit: its row again, not added
+              on[e] = m != 0ull;
+              if (on[e]) {
+                k = __clzll((long long)m);
+                m &= ~(1ull << (63 - k));
+              }
+              v[e][0] = *reinterpret_cast<const f32x4*>(b + k * kPitch);
+              v[e][1] = *reinterpret_cast<const f32x4*>(b + k * kPitch + 4);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (on[e]) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) sums[x][i] += v[e][i >> 2][i & 3];
+              }
+          }
+        }
+      }
+    }
+  }
+}
+
 template <int DW>
 __global__ void __launch_bounds__(DW * 64, 2)
 k_spmm_direct(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
@@ -67,7 +162,7 @@ k_spmm_direct(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
   constexpr int kDW = 32 * DW;  // bitmap words of a row in LDS at once,
   __shared__ f32x4 part[DW][kDA * kDB][64];  // in the room of the partial tiles
   static_assert(kDW * kDM * 4 == sizeof(part), "");
-  __shared__ uint32_t tiny[DW];
+  __shared__ uint32_t tiny[DW], redo[DW];
   uint32_t(*const words)[kDM] = reinterpret_cast<uint32_t(*)[kDM]>(&part[0][0][0]);
   const int64_t tile = xcd_tile(blockIdx.x, per_xcd);
   if (tile >= row_blocks * col_blocks) return;
@@ -215,12 +310,15 @@ k_spmm_direct(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
   for (int w = 0; w < DW; ++w) any_tiny |= tiny[w];
 
   // row tile a, accumulator e of tile b of lane (j, q): row 16a + j, column
-  // 8q + 2e + b
+  // 8q + 2e + b.  Outputs that are not to be trusted wait (a bit each in bad).
+  constexpr int NX = kDA / DW;
+  uint32_t bad[NX], any_bad = 0u;
 #pragma unroll
-  for (int x = 0; x < kDA / DW; ++x) {
-    const int a = wave * (kDA / DW) + x;
+  for (int x = 0; x < NX; ++x) {
+    const int a = wave * NX + x;
     const int64_t row = m0 + 16 * a + j;
     f32x4 sum[kDB];
+    bad[x] = 0u;
 #pragma unroll
     for (int b = 0; b < kDB; ++b) {
       const int i = a * kDB + b;
@@ -234,13 +332,14 @@ k_spmm_direct(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
       const int64_t col = n0 + 8 * q + 4 * h;
       if (col >= N) continue;
       f32x4 v = {sum[0][2 * h], sum[1][2 * h], sum[0][2 * h + 1], sum[1][2 * h + 1]};
+      uint32_t wait = 0u;
 #pragma unroll
       for (int b = 0; b < 4; ++b)
-        if ((out_of_range(v[b]) || (any_tiny && v[b] == 0.0f)) && col + b < N)
-          v[b] = row_sum(W + row * ldw, K, B + col + b, ldb);
+        if (not_exact(v[b], any_tiny != 0u) && col + b < N) wait |= 1u << b;
+      bad[x] |= wait << (4 * h);
       v *= alpha;
       float* c = C + row * ldc + col;
-      if (vec && col + 3 < N) {
+      if (vec && col + 3 < N && wait == 0u) {
         if (beta != 0.0f) {
           const f32x4 o = *reinterpret_cast<const f32x4*>(c);
 #pragma unroll
@@ -250,9 +349,30 @@ k_spmm_direct(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
       } else {
 #pragma unroll
         for (int b = 0; b < 4; ++b)
-          if (col + b < N) c[b] = beta != 0.0f ? fmaf(beta, c[b], v[b]) : v[b];
+          if (col + b < N && !((wait >> b) & 1u))
+            c[b] = beta != 0.0f ? fmaf(beta, c[b], v[b]) : v[b];
       }
     }
+    any_bad |= bad[x];
+  }
+  const uint64_t waiting = __ballot(any_bad != 0u);
+  if (lane == 0) redo[wave] = waiting != 0ull ? 1u : 0u;
+  __syncthreads();
+  any_bad = 0u;
+#pragma unroll
+  for (int w = 0; w < DW; ++w) any_bad |= redo[w];
+  if (any_bad == 0u) return;  // the same for the whole workgroup
+  float again[NX][8];
+  vector_sums<DW>(W, M, K, ldw, B, ldb, N, m0, n0, reinterpret_cast<float*>(&part[0][0][0]), again);
+#pragma unroll
+  for (int x = 0; x < NX; ++x) {
+    float* c = C + (m0 + 16 * (wave * NX + x) + j) * ldc + n0 + 8 * q;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if ((bad[x] >> i) & 1u) {
+        const float v = alpha * again[x][i];
+        c[i] = beta != 0.0f ? fmaf(beta, c[i], v) : v;
+      }
   }
 }
 

@@ -61,3 +61,52 @@ def test_routed_scaled(bws, dev, scale):
     assert bool(wide.any())
     for i in torch.nonzero(wide).view(-1).tolist():
         assert _same(C[:, 256 * i:256 * i + 256], S[:, 256 * i:256 * i + 256])
+
+
+# 8, 4 and 2 waves of the one-launch product; N past and off a lane's 8 columns
+@pytest.mark.parametrize("M,K,N", [(300, 9000, 100), (3300, 4200, 301), (2048, 200, 1999)])
+def test_direct_outputs(bws, dev, M, K, N):
+    """Outputs over such values: the vector-add kernel's bits.  The others: the
+    product's without them."""
+    A = bws.Bitmap(to_dev(bws.gen_bitmap_iid(M, M, K, 0.1), dev), M, K)
+    g = torch.Generator(device=dev).manual_seed(N)
+    B = torch.randn((K, N), device=dev, generator=g)
+    plain = bws.spmm(A, B)
+    B[3, 1], B[K - 1, 2], B[5, N - 1], B[:, 8:16] = INF, NAN, -INF, 3e38
+    B[:, 40:49] *= 1e-35
+    B[:, 64] = 0.0
+    B[0, 64] = 1e-42
+    C0 = torch.randn((M, N), device=dev, generator=g)
+    C = bws.spmm(A, B, alpha=-0.5, beta=0.25, out=C0.clone())
+    V = bws.spmm(A, B, alpha=-0.5, beta=0.25, out=C0.clone(), plan=bws.make_plan(1))
+    held = torch.zeros(N, dtype=torch.bool, device=dev)
+    held[[1, 2, N - 1, 64]] = held[8:16] = held[40:49] = True
+    assert _same(C[:, held], V[:, held])
+    # (beta's term: one fused multiply-add)
+    E = (0.25 * C0.double() - 0.5 * plain.double()).float()
+    assert torch.equal(C[:, ~held], E[:, ~held])
+
+
+def _us(f):
+    best = 1e9
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(4):
+            f()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
+@pytest.mark.parametrize("M,K,N,p", [(1024, 1024, 1024, 0.1), (4096, 512, 3072, 0.3)])
+def test_time_does_not_run_away(bws, dev, M, K, N, p):
+    """An infinity in every column: within 10 times of ordinary values (4 and 2
+    times measured; output by output it was 30 and more)."""
+    A = bws.Bitmap(to_dev(bws.gen_bitmap_iid(1, M, K, p), dev), M, K)
+    B = torch.randn((K, N), device=dev)
+    C = torch.empty((M, N), device=dev)
+    t0 = _us(lambda: bws.spmm(A, B, out=C))
+    B[K // 2] = INF
+    assert _us(lambda: bws.spmm(A, B, out=C)) <= 10 * t0
