@@ -127,18 +127,22 @@ size_t esize(int32_t d) { return d == BWS_DTYPE_F32 ? 4 : 2; }
 // steps, so that short products and many of them go to the vector-add kernels,
 // whose time falls with K and with the mask's density.  us, one launch against
 // vector-add at 1% | 5% density:
-//   tiles  256, K   64:  6.0 |  4.5,  4.8     K  128:  6.2 |  5.9,  6.7
+//   tiles  256, K   64:  6.0 |  4.5,  4.8     K  128:  6.9 |  6.5,  7.4
+//                                             K  160:  7.1 |  7.3,  8.1
 //   tiles  512, K  128:  7.5 |  6.5,  7.3     K  256:  9.1 |  9.4, 10.9
 //   tiles 1024, K  512: 18.6 | 18.3, 20.0     K 1024: 28.0 | 32.3, 34.0
 //                                             K 2048: 48.0 | 57.8, 61.9
 //   tiles 1536, K 1024: 43.4 | 28.7, 39.8
 // Rows that are not 16-byte pieces leave only the row kernel on the other side:
+//   tiles  256, K  128:  9.5 | 16.2 (1%), 21.5 (10%)
+//   tiles  512, K  128: 11.2 |  9.6 (1%), 15.3 (10%); K 192: 12.0 | 12.4
 //   tiles 1056, K   64: 23.6 | 20.1, 19.3     K  256: 28.2 | 44.6 (2%)
+//   tiles 2209, K  128: 43.8 | 42.3 (1%), 49.2 (10%); K 192: 47.4 | 52.9
 //   tiles 4096, K 4095:  364 |  480,  723 (432 at 0.1%)
 //   tiles 16384, K 256:  312 |  198,  260
 int64_t direct_max_tiles(int64_t K, bool aligned) {
-  if (K < 128) return 0;
-  if (!aligned) return K < 1024 ? 2304 : (int64_t)1 << 28;
+  if (K < (aligned ? 160 : 128)) return 0;
+  if (!aligned) return K < 192 ? 256 : K < 1024 ? 2304 : (int64_t)1 << 28;
   return K < 256 ? 256 : K < 1024 ? 512 : 1024;
 }
 

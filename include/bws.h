@@ -370,8 +370,8 @@ typedef struct {
 /* C = alpha * (A · B) + beta * C, A M x K bitmap, B K x N dense (dtype b_dtype,
  * leading dimension ldb), C M x N FP32.  beta == 0 never reads C.
  * FP32 with a 0/1 A, an F32 B and no plan: outputs of up to 256, 512 and 1024 tiles
- * of 64 x 64 with K of at least 128, 256 and 1024 (larger ones too where rows of B
- * or C are off 16 bytes) run on the matrix cores without a workspace, each b split
+ * of 64 x 64 with K of at least 160, 256 and 1024 (larger ones and K from 128 too
+ * where rows of B or C are off 16 bytes) run on the matrix cores without a workspace, each b split
  * exactly into three BF16 parts and every product and sum in FP32.
  * Outputs that meet an infinity or a NaN, overflow, or are below 2^-80 beside
  * b below 2^-100, are summed by vector adds in ascending k instead: the tiles of

@@ -1,0 +1,28 @@
+"""Short products of 0/1 masks at FP32 that the vector-add kernels finish first:
+they take those, so they give those kernels' bits (sums in ascending k; the
+matrix cores sum in another order and differ in some)."""
+import pytest
+import torch
+
+from _helpers import to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(bws, dev, M, K, N, p):
+    A = bws.Bitmap(to_dev(bws.gen_bitmap_iid(M + N, M, K, p), dev), M, K)
+    return A, torch.randn((K, N), device=dev, generator=torch.Generator(device=dev).manual_seed(K))
+
+
+# 16-byte rows below K = 160; others below 192 where there are more than 256 tiles
+@pytest.mark.parametrize("M,K,N", [(256, 128, 256), (1024, 159, 1024), (500, 130, 64), (16384, 128, 65),
+                                   (2000, 191, 2001), (32768, 128, 33)])
+def test_one_launch_short_k(bws, dev, M, K, N):
+    A, B = _operands(bws, dev, M, K, N, 0.3)
+    assert torch.equal(bws.spmm(A, B), bws.spmm(A, B, plan=bws.make_plan(1)))
+
+
+@pytest.mark.parametrize("M,K,N", [(256, 160, 256), (1000, 128, 1001), (2000, 192, 2001)])
+def test_one_launch_from_there(bws, dev, M, K, N):
+    A, B = _operands(bws, dev, M, K, N, 0.3)
+    assert not torch.equal(bws.spmm(A, B), bws.spmm(A, B, plan=bws.make_plan(1)))
