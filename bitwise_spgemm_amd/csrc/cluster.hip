@@ -828,12 +828,15 @@ bws_status bws_spmm_clustered(const bws_bitmap* A, const int32_t* slot_row,
   if (N % 4 != 0 || ldb % 4 != 0 || ldc % 4 != 0 || reinterpret_cast<uintptr_t>(B) % 16 != 0 ||
       reinterpret_cast<uintptr_t>(C) % 16 != 0 || reinterpret_cast<uintptr_t>(plan_stream) % 256)
     return BWS_EUNSUPPORTED;
-  // Outputs of up to 1024 tiles of 64 x 64: the streamed kernel has few 256 x 256
-  // workgroups and walks K at one workgroup's pace, the one-launch product on the
-  // matrix cores does not need the plan.  us, streamed at 1% to 50% density
-  // against that: 1024³ 41 to 236 | 10, 2048³ 79 to 412 | 48, 4096² x 1024 129 to
-  // 306 | 85; at 2048 tiles, 4096 x 1024 x 2048, 40 to 83 | 60 (by the tiles).
-  if (spmm_direct_ok(A, ldb, N, 1024))
+  // Outputs of up to 1024 tiles of 64 x 64, up to 512 where K is short: the streamed
+  // kernel has few 256 x 256 workgroups and walks K at one workgroup's pace, the
+  // one-launch product on the matrix cores does not need the plan.  us, streamed at
+  // 1% to 50% density against that: 1024³ 41 to 236 | 10, 2048³ 79 to 412 | 48, 4096²
+  // x 1024 129 to 306 | 85; at 2048 tiles, 4096 x 1024 x 2048, 40 to 83 | 60 (by the
+  // tiles).  Short K, 1%: 512 tiles, K 32 7.6 | 7.1, K 64 8.0 | 7.5; 768, K 64
+  // 9.5 | 9.9, K 128 11.3 | 11.4, K 192 13.3 | 12.8; 1024, K 64 9.5 to 9.8 | 10.8,
+  // K 128 11.7 to 12.1 | 12.3, K 192 13.9 to 14.3 | 13.6.
+  if (spmm_direct_ok(A, ldb, N, A->cols < 192 ? 512 : 1024))
     return launch_spmm_direct(A, B, ldb, N, C, ldc, alpha, beta, s);
   return launch_spmm_stream(static_cast<const uint32_t*>(plan_stream), slot_row, A->rows, A->cols,
                             B, ldb, N, C, ldc, alpha, beta, s);

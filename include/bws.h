@@ -477,10 +477,9 @@ bws_status bws_cluster_stream(const bws_bitmap* A, const int32_t* slot_row,
  * the end; other rows sum their own bits.  FP32 vector adds; the summation
  * order differs from bws_spmm's, and the result stays within FP32 rounding of
  * A·B relative to |A|·|B| (the subtracted terms are bits of the base).  Outputs
- * of up to 1024 tiles of 64 x 64 run as bws_spmm's small ones do, on the matrix
- * cores from A itself.  Needs
- * N, ldb and ldc multiples of 4 and 16-byte aligned B and C
- * (BWS_EUNSUPPORTED otherwise). */
+ * of up to 1024 tiles of 64 x 64 (512 where K is below 192) run as bws_spmm's
+ * small ones do, on the matrix cores from A itself.  Needs N, ldb and ldc
+ * multiples of 4 and 16-byte aligned B and C (BWS_EUNSUPPORTED otherwise). */
 bws_status bws_spmm_clustered(const bws_bitmap* A, const int32_t* slot_row,
                               const void* plan_stream, const float* B, int64_t ldb, int64_t N,
                               float* C, int64_t ldc, float alpha, float beta, bws_stream stream);

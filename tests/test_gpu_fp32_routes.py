@@ -26,3 +26,18 @@ def test_one_launch_short_k(bws, dev, M, K, N):
 def test_one_launch_from_there(bws, dev, M, K, N):
     A, B = _operands(bws, dev, M, K, N, 0.3)
     assert not torch.equal(bws.spmm(A, B), bws.spmm(A, B, plan=bws.make_plan(1)))
+
+
+@pytest.mark.parametrize("M,K,N,streamed", [(2048, 64, 2048, True), (4096, 191, 1024, True),
+                                            (1500, 16, 2048, True), (2048, 192, 2048, False),
+                                            (1024, 64, 2048, False)])
+def test_clustered_short_k(bws, dev, M, K, N, streamed):
+    """Above 512 tiles the streamed kernel runs below K = 192: it takes the masks
+    from the plan (an empty mask's plan gives zeros), the one-launch product from A."""
+    A, B = _operands(bws, dev, M, K, N, 0.3)
+    empty = bws.cluster_rows(bws.Bitmap(torch.zeros_like(A.words), M, K))
+    C = bws.spmm_clustered(A, empty, B)
+    assert bool((C == 0).all()) == streamed
+    ref = bws.unpack_bitmap(A).double() @ B.double()
+    bound = 1e-5 * (bws.unpack_bitmap(A).double() @ B.double().abs())
+    assert bool(((bws.spmm_clustered(A, bws.cluster_rows(A), B).double() - ref).abs() <= bound).all())
