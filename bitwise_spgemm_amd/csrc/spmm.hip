@@ -155,6 +155,14 @@ bool stream_ok(const bws_bitmap* A, const void* B, int64_t ldb, int64_t N, const
   return ceil_div(A->rows, kStreamTileRows) * ceil_div(N, kStreamTileCols) >= kStreamMinTiles;
 }
 
+// From which K the product is routed by the mask's density: the estimate and the
+// decision cost a sparse mask up to 1 us, the planes a dense one 10 us before they
+// save anything.  us, streamed | routed at 1% to 5% and at 50%: 4096 x 4096, K 32
+// 18.2 to 18.8 | 19.3 to 19.7, 26.6 | 29.6; K 64 18.2 to 19.5 | 19.5 to 20.5,
+// 33.9 | 30.4; K 96 20.1 to 22.0 | 20.3 to 22.9, 45 | 31; K 128 19.7 to 23.1 |
+// 20.2 to 23.3, 52 | 31; K 256 23.2 to 29.7 | 23.1 to 29.4, 91 | 42.
+constexpr int64_t kRoutedMinK = 96;
+
 }  // namespace
 
 bws_status spmm_dispatch(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb,
@@ -228,7 +236,8 @@ size_t bws_spmm_best_workspace_size(const bws_bitmap* A, int64_t N, int32_t prec
     return bws_spmm_workspace_size(A, N, precision, plan);
   if (N % 4 == 0 &&
       ceil_div(A->rows, kStreamTileRows) * ceil_div(N, kStreamTileCols) >= kStreamMinTiles)
-    return f32_routed_bytes(A->rows, A->cols, N);
+    return A->cols < kRoutedMinK ? mask_stream_bytes(A->rows, A->cols)
+                                 : f32_routed_bytes(A->rows, A->cols, N);
   return 0;  // neither the one-launch product nor the vector-add tiles use one
 }
 
@@ -272,7 +281,7 @@ bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t
                               stream);
   // and outputs that fill the chip with 256 x 256 tiles by the mask's density,
   // with room for B's planes in the workspace
-  if (f32_auto && stream_ok(A, B, ldb, N, C, ldc) &&
+  if (f32_auto && A->cols >= kRoutedMinK && stream_ok(A, B, ldb, N, C, ldc) &&
       ws_ok(workspace, workspace_bytes, f32_routed_bytes(A->rows, A->cols, N)))
     return launch_spmm_f32_routed(A, workspace, static_cast<const float*>(B), ldb, N, C, ldc,
                                   alpha, beta, stream);

@@ -414,7 +414,7 @@ size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision
  * rows of a multiple of 8 columns (also used for a 16-bit B whose rows are off 16
  * bytes; the same bits as without it at BF16 / FP16, at BF16X2 as with the split
  * of N % 8 == 0); at FP32, for outputs of at least 192 tiles of 256 x 256 (N % 4 ==
- * 0): room for B split exactly into three BF16 parts (6 bytes per element), so
+ * 0) and K of at least 96: room for B split exactly into three BF16 parts (6 bytes per element), so
  * that masks with more than one bit in eight run on the matrix cores (at 4096³ a
  * third to a quarter of the vector kernel's time at 50% density).  The density
  * is estimated from a fixed sample of A's words on the device: the same A always

@@ -41,3 +41,16 @@ def test_clustered_short_k(bws, dev, M, K, N, streamed):
     ref = bws.unpack_bitmap(A).double() @ B.double()
     bound = 1e-5 * (bws.unpack_bitmap(A).double() @ B.double().abs())
     assert bool(((bws.spmm_clustered(A, bws.cluster_rows(A), B).double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("M,K,N,streamed", [(4096, 32, 4096, True), (3072, 95, 4096, True),
+                                            (3072, 96, 4096, False)])
+def test_routed_short_k(bws, dev, M, K, N, streamed):
+    """A dense mask of a large output: below K = 96 the streamed kernel's bits (its
+    sums are the vector-add kernel's), and a workspace for the mask stream alone."""
+    A, B = _operands(bws, dev, M, K, N, 0.5)
+    assert torch.equal(bws.spmm(A, B), bws.spmm(A, B, plan=bws.make_plan(1))) == streamed
+    L, s = bws.lib(), A.struct()
+    sizes = [f(bws.C.byref(s), N, 0, None) for f in (L.bws_spmm_workspace_size,
+                                                     L.bws_spmm_best_workspace_size)]
+    assert (sizes[0] == sizes[1]) == streamed
