@@ -682,6 +682,29 @@ def _rows16(B: torch.Tensor) -> bool:
             and B.data_ptr() % 16 == 0)
 
 
+def _product_workspace(s: _Bitmap, B: torch.Tensor, precision: str, plan,
+                       min_bits: int = 0) -> Optional[torch.Tensor]:
+    """The workspace with which bws_spmm has every kernel to choose from, or where
+    there is no memory for it (FP32: B's planes, 1.5 times B; 16 bits: B once
+    more), what the kernels without it take."""
+    N, prec = B.shape[1], PRECISION[precision]
+    pl = None if plan is None else C.byref(plan)
+    b16 = (precision in ("bf16", "fp16") and not s.values and B.dtype != torch.float32
+           and min_bits == 0)
+    if b16 and _rows16(B):
+        return None  # it would hold a rounded or padded B: not needed for this one
+    best = lib().bws_spmm_best_workspace_size(C.byref(s), N, prec, pl)
+    if not best:
+        return None
+    try:
+        return _workspace(best, B.device)
+    except torch.OutOfMemoryError:
+        least = 0 if b16 else lib().bws_spmm_workspace_size(C.byref(s), N, prec, pl)
+        if least >= best:
+            raise
+    return _workspace(least, B.device) if least else None
+
+
 def spmm(A: Bitmap, B: torch.Tensor, precision: str = "fp32", alpha: float = 1.0,
          beta: float = 0.0, out: Optional[torch.Tensor] = None, plan=None) -> torch.Tensor:
     """C = alpha * A·B + beta * C (C FP32, M x N)."""
@@ -695,11 +718,7 @@ def spmm(A: Bitmap, B: torch.Tensor, precision: str = "fp32", alpha: float = 1.0
             raise ValueError("beta != 0 needs `out`")
     s = A.struct()
     pl = None if plan is None else C.byref(plan)
-    wsz = lib().bws_spmm_best_workspace_size(C.byref(s), N, PRECISION[precision], pl)
-    if (precision in ("bf16", "fp16") and A.values is None and _rows16(B)
-            and (plan is None or plan.mfma_min_bits == 0)):
-        wsz = 0  # the workspace would hold a rounded or padded B: not needed for this one
-    ws = _workspace(wsz, dev) if wsz else None
+    ws = _product_workspace(s, B, precision, plan, 0 if plan is None else plan.mfma_min_bits)
     _check(lib().bws_spmm(C.byref(s), _ptr(B), DTYPE[B.dtype], B.stride(0), N, _ptr(out),
                           out.stride(0), alpha, beta, PRECISION[precision], pl, _ptr(ws),
                           0 if ws is None else ws.numel(), _stream(dev)),
@@ -737,10 +756,7 @@ def spmm_tA(AT: Bitmap, dC: torch.Tensor, precision: str = "fp32", alpha: float 
         out = torch.empty((AT.rows, N), dtype=torch.float32, device=dev)
     s = AT.struct()
     pl = None if plan is None else C.byref(plan)
-    wsz = lib().bws_spmm_best_workspace_size(C.byref(s), N, PRECISION[precision], pl)
-    if precision in ("bf16", "fp16") and AT.values is None and _rows16(dC):
-        wsz = 0  # the workspace would hold a rounded or padded dC: not needed for this one
-    ws = _workspace(wsz, dev) if wsz else None
+    ws = _product_workspace(s, dC, precision, plan)
     _check(lib().bws_spmm_tA(C.byref(s), _ptr(dC), DTYPE[dC.dtype], dC.stride(0), N, _ptr(out),
                              out.stride(0), alpha, beta, PRECISION[precision], pl, _ptr(ws),
                              0 if ws is None else ws.numel(), _stream(dev)),
