@@ -229,9 +229,11 @@ size_t bws_spmm_best_workspace_size(const bws_bitmap* A, int64_t N, int32_t prec
                                     const bws_plan* plan) {
   if (!A || A->rows <= 0 || A->cols <= 0 || N <= 0 || A->values)
     return bws_spmm_workspace_size(A, N, precision, plan);
-  if (precision != BWS_PREC_FP32)
+  if (precision != BWS_PREC_FP32) {
+    if (!plan && spmm_direct16_ok(A, precision, N, N)) return 0;
     return plan || N % 8 == 0 ? bws_spmm_workspace_size(A, N, precision, plan)
                               : spmm_pad_workspace(A->cols, N, precision);
+  }
   if (plan && (plan->kernel != 0 || plan->rows_per_wg != 0))
     return bws_spmm_workspace_size(A, N, precision, plan);
   if (N % 4 == 0 &&

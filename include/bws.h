@@ -408,15 +408,17 @@ typedef struct {
  * 2062-2248) with the operand roles of a bitmap A and a dense B. */
 size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision,
                                const bws_plan* plan);
-/* The workspace with which bws_spmm has every kernel to choose from: at least
- * bws_spmm_workspace_size, 0 where none helps.  More than that on a 0/1 A without
- * a plan: for BF16 / FP16 / BF16X2 with N % 8 != 0, room for B in 16 bits with
+/* The workspace with which bws_spmm has every kernel to choose from.  With a plan
+ * that names a kernel, or a value-carrying A, bws_spmm_workspace_size.  On a 0/1 A
+ * without one it is 0 for the outputs that run without a workspace (the small ones
+ * above; at FP32 all below 192 tiles of 256 x 256) and otherwise at least that,
+ * and more: for BF16 / FP16 / BF16X2 with N % 8 != 0, room for B in 16 bits with
  * rows of a multiple of 8 columns (also used for a 16-bit B whose rows are off 16
  * bytes; the same bits as without it at BF16 / FP16, at BF16X2 as with the split
  * of N % 8 == 0); at FP32, for outputs of at least 192 tiles of 256 x 256 (N % 4 ==
- * 0) and K of at least 96: room for B split exactly into three BF16 parts (6 bytes per element), so
- * that masks with more than one bit in eight run on the matrix cores (at 4096³ a
- * third to a quarter of the vector kernel's time at 50% density).  The density
+ * 0) and K of at least 96: room for B split exactly into three BF16 parts (6 bytes
+ * per element), so that masks with more than one bit in eight run on the matrix
+ * cores (at 4096³ a third of the vector kernel's time at 50% density).  The density
  * is estimated from a fixed sample of A's words on the device: the same A always
  * takes the same kernel.  256-column blocks of B that hold an infinity, a NaN, a
  * value of 2^96 and more or a nonzero one below 2^-100 stay with the vector

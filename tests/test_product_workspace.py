@@ -48,3 +48,29 @@ def test_no_memory_at_all(bws, monkeypatch):
     with pytest.raises(torch.OutOfMemoryError):
         bws._product_workspace(_struct(bws, 4096, 4096), torch.empty((4096, 4096), device="meta"),
                                "fp32", None)
+
+
+def test_best_size(bws):
+    """Without a plan: 0 for every output that runs without a workspace, else at
+    least what bws_spmm_workspace_size reports; with a plan or values, just that."""
+    L = bws.lib()
+    for M in (64, 500, 2048, 4096):
+        for K in (64, 1280, 2048):
+            for N in (8, 300, 304, 1024, 4096):
+                tiles = -(-M // 64) * -(-N // 64)
+                for precision in ("fp32", "bf16", "fp16", "bf16x2"):
+                    s, prec = _struct(bws, M, K), bws.PRECISION[precision]
+                    args = (bws.C.byref(s), N, prec)
+                    best, least = L.bws_spmm_best_workspace_size(*args, None), \
+                        L.bws_spmm_workspace_size(*args, None)
+                    if precision == "fp32":
+                        none = -(-M // 256) * -(-N // 256) < 192
+                    else:
+                        none = tiles <= (512 if precision == "bf16x2" else 0 if K < 1280
+                                         else 256 if K < 2048 else 512)
+                    assert best == 0 if none else best >= least, (M, K, N, precision, best, least)
+                    plan = bws.make_plan(1, 256, 16, 64)
+                    v = _struct(bws, M, K, values=True)
+                    for x, p in ((s, bws.C.byref(plan)), (v, None)):
+                        assert L.bws_spmm_best_workspace_size(bws.C.byref(x), N, prec, p) == \
+                            L.bws_spmm_workspace_size(bws.C.byref(x), N, prec, p)
