@@ -146,6 +146,11 @@ int64_t direct_max_tiles(int64_t K, bool aligned) {
   return K < 256 ? 256 : K < 1024 ? 512 : 1024;
 }
 
+// The plan, or NULL where it names nothing: the built-in choice.
+const bws_plan* named(const bws_plan* p) {
+  return p && (p->kernel != 0 || p->rows_per_wg != 0 || p->mfma_min_bits != 0) ? p : nullptr;
+}
+
 // The streamed FP32 kernel: 16-byte rows of B and C, and enough 256 x 256
 // tiles to occupy the chip (one workgroup per CU).
 bool stream_ok(const bws_bitmap* A, const void* B, int64_t ldb, int64_t N, const float* C,
@@ -201,7 +206,7 @@ extern "C" {
 
 size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision,
                                const bws_plan* plan) {
-  (void)N;
+  plan = named(plan);
   if (!A || A->rows < 0 || A->cols < 0 || N < 0) return 0;
   if (precision == BWS_PREC_FP32 && !A->values && N % 4 == 0 && plan && plan->kernel == 1 &&
       plan->rows_per_wg == 0 && plan->k_stage == kSubsetKStage)
@@ -227,6 +232,7 @@ size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision
 
 size_t bws_spmm_best_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision,
                                     const bws_plan* plan) {
+  plan = named(plan);
   if (!A || A->rows <= 0 || A->cols <= 0 || N <= 0 || A->values)
     return bws_spmm_workspace_size(A, N, precision, plan);
   if (precision != BWS_PREC_FP32) {
@@ -234,7 +240,7 @@ size_t bws_spmm_best_workspace_size(const bws_bitmap* A, int64_t N, int32_t prec
     return plan || N % 8 == 0 ? bws_spmm_workspace_size(A, N, precision, plan)
                               : spmm_pad_workspace(A->cols, N, precision);
   }
-  if (plan && (plan->kernel != 0 || plan->rows_per_wg != 0))
+  if (plan && (plan->kernel != 0 || plan->rows_per_wg != 0))  // (min_bits alone: 16 bits only)
     return bws_spmm_workspace_size(A, N, precision, plan);
   if (N % 4 == 0 &&
       ceil_div(A->rows, kStreamTileRows) * ceil_div(N, kStreamTileCols) >= kStreamMinTiles)
@@ -258,6 +264,7 @@ bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t
                 !valu_cfg_valid(plan_valu_cfg(plan, A->rows, N, A->values != nullptr))) ||
                (plan->kernel == 2 && !mfma_tile_valid(plan->rows_per_wg, plan->cols_per_wg))))
     return BWS_EINVAL;
+  plan = named(plan);
   if (A->rows == 0 || N == 0) return BWS_OK;
   if (!C || ldc < N) return BWS_EINVAL;
   if (A->cols > 0 && (!B || ldb < N)) return BWS_EINVAL;
