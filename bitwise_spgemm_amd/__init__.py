@@ -74,7 +74,7 @@ class _Groups(C.Structure):
 class _Plan(C.Structure):
     _fields_ = [("kernel", C.c_int32), ("rows_per_wg", C.c_int32), ("waves_per_wg", C.c_int32),
                 ("k_stage", C.c_int32), ("mfma_min_bits", C.c_int32), ("cols_per_wg", C.c_int32),
-                ("mfma_staging", C.c_int32), ("reserved", C.c_int32)]
+                ("mfma_staging", C.c_int32), ("flags", C.c_int32)]
 
 
 class _Problem(C.Structure):

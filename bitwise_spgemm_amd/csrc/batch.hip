@@ -26,6 +26,8 @@ bool valu_direct_ok(int32_t b_dtype, const void* B, int64_t ldb, int64_t N, cons
                     int64_t ldc);
 ValuCfg plan_valu_cfg(const bws_plan* plan, int64_t M, int64_t N, bool vals);
 bool spmm_vals_ok(int64_t K);
+bool spmm_stream_ok(const bws_bitmap* A, const void* B, int64_t ldb, int64_t N, const float* C,
+                    int64_t ldc);
 
 namespace {
 
@@ -99,6 +101,10 @@ Choice classify(const bws_problem& p, int32_t b_dtype, int32_t precision, const 
   } else if (p.nnz_hint > 0) {
     cache_get(make_key(p.A.rows, p.A.cols, p.N, p.nnz_hint, precision), &eff);
   }
+  // a tuned tile that lost to the built-in choice: in 16 bits that is the batch's
+  // own (below); an FP32 launch has no other kernels than these tiles
+  if (!explicit_plan && (eff.flags & BWS_PLAN_GROUPED) && precision != BWS_PREC_FP32)
+    eff = bws_plan{};
   int kernel = eff.kernel;
   if (precision == BWS_PREC_FP32) kernel = 1;
   else if (kernel == 0) kernel = p.A.values ? 1 : 2;
@@ -131,6 +137,10 @@ Choice classify(const bws_problem& p, int32_t b_dtype, int32_t precision, const 
     c.kind = 1;
     c.vals = p.A.values != nullptr;
     c.cfg = plan_valu_cfg(eff.rows_per_wg ? &eff : nullptr, p.A.rows, p.N, c.vals);
+    if (c.vals) {  // the value product has its rows alone to choose: one launch for all with equal ones
+      c.cfg.waves = 16;
+      c.cfg.kstage = c.cfg.rows == 64 ? 32 : 64;
+    }
     return c;
   }
   c.kind = 3;
@@ -348,6 +358,8 @@ bws_status bws_autotune(const bws_bitmap* A, int64_t nnz, const void* B, int32_t
                                     {128, 16, 32}, {128, 8, 32}, {128, 8, 64},  {64, 16, 32},
                                     {64, 8, 32}};
   for (const auto& c : cfgs) {
+    // the value product has its rows alone to choose
+    if (A->values && (c[1] != 16 || c[2] != (c[0] == 64 ? 32 : 64))) continue;
     bws_plan p{};
     p.kernel = 1;
     p.rows_per_wg = c[0];
@@ -369,26 +381,44 @@ bws_status bws_autotune(const bws_bitmap* A, int64_t nnz, const void* B, int32_t
   hipEvent_t e0, e1;
   BWS_TRY(hip_check(hipEventCreate(&e0)));
   BWS_TRY(hip_check(hipEventCreate(&e1)));
-  float best_t = -1.0f;
+  // BWS_EINVAL and BWS_EUNSUPPORTED: not applicable here
+  auto timed = [&](const bws_plan* p, float& ms) -> bws_status {
+    auto run = [&] {
+      return bws_spmm(A, B, b_dtype, ldb, N, C, ldc, 1.0f, 0.0f, precision, p, nullptr, 0, stream);
+    };
+    BWS_TRY(run());
+    BWS_TRY(hip_check(hipEventRecord(e0, stream)));
+    for (int r = 0; r < repeats; ++r) BWS_TRY(run());
+    BWS_TRY(hip_check(hipEventRecord(e1, stream)));
+    BWS_TRY(hip_check(hipEventSynchronize(e1)));
+    BWS_TRY(hip_check(hipEventElapsedTime(&ms, e0, e1)));
+    ms /= (float)repeats;
+    return BWS_OK;
+  };
+  float best_t = -1.0f, plain_t = -1.0f;
   bws_plan best_p{};
   bws_status st = BWS_OK;
   for (const bws_plan& p : cand) {
-    st = bws_spmm(A, B, b_dtype, ldb, N, C, ldc, 1.0f, 0.0f, precision, &p, nullptr, 0, stream);
-    if (st == BWS_EINVAL || st == BWS_EUNSUPPORTED) continue;  // not applicable here
-    if (st != BWS_OK) break;
-    hipEventRecord(e0, stream);
-    for (int r = 0; r < repeats && st == BWS_OK; ++r)
-      st = bws_spmm(A, B, b_dtype, ldb, N, C, ldc, 1.0f, 0.0f, precision, &p, nullptr, 0, stream);
-    hipEventRecord(e1, stream);
-    if (st != BWS_OK) break;
-    if ((st = hip_check(hipEventSynchronize(e1))) != BWS_OK) break;
     float ms = 0;
-    hipEventElapsedTime(&ms, e0, e1);
-    ms /= (float)repeats;
+    st = timed(&p, ms);
+    if (st == BWS_EINVAL || st == BWS_EUNSUPPORTED) continue;
+    if (st != BWS_OK) break;
     if (best_t < 0 || ms < best_t) {
       best_t = ms;
       best_p = p;
     }
+  }
+  // The built-in choice.  It is timed without a workspace, as the tiles are, so
+  // the streamed and routed FP32 products are not: from K = 512 they are the faster
+  // ones (us, with the workspace | best tile, 1%, 5% and 30%: 4096³ 106 | 149, 217
+  // | 237, 357 | 750; 4096 x 512 x 3072 25.6 | 27.6, 39.5 | 39.6, 58 | 101;
+  // 3072 x 256 x 4096, 1% 20.9 | 20.2).
+  if (best_t >= 0 && (st == BWS_OK || st == BWS_EINVAL || st == BWS_EUNSUPPORTED)) {
+    st = timed(nullptr, plain_t);
+    const bool streamed = precision == BWS_PREC_FP32 && !A->values && b_dtype == BWS_DTYPE_F32 &&
+                          A->cols >= 512 && spmm_stream_ok(A, B, ldb, N, C, ldc);
+    if (st == BWS_OK && (plain_t <= 1.02f * best_t || streamed)) best_p.flags = BWS_PLAN_GROUPED;
+    if (st == BWS_OK && plain_t < best_t) best_t = plain_t;
   }
   hipEventDestroy(e0);
   hipEventDestroy(e1);
@@ -417,13 +447,13 @@ bws_status bws_autotune_save(const char* path) {
   FILE* f = fopen(path, "w");
   if (!f) return BWS_EINVAL;
   std::lock_guard<std::mutex> lk(g_mu);
-  fprintf(f, "# bws autotune cache: precision log2M log2K log2N density_class kernel rows waves kstage cols\n");
+  fprintf(f, "# bws autotune cache: precision log2M log2K log2N density_class kernel rows waves kstage cols flags\n");
   for (const auto& kv : cache()) {
     const Key& k = kv.first;
     const bws_plan& p = kv.second;
-    fprintf(f, "%d %d %d %d %d %d %d %d %d %d\n", std::get<0>(k), std::get<1>(k), std::get<2>(k),
+    fprintf(f, "%d %d %d %d %d %d %d %d %d %d %d\n", std::get<0>(k), std::get<1>(k), std::get<2>(k),
             std::get<3>(k), std::get<4>(k), p.kernel, p.rows_per_wg, p.waves_per_wg, p.k_stage,
-            p.cols_per_wg);
+            p.cols_per_wg, p.flags);
   }
   fclose(f);
   return BWS_OK;
@@ -437,10 +467,10 @@ bws_status bws_autotune_load(const char* path) {
   bws_status st = BWS_OK;
   while (fgets(line, sizeof line, f)) {
     if (line[0] == '#') continue;
-    int v[10] = {0};
-    const int n = sscanf(line, "%d %d %d %d %d %d %d %d %d %d", &v[0], &v[1], &v[2], &v[3], &v[4],
-                         &v[5], &v[6], &v[7], &v[8], &v[9]);
-    if (n != 9 && n != 10) {
+    int v[11] = {0};
+    const int n = sscanf(line, "%d %d %d %d %d %d %d %d %d %d %d", &v[0], &v[1], &v[2], &v[3], &v[4],
+                         &v[5], &v[6], &v[7], &v[8], &v[9], &v[10]);
+    if (n < 9 || n > 11) {  // earlier files end at kstage or cols
       st = BWS_EINVAL;
       continue;
     }
@@ -450,6 +480,7 @@ bws_status bws_autotune_load(const char* path) {
     p.waves_per_wg = v[7];
     p.k_stage = v[8];
     p.cols_per_wg = v[9];
+    p.flags = v[10];
     cache_put(Key(v[0], v[1], v[2], v[3], v[4]), p);
   }
   fclose(f);

@@ -146,9 +146,11 @@ int64_t direct_max_tiles(int64_t K, bool aligned) {
   return K < 256 ? 256 : K < 1024 ? 512 : 1024;
 }
 
-// The plan, or NULL where it names nothing: the built-in choice.
+// The plan, or NULL where it names nothing or is for grouped launches: the
+// built-in choice.
 const bws_plan* named(const bws_plan* p) {
-  return p && (p->kernel != 0 || p->rows_per_wg != 0 || p->mfma_min_bits != 0) ? p : nullptr;
+  if (!p || (p->flags & BWS_PLAN_GROUPED)) return nullptr;
+  return p->kernel != 0 || p->rows_per_wg != 0 || p->mfma_min_bits != 0 ? p : nullptr;
 }
 
 // The streamed FP32 kernel: 16-byte rows of B and C, and enough 256 x 256
@@ -169,6 +171,11 @@ bool stream_ok(const bws_bitmap* A, const void* B, int64_t ldb, int64_t N, const
 constexpr int64_t kRoutedMinK = 96;
 
 }  // namespace
+
+bool spmm_stream_ok(const bws_bitmap* A, const void* B, int64_t ldb, int64_t N, const float* C,
+                    int64_t ldc) {
+  return stream_ok(A, B, ldb, N, C, ldc);
+}
 
 bws_status spmm_dispatch(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb,
                          int64_t N, float* C, int64_t ldc, float alpha, float beta,

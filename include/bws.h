@@ -347,7 +347,10 @@ bws_status bws_cluster_rows(const bws_bitmap* A, int32_t max_clusters, int32_t* 
  *                 sparse MFMA), half the MFMA instructions of the dense
  *                 kernel, results equal to it up to FP32 summation order;
  *                 other operands run as AUTO
- *   reserved      pass 0 */
+ *   flags         0, or BWS_PLAN_GROUPED, which bws_autotune sets: the plan is
+ *                 for grouped launches; bws_spmm and its workspace queries take
+ *                 it for no plan (the built-in choice was the faster one) */
+enum { BWS_PLAN_GROUPED = 1 };
 enum {
   BWS_MFMA_AUTO = 0,
   BWS_MFMA_LUT = 1,   /* 64 x 64 per wave, A fragments from an LDS table      */
@@ -364,7 +367,7 @@ typedef struct {
   int32_t mfma_min_bits;
   int32_t cols_per_wg;
   int32_t mfma_staging;
-  int32_t reserved;
+  int32_t flags;
 } bws_plan;
 
 /* C = alpha * (A · B) + beta * C, A M x K bitmap, B K x N dense (dtype b_dtype,
@@ -573,14 +576,19 @@ bws_status bws_spmm_batched(const bws_problem* problems, int32_t count, int32_t 
                             int32_t precision, const bws_plan* plan, void* workspace,
                             size_t workspace_bytes, bws_stream stream);
 
-/* Autotuner: times the candidate tile configurations of bws_spmm for this
- * problem on `stream` (HIP events; the call synchronises and overwrites C)
- * and returns the fastest in *best, also recording it in the process-wide
- * cache under the problem's shape class (M, K, N rounded up to powers of two,
- * log2 of the density rounded to an integer, precision).  bws_batch_prepare
- * consults the cache for problems with a nonzero nnz_hint when it is given no
- * plan; bws_spmm never does (its NULL plan means the built-in defaults).  nnz
- * is the bitmap's set-bit count (the caller knows it).
+/* Autotuner: times the candidate tile configurations of bws_spmm and its
+ * built-in choice for this problem on `stream` (HIP events; the call synchronises
+ * and overwrites C) and returns the fastest tile in *best, with BWS_PLAN_GROUPED
+ * where the built-in choice was at least as fast (2%), or is a kernel that needs
+ * a workspace and is known to be (FP32, a 0/1 A, at least 192 tiles of 256 x 256,
+ * K of at least 512); *best_ms is the shorter of the two times.  The plan is also
+ * recorded in the process-wide cache under the problem's shape class (M, K, N
+ * rounded up to powers of two, log2 of the density rounded to an integer,
+ * precision).  bws_batch_prepare consults the cache for problems with a nonzero
+ * nnz_hint when it is given no plan (at FP32 it takes the tile; in 16 bits a plan
+ * with BWS_PLAN_GROUPED leaves the choice to it); bws_spmm never does (its NULL
+ * plan means the built-in defaults).  nnz is the bitmap's set-bit count (the
+ * caller knows it).
  * bws_autotune_save / _load write and read the cache as a text file. */
 bws_status bws_autotune(const bws_bitmap* A, int64_t nnz, const void* B, int32_t b_dtype,
                         int64_t ldb, int64_t N, float* C, int64_t ldc, int32_t precision,
