@@ -201,12 +201,15 @@ def _check(status: int, where: str):
         raise BwsError(status, where)
 
 
+# the handle alone: a stream object per call is a microsecond of a call that takes
+# seven on the GPU (not a public call of torch: without it, the public one)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 def _stream(device=None) -> int:
-    # the handle alone: a stream object per call is a microsecond of a call that
-    # takes seven on the GPU
     index = None if device is None else torch.device(device).index
-    return torch._C._cuda_getCurrentRawStream(
-        torch.cuda.current_device() if index is None else index)
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def _ptr(t: Optional[torch.Tensor]):
