@@ -1,0 +1,61 @@
+"""Split BF16 above 512 tiles of 64 x 64, where a workspace decides the kernel:
+two passes over B's planes, or one that splits in registers.  (Smaller outputs
+run in one launch either way.)"""
+import pytest
+import torch
+
+from _helpers import to_dev
+
+pytestmark = pytest.mark.gpu
+
+# ragged M, K and N; N off 8: the planes' rows are padded
+SHAPES = [(2100, 97, 1352), (2100, 97, 1355), (1990, 300, 1100), (4200, 33, 643), (2049, 130, 1021)]
+
+
+def _product(bws, A, B, C, alpha, beta, ws):
+    s = A.struct()
+    assert bws.lib().bws_spmm(bws.C.byref(s), B.data_ptr(), 0, B.stride(0), B.shape[1], C.data_ptr(),
+                              C.stride(0), alpha, beta, bws.PRECISION["bf16x2"], None,
+                              None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+                              torch.cuda.current_stream().cuda_stream) == 0
+    return C
+
+
+def _room(bws, A, N, dev):
+    s = A.struct()
+    n = bws.lib().bws_spmm_best_workspace_size(bws.C.byref(s), N, bws.PRECISION["bf16x2"], None)
+    assert n > 0
+    return torch.empty(n, dtype=torch.uint8, device=dev)
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("alpha,beta,pad", [(1.0, 0.0, 0), (0.5, -2.0, 3)])
+def test_two_forms(bws, dev, M, K, N, alpha, beta, pad):
+    A = bws.Bitmap(to_dev(bws.gen_bitmap_iid(M, M, K, 0.4), dev), M, K)
+    g = torch.Generator(device=dev).manual_seed(N)
+    B = torch.randn((K, N + pad), device=dev, generator=g)[:, pad:]
+    C0 = torch.randn((M, N + 2 * pad), device=dev, generator=g)
+    D = bws.unpack_bitmap(A).double()
+    c0 = C0[:, pad:pad + N].double()
+    R = alpha * (D @ B.double()) + beta * c0
+    S = abs(alpha) * (D @ B.double().abs()) + 2 * abs(beta) * c0.abs()
+    out = []
+    for ws in (_room(bws, A, N, dev), None):
+        C = C0.clone()
+        out.append(_product(bws, A, B, C[:, pad:pad + N], alpha, beta, ws))
+        assert bool(((out[-1].double() - R).abs() <= 1e-5 * S).all())
+        assert torch.equal(C[:, :pad], C0[:, :pad]) and torch.equal(C[:, pad + N:], C0[:, pad + N:])
+    assert not torch.equal(out[0], out[1])  # two kernels
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_two_passes_round_once(bws, dev, M, K, N):
+    """b = i + j/256, whole i in [129, 254], |j| <= 127: hi = i and lo = j/256, whose
+    sums are exact; they meet in the second pass, in one rounding."""
+    A = bws.Bitmap(to_dev(bws.gen_bitmap_iid(M + 1, M, K, 0.6), dev), M, K)
+    g = torch.Generator(device=dev).manual_seed(K)
+    B = (torch.randint(129, 255, (K, N), device=dev, generator=g).double()
+         + torch.randint(-127, 128, (K, N), device=dev, generator=g).double() / 256)
+    R = bws.unpack_bitmap(A).double() @ B
+    C = torch.empty((M, N), device=dev)
+    assert torch.equal(_product(bws, A, B.float(), C, 1.0, 0.0, _room(bws, A, N, dev)), R.float())
