@@ -97,7 +97,7 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
   __shared__ int32_t s_base[kGroupPF + 1];     // spilled rows before a chunk
   __shared__ int32_t s_nnz[NW];
   const int lane = lane_id();
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // XCD-contiguous tile ranges: the tiles of neighbouring words of the same
   // rows share an XCD, so the 128-byte lines of group_id they fill together
   // are merged in one L2 before they are written
@@ -179,13 +179,17 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
       cnt += __popcll(spillers);
     };
     const uint32_t vb = valid_bits(w, cols);
+    // a single wave meets its own lanes' LDS words alone and needs no barrier
+    auto sync = [] {
+      if constexpr (NW > 1) __syncthreads();
+    };
     for (int b0 = 0; b0 < nrows; b0 += 64 * kGroupPF) {
       const int nch = min(kGroupPF, (nrows - b0 + 63) / 64);
       // a wave's chunks are wave, wave + NW, ..: their words are all loaded before
       // the first is placed, four chunks at a time under a wave-uniform test,
       // unconditional within it (rows past the tile read its last row and are
       // zeroed)
-      if (b0) __syncthreads();  // the words before have been read
+      if (b0) sync();  // the words before have been read
       constexpr int kPer = kGroupPF / NW;
       uint32_t mm[kPer];
 #pragma unroll
@@ -208,19 +212,20 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
           }
         }
       }
-      __syncthreads();
+      sync();
       if (wave == 0) {
         uint32_t next = s_word[lane];
 #pragma unroll 1
         for (int u = 0; u < nch; ++u) {
-          const uint32_t m = next;
-          next = s_word[(u + 1 < nch ? u + 1 : u) * 64 + lane];
+          // (a chunk ahead, except with many groups: 3% slower there)
+          const uint32_t m = GC > 0 ? next : s_word[u * 64 + lane];
+          if (GC > 0) next = s_word[(u + 1 < nch ? u + 1 : u) * 64 + lane];
           chunk(b0 + 64 * u, m, u);
         }
-        if (lane == 0) s_base[kGroupPF] = cnt;
+        if (NW > 1 && lane == 0) s_base[kGroupPF] = cnt;
       }
-      __syncthreads();
-#pragma unroll 2
+      sync();
+#pragma unroll(NW > 1 ? 2 : 1)
       for (int u = wave; u < nch; u += NW) {
         const int j = b0 + 64 * u + lane;
         const uint32_t m = s_word[u * 64 + lane];
@@ -243,10 +248,12 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
         }
       }
     }
-    cnt = s_base[kGroupPF];
-    const int32_t snnz_wave = wave_sum(snnz_lane);
-    if (lane == 0) s_nnz[wave] = snnz_wave;
-    __syncthreads();
+    int32_t snnz = wave_sum(snnz_lane);  // of this wave's chunks
+    if constexpr (NW > 1) {
+      cnt = __builtin_amdgcn_readfirstlane(s_base[kGroupPF]);
+      if (lane == 0) s_nnz[wave] = snnz;
+      __syncthreads();
+    }
     if (spill_rev)
       for (int j = nrows + threadIdx.x; j < T; j += 64 * NW) spill_rev[t * T + j] = -1;
     if (spill_table)
@@ -274,9 +281,11 @@ k_group_rows(const uint32_t* __restrict__ W, int64_t rows, int64_t cols, int64_t
     }
     const uint32_t gm_lane = gms.lane_value(lane);
     if (lane < G) group_mask[t * G + lane] = gm_lane;
-    int32_t snnz = 0;
+    if constexpr (NW > 1) {
+      snnz = 0;
 #pragma unroll
-    for (int x = 0; x < NW; ++x) snnz += s_nnz[x];
+      for (int x = 0; x < NW; ++x) snnz += s_nnz[x];
+    }
     const int32_t tile_nnz = wave_sum(lane < G ? __popc(gm_lane) : 0);
     if (lane == 0) {
       spill_cnt[t] = cnt;
