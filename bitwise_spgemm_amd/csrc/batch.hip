@@ -17,9 +17,9 @@ namespace bws {
 bws_status spmm_dispatch(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb,
                          int64_t N, float* C, int64_t ldc, float alpha, float beta,
                          int32_t precision, const bws_plan* plan, hipStream_t s);
-bws_status spmm_valu_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
+bws_status spmm_valu_batch(const BatchEntry* entries, const int64_t* off, int count,
                            int64_t total_tiles, const ValuCfg& cfg, bool vals, hipStream_t s);
-bws_status spmm_mfma_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
+bws_status spmm_mfma_batch(const BatchEntry* entries, const int64_t* off, int count,
                            int64_t total_tiles, const MfmaTile& t, int32_t b_dtype,
                            int32_t precision, int vec, hipStream_t s);
 bool valu_direct_ok(int32_t b_dtype, const void* B, int64_t ldb, int64_t N, const float* C,
@@ -213,12 +213,8 @@ bws_status bws_batch_prepare(const bws_problem* problems, int32_t count, int32_t
     choice[(size_t)i] = classify(problems[i], b_dtype, precision, plan, together);
     order.push_back(i);
   }
-  // within a launch the problems with the longest tiles (K) first, so that the
-  // last workgroups to start are short ones
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-    const Choice &x = choice[(size_t)a], &y = choice[(size_t)b];
-    return x < y || (!(y < x) && problems[a].A.cols > problems[b].A.cols);
-  });
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int a, int b) { return choice[(size_t)a] < choice[(size_t)b]; });
 
   std::vector<BatchEntry> entries;
   std::vector<int64_t> offs;
@@ -243,7 +239,17 @@ bws_status bws_batch_prepare(const bws_problem* problems, int32_t count, int32_t
     } else {
       L.first = (int32_t)entries.size();
       L.count = (int32_t)(end - pos);
-      int64_t tiles = 0, slots = 0;
+      const int64_t bm = c.kind == 2 ? c.tile.bm : c.cfg.rows;
+      const int64_t bn = c.kind == 2 ? c.tile.bn : 256;
+      int64_t tiles = 0, before = 0;
+      for (size_t x = pos; x < end; ++x)
+        tiles += ceil_div(problems[order[x]].A.rows, bm) * ceil_div(problems[order[x]].N, bn);
+      const bool shares = batch_range(tiles, L.count) == 0;
+      // with shares the problems with the longest tiles (K) first, so that the last
+      // workgroups to start are short ones
+      if (shares)
+        std::stable_sort(order.begin() + (ptrdiff_t)pos, order.begin() + (ptrdiff_t)end,
+                         [&](int a, int b) { return problems[a].A.cols > problems[b].A.cols; });
       for (size_t x = pos; x < end; ++x) {
         const bws_problem& p = problems[order[x]];
         BatchEntry e{};
@@ -258,16 +264,13 @@ bws_status bws_batch_prepare(const bws_problem* problems, int32_t count, int32_t
         e.ldb = p.ldb;
         e.N = p.N;
         e.ldc = p.ldc;
-        const int64_t bm = c.kind == 2 ? c.tile.bm : c.cfg.rows;
-        const int64_t bn = c.kind == 2 ? c.tile.bn : 256;
         e.row_blocks = ceil_div(e.M, bm);
         e.col_blocks = ceil_div(e.N, bn);
-        offs.push_back(slots);
-        tiles += e.row_blocks * e.col_blocks;
-        slots += ceil_div(e.row_blocks * e.col_blocks, 8);
+        offs.push_back(before);
+        before += shares ? ceil_div(e.row_blocks * e.col_blocks, 8) : e.row_blocks * e.col_blocks;
         entries.push_back(e);
       }
-      offs.push_back(slots);
+      offs.push_back(before);
       L.total_tiles = tiles;
     }
     pos = end;

@@ -220,33 +220,53 @@ __device__ __forceinline__ T wave_incl_scan(T v) {
   return v;
 }
 
-// Grouped launches: workgroup b runs on XCD b % 8 and takes slot b / 8 of that
-// XCD.  Every problem gives each XCD an eighth of its tiles (a contiguous range
-// of the column-block-major order, so an XCD's L2 holds few panels of B);
-// slot_off[i] is the first slot of problem i, slot_off[i + 1] - slot_off[i] the
+// Grouped launches: workgroup b runs on XCD b % 8.
+//
+// Shares (range == 0): the workgroup takes
+// slot b / 8 of its XCD.  Every problem gives each XCD an eighth of its tiles (a
+// contiguous range of the column-block-major order, so an XCD's L2 holds few
+// panels of B); off[i] is the first slot of problem i, off[i + 1] - off[i] the
 // largest of its eight shares.  A range of equal tile counts over the whole
 // table, as the single-problem kernels use, gave XCDs up to 1.4 times the mean
 // work where the problems' K differ (32 problems, K 256 to 8192).
+//
+// Ranges, for launches of at most a workgroup per CU, where no tile waits for a
+// place, and of at most eight tiles a problem: every XCD takes range consecutive
+// tiles of the launch, off[i] the tiles of the problems before i, so that a
+// problem's tiles share its B in one or two L2s.  us, shares | ranges, FP16 from an
+// FP32 B: 37 problems of 16 to 3000 rows and columns, N = 64 (230 tiles) 93 | 72,
+// N = 100 114 | 93, 8 of 256 to 4096, N = 64 (70) 127 | 96; BF16, 64 of 64 to 512,
+// N = 1000 (504) 31 | 26.  Beyond that shares win: 16 of 100 to 1000, N = 1000 (440)
+// 45 | 56, split BF16, 32 of 256 to 4096, N = 8 (430) 138 | 218.
 __device__ __forceinline__ bool batch_tile(const BatchEntry* __restrict__ entries,
-                                           const int64_t* __restrict__ slot_off, int count,
-                                           int& problem, int64_t& tile) {
+                                           const int64_t* __restrict__ off, int count,
+                                           int64_t range, int& problem, int64_t& tile) {
   const int64_t slot = blockIdx.x >> 3;
-  if (slot >= slot_off[count]) return false;
+  const int64_t at = range ? (blockIdx.x & 7) * range + slot : slot;
+  if (at >= off[count]) return false;
   int lo = 0, hi = count;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
-    if (slot_off[mid] <= slot) lo = mid;
+    if (off[mid] <= at) lo = mid;
     else hi = mid;
   }
   problem = lo;
+  if (range) {
+    tile = at - off[lo];
+    return true;
+  }
   const int64_t tiles = entries[lo].row_blocks * entries[lo].col_blocks;
   const int64_t x = (blockIdx.x + lo) & 7;  // the larger shares go round the XCDs
-  tile = tiles * x / 8 + slot - slot_off[lo];
+  tile = tiles * x / 8 + slot - off[lo];
   return tile < tiles * (x + 1) / 8;
 }
-// Workgroups of such a launch (every share rounded up to the largest).
-inline int64_t batch_grid(int64_t total_tiles, int count) {
-  return 8 * (total_tiles / 8 + count);
+// Tiles per XCD of a launch with ranges, 0 for one with shares.
+inline int64_t batch_range(int64_t total_tiles, int count) {
+  return total_tiles <= 256 || total_tiles <= 8 * (int64_t)count ? ceil_div(total_tiles, 8) : 0;
+}
+// Workgroups of the launch (every share rounded up to the largest).
+inline int64_t batch_grid(int64_t total_tiles, int count, int64_t range) {
+  return 8 * (range ? range : total_tiles / 8 + count);
 }
 
 __device__ __forceinline__ uint32_t lo32(uint64_t x) { return (uint32_t)x; }

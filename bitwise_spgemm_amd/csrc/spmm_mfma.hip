@@ -456,11 +456,11 @@ k_spmm_mfma4(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
 
 template <int PREC, int WM, int WN, int NBUF, int KS>
 __global__ void __launch_bounds__(256, 2)
-k_spmm_mfma4_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ slot_off,
-                   int count) {
+k_spmm_mfma4_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ off,
+                   int count, int64_t range) {
   int lo;
   int64_t tile;
-  if (!batch_tile(entries, slot_off, count, lo, tile)) return;
+  if (!batch_tile(entries, off, count, range, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   mfma4_tile<PREC, WM, WN, NBUF, KS>(e.W, e.M, e.K, e.ldw, static_cast<const uint16_t*>(e.B),
                                      e.ldb, e.N, e.C, e.ldc, 1.0f, 0.0f, tile,
@@ -481,11 +481,11 @@ k_spmm_mfma3(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
 
 template <int PREC, int TB, int WM, int WN>
 __global__ void __launch_bounds__(256, 2)
-k_spmm_mfma3_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ slot_off,
-                   int count, int vec) {
+k_spmm_mfma3_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ off,
+                   int count, int64_t range, int vec) {
   int lo;
   int64_t tile;
-  if (!batch_tile(entries, slot_off, count, lo, tile)) return;
+  if (!batch_tile(entries, off, count, range, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   mfma3_tile<PREC, TB, WM, WN>(e.W, e.M, e.K, e.ldw, e.B, e.ldb, e.N, e.C, e.ldc, 1.0f, 0.0f,
                                tile, e.row_blocks, vec);
@@ -600,56 +600,57 @@ bws_status launch_mfma_cfg(const MfmaTile& t, const bws_bitmap* A, const void* B
 }
 
 template <int PREC, int TB, int WM, int WN>
-void launch_mfma3_batch(dim3 grid, const BatchEntry* entries, const int64_t* slot_off, int count,
-                        int vec, hipStream_t s) {
+void launch_mfma3_batch(dim3 grid, const BatchEntry* entries, const int64_t* off, int count,
+                        int64_t range, int vec, hipStream_t s) {
   hipLaunchKernelGGL((k_spmm_mfma3_batch<PREC, TB, WM, WN>), grid, dim3(256), 0, s, entries,
-                     slot_off, count, vec);
+                     off, count, range, vec);
 }
 
 template <int PREC, int TB>
-bws_status launch_mfma_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
+bws_status launch_mfma_batch(const BatchEntry* entries, const int64_t* off, int count,
                              int64_t total_tiles, const MfmaTile& t, int vec, hipStream_t s) {
-  if (batch_grid(total_tiles, count) > kMaxGrid) return BWS_ECAPACITY;
+  const int64_t range = batch_range(total_tiles, count);
+  if (batch_grid(total_tiles, count, range) > kMaxGrid) return BWS_ECAPACITY;
   if (total_tiles == 0) return BWS_OK;
   if (!has_tile<PREC, TB>(t.bm, t.bn)) return BWS_EUNSUPPORTED;
-  const dim3 grid((unsigned)batch_grid(total_tiles, count));
+  const dim3 grid((unsigned)batch_grid(total_tiles, count, range));
   bool done = false;
   if constexpr (TB != 0 && PREC != 3) {
     if (t.dma) {
       if (t.bm == 32)
         hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 16, 32, 2, 128>), grid, dim3(256), 0, s,
-                           entries, slot_off, count);
+                           entries, off, count, range);
       else if (t.bm == 64 && t.bn == 64)
         hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 32, 32, 2, 128>), grid, dim3(256), 0, s,
-                           entries, slot_off, count);
+                           entries, off, count, range);
       else if (t.bm == 64)
         hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 32, 64, 2, 128>), grid, dim3(256), 0, s,
-                           entries, slot_off, count);
+                           entries, off, count, range);
       else if (t.bn == 256)
         hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 64, 128, 2, 64>), grid, dim3(256), 0, s,
-                           entries, slot_off, count);
+                           entries, off, count, range);
       else if (t.bm == 256)
         hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 128, 64, 2, 64>), grid, dim3(256), 0, s,
-                           entries, slot_off, count);
+                           entries, off, count, range);
       else
         hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 64, 64, 2, 64>), grid, dim3(256), 0, s,
-                           entries, slot_off, count);
+                           entries, off, count, range);
       return launch_check();
     }
   }
   if constexpr (has_tile<PREC, TB>(128, 256)) {
     if (t.bn == 256) {
-      launch_mfma3_batch<PREC, TB, 64, 128>(grid, entries, slot_off, count, vec, s);
+      launch_mfma3_batch<PREC, TB, 64, 128>(grid, entries, off, count, range, vec, s);
       done = true;
     }
   }
   if constexpr (has_tile<PREC, TB>(256, 128)) {
     if (!done && t.bm == 256) {
-      launch_mfma3_batch<PREC, TB, 128, 64>(grid, entries, slot_off, count, vec, s);
+      launch_mfma3_batch<PREC, TB, 128, 64>(grid, entries, off, count, range, vec, s);
       done = true;
     }
   }
-  if (!done) launch_mfma3_batch<PREC, TB, 64, 64>(grid, entries, slot_off, count, vec, s);
+  if (!done) launch_mfma3_batch<PREC, TB, 64, 64>(grid, entries, off, count, range, vec, s);
   return launch_check();
 }
 
@@ -735,10 +736,10 @@ bool mfma_tile_valid(int bm, int bn) {
   return (bm == 0 || bm == 128 || bm == 256) && (bn == 0 || bn == 128 || bn == 256);
 }
 
-bws_status spmm_mfma_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
+bws_status spmm_mfma_batch(const BatchEntry* entries, const int64_t* off, int count,
                            int64_t total_tiles, const MfmaTile& t, int32_t b_dtype,
                            int32_t precision, int vec, hipStream_t s) {
-#define BWS_MB(P, T) return launch_mfma_batch<P, T>(entries, slot_off, count, total_tiles, t, vec, s)
+#define BWS_MB(P, T) return launch_mfma_batch<P, T>(entries, off, count, total_tiles, t, vec, s)
   if (precision == BWS_PREC_BF16) {
     if (b_dtype == BWS_DTYPE_BF16) BWS_MB(1, 1);
     if (b_dtype == BWS_DTYPE_F32) BWS_MB(1, 0);

@@ -22,12 +22,12 @@ k_spmm_vals(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
 // Grouped launch: a workgroup finds its problem and tile with batch_tile.
 template <int VR>
 __global__ void __launch_bounds__(kVW * 64)
-k_spmm_vals_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ slot_off,
-                  int count) {
+k_spmm_vals_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ off,
+                  int count, int64_t range) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kValsLds];
   int lo;
   int64_t tile;
-  if (!batch_tile(entries, slot_off, count, lo, tile)) return;
+  if (!batch_tile(entries, off, count, range, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   vals_tile<VR>(e.W, e.M, e.K, e.ldw, e.row_ptr, e.values, static_cast<const float*>(e.B), e.ldb,
                 e.N, e.C, e.ldc, 1.0f, 0.0f, tile, e.row_blocks, smem);
@@ -77,16 +77,17 @@ bws_status spmm_vals_f32(const bws_bitmap* A, const float* B, int64_t ldb, int64
   }
 }
 
-bws_status spmm_vals_f32_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
+bws_status spmm_vals_f32_batch(const BatchEntry* entries, const int64_t* off, int count,
                                int64_t total_tiles, int32_t rows, hipStream_t s) {
-  const int64_t grid = batch_grid(total_tiles, count);
+  const int64_t range = batch_range(total_tiles, count);
+  const int64_t grid = batch_grid(total_tiles, count, range);
   if (grid > kMaxGrid) return BWS_ECAPACITY;
   if (total_tiles == 0) return BWS_OK;
   const dim3 g((unsigned)grid), b(kVW * 64);
   switch (rows) {
-    case 256: hipLaunchKernelGGL(k_spmm_vals_batch<16>, g, b, 0, s, entries, slot_off, count); break;
-    case 128: hipLaunchKernelGGL(k_spmm_vals_batch<8>, g, b, 0, s, entries, slot_off, count); break;
-    case 64: hipLaunchKernelGGL(k_spmm_vals_batch<4>, g, b, 0, s, entries, slot_off, count); break;
+    case 256: hipLaunchKernelGGL(k_spmm_vals_batch<16>, g, b, 0, s, entries, off, count, range); break;
+    case 128: hipLaunchKernelGGL(k_spmm_vals_batch<8>, g, b, 0, s, entries, off, count, range); break;
+    case 64: hipLaunchKernelGGL(k_spmm_vals_batch<4>, g, b, 0, s, entries, off, count, range); break;
     default: return BWS_EINVAL;
   }
   return launch_check();

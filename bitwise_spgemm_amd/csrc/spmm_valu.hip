@@ -19,7 +19,7 @@ namespace bws {
 bool spmm_vals_ok(int64_t K);
 bws_status spmm_vals_f32(const bws_bitmap* A, const float* B, int64_t ldb, int64_t N, float* C,
                          int64_t ldc, float alpha, float beta, int32_t rows, hipStream_t s);
-bws_status spmm_vals_f32_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
+bws_status spmm_vals_f32_batch(const BatchEntry* entries, const int64_t* off, int count,
                                int64_t total_tiles, int32_t rows, hipStream_t s);
 
 namespace {
@@ -520,11 +520,11 @@ k_spmm_rows2_groups(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_
 // Grouped launch: a workgroup finds its problem and tile with batch_tile.
 template <int WAVES, int RPW, int KS>
 __global__ void __launch_bounds__(WAVES * 64)
-k_spmm_rows2_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ slot_off,
-                   int count) {
+k_spmm_rows2_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ off,
+                   int count, int64_t range) {
   int lo;
   int64_t tile;
-  if (!batch_tile(entries, slot_off, count, lo, tile)) return;
+  if (!batch_tile(entries, off, count, range, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   rows2_tile<WAVES, RPW, KS>(e.W, e.M, e.K, e.ldw, e.row_ptr, e.values,
                                    static_cast<const float*>(e.B), e.ldb, e.N, e.C, e.ldc, 1.0f,
@@ -686,25 +686,26 @@ inline int grid_for(int64_t items, int64_t per_block) {
 }
 
 template <int WAVES, int RPW, int KS>
-bws_status launch_rows2_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
+bws_status launch_rows2_batch(const BatchEntry* entries, const int64_t* off, int count,
                               int64_t total_tiles, hipStream_t s) {
-  const int64_t grid = batch_grid(total_tiles, count);
+  const int64_t range = batch_range(total_tiles, count);
+  const int64_t grid = batch_grid(total_tiles, count, range);
   if (grid > kMaxGrid) return BWS_ECAPACITY;
   if (total_tiles == 0) return BWS_OK;
   hipLaunchKernelGGL((k_spmm_rows2_batch<WAVES, RPW, KS>), dim3((unsigned)grid),
-                     dim3(WAVES * 64), 0, s, entries, slot_off, count);
+                     dim3(WAVES * 64), 0, s, entries, off, count, range);
   return launch_check();
 }
 
 }  // namespace
 
 // Grouped vector-add launch (FP32 B meeting the direct-staging conditions).
-bws_status spmm_valu_batch(const BatchEntry* entries, const int64_t* slot_off, int count,
+bws_status spmm_valu_batch(const BatchEntry* entries, const int64_t* off, int count,
                            int64_t total_tiles, const ValuCfg& cfg, bool vals, hipStream_t s) {
-  if (vals) return spmm_vals_f32_batch(entries, slot_off, count, total_tiles, cfg.rows, s);
+  if (vals) return spmm_vals_f32_batch(entries, off, count, total_tiles, cfg.rows, s);
 #define BWS_VB(WV, RP, KS)                                        \
   if (cfg.waves == WV && cfg.rows == WV * RP && cfg.kstage == KS) \
-    return launch_rows2_batch<WV, RP, KS>(entries, slot_off, count, total_tiles, s);
+    return launch_rows2_batch<WV, RP, KS>(entries, off, count, total_tiles, s);
   BWS_VB(8, 32, 64)
   BWS_VB(16, 16, 64)
   BWS_VB(16, 16, 32)

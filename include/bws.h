@@ -518,14 +518,14 @@ bws_status bws_sddmm(const bws_bitmap* A, const void* dC, const void* B, int32_t
  * inside graph capture) validates the HOST array `problems`, picks each
  * problem's tile configuration (the plan's, or the autotuner's cached choice
  * for the problem's shape class, or the default), and writes the device
- * problem table and slot offsets into `workspace` on `stream` (after the work
+ * problem table and tile offsets into `workspace` on `stream` (after the work
  * already queued there, which may still use that memory; prepare returns
  * when the copies are done).  bws_batch_run enqueues the
  * launches on `stream` and is capturable into a hipGraph; the workspace must
  * stay untouched between the two.  Workgroups find their problem by a binary
- * search over the slot offsets, every XCD taking an eighth of each problem's
- * tiles, so problems of very different sizes share a
- * launch without padding. */
+ * search over the tile offsets (in launches of many tiles every XCD takes an
+ * eighth of each problem's, in others a range of the launch's), so problems of very
+ * different sizes share a launch without padding. */
 typedef struct {
   bws_bitmap A;      /* M x K                                     */
   const void* B;     /* K x N, dtype of the launch                */
@@ -558,7 +558,7 @@ typedef struct {
   int32_t precision;
   int32_t n_launch;
   bws_batch_launch launch[BWS_BATCH_MAX_LAUNCH];
-  void* workspace;                /* device problem table and slot offsets          */
+  void* workspace;                /* device problem table and tile offsets          */
   const bws_problem* problems;    /* the caller's array; kind 3 launches read it at run
                                      time, so it must outlive the batch             */
   bws_plan plan;                  /* the plan given to prepare (kernel 0 = none)    */
