@@ -73,7 +73,7 @@ struct MfmaTile {
 bool dma_ok(int32_t precision, int32_t b_dtype, const void* B, int64_t ldb, int64_t N);
 MfmaTile mfma_tile_for(const bws_plan* plan, int32_t precision, int32_t b_dtype, int64_t M,
                        int64_t N);
-void mfma_auto_tile(MfmaTile& t, int64_t t64, int64_t t256);
+void mfma_auto_tile(MfmaTile& t, int64_t t64, int64_t t128, int64_t t256);
 bool mfma_tile_valid(int bm, int bn);
 
 // One problem of a grouped launch, as the kernels read it from the workspace.

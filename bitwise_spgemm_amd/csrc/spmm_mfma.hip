@@ -665,7 +665,7 @@ bool dma_ok(int32_t precision, int32_t b_dtype, const void* B, int64_t ldb, int6
 }
 
 // The direct-to-LDS tile for an output (or a grouped launch's outputs together)
-// of t64 tiles of 64 x 64 and t256 of 128 x 256: the larger tile when it still
+// of t64 tiles of 64 x 64, t128 of 64 x 128 and t256 of 128 x 256: the larger tile when it still
 // gives about 1.5 workgroups per CU (two fit on a CU), and below that the one that
 // keeps every CU's waves busy.  A K stage is a barrier and a copy's latency
 // whatever the tile, so small outputs want many small workgroups and 128-row
@@ -679,15 +679,18 @@ bool dma_ok(int32_t precision, int32_t b_dtype, const void* B, int64_t ldb, int6
 //   4096² x 512          (t64 512)   34 |  30 |  35 |  54
 //   2048³                (t64 1024)  36 |  28 |  26 |  32
 //   1024 x 4096²         (t64 1024)  62 |  46 |  42 |  55
+//   2048 x 2048 x 2112   (t64 1056)             42 |  37
 //   3000 x 700 x 2000    (t64 1504)  29 |  22 |  24 |  19
 //   4096² x 2048         (t64 2048) 119 |  88 |  80 |  66
+// 64 x 128 up to the 512 tiles that run at once, two on a CU: one more is a second
+// round (1024 to 1280 tiles of 64 x 64: 8 to 20% over 128 x 128 at K 16 to 4096).
 // All take the K steps in the same order: the results are the same bits.
-void mfma_auto_tile(MfmaTile& t, int64_t t64, int64_t t256) {
+void mfma_auto_tile(MfmaTile& t, int64_t t64, int64_t t128, int64_t t256) {
   t.bm = t.bn = 128;
   t.ks = 64;
   if (t256 >= 384) {
     t.bn = 256;
-  } else if (t64 <= 1280) {
+  } else if (t64 <= 768 || t128 <= 512) {
     t.ks = 128;
     t.bm = t64 <= 256 ? 32 : 64;
     t.bn = t64 <= 768 ? 64 : 128;
@@ -712,7 +715,8 @@ MfmaTile mfma_tile_for(const bws_plan* plan, int32_t precision, int32_t b_dtype,
   int bn = plan && plan->kernel == 2 ? plan->cols_per_wg : 0;
   if (bm == 0 || bn == 0) {
     MfmaTile best;
-    mfma_auto_tile(best, ceil_div(M, 64) * ceil_div(N, 64), ceil_div(M, 128) * ceil_div(N, 256));
+    mfma_auto_tile(best, ceil_div(M, 64) * ceil_div(N, 64), ceil_div(M, 64) * ceil_div(N, 128),
+                   ceil_div(M, 128) * ceil_div(N, 256));
     // the small tiles exist with direct-to-LDS staging in two stages only
     if (best.bm < 128 && (!t.dma || t.nbuf != 2)) best.bm = best.bn = 128;
     if (best.bm < 128) t.ks = best.ks;
