@@ -267,7 +267,7 @@ struct GroupTab {
 };
 
 // One output tile; the tile index is column-block-major within the problem.
-template <int WAVES, int RPW, int KS, bool GRP = false>
+template <int WAVES, int RPW, int KS, bool VALS, bool GRP = false>
 __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64_t M, int64_t K,
                                            int64_t ldw, const int64_t* __restrict__ row_ptr,
                                            const float* __restrict__ values,
@@ -276,6 +276,7 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
                                            float beta, int64_t tile, int64_t row_blocks,
                                            GroupTab gt = GroupTab{nullptr, nullptr, 1, 1}) {
   static_assert(KS == 32 || KS == 64, "stage is one or two bitmap words");
+  static_assert(VALS || !GRP, "grouped values walk like values");
   constexpr int WPS = KS / 32;  // bitmap words per stage
   __shared__ float4 sB0[KS][64];
   __shared__ float4 sB1[KS][64];
@@ -323,10 +324,10 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
     return ((((uint64_t)w_hi) << 32) | w_lo) & smask;
   };
 
-  int64_t e_l = 0;         // GRP: lane l < RPW: value offset of row l at the current stage
-  int cnt_cur = 0;         // GRP: set bits of row l in the current stage
-  float vv[GRP ? RPW : 1];
-  if (GRP && values) e_l = row_lane ? row_ptr[mw + rl] : 0;
+  int64_t e_l = 0;         // VALS: lane l < RPW: value offset of row l at the current stage
+  int cnt_cur = 0;         // VALS: set bits of row l in the current stage
+  float vv[VALS ? RPW : 1];
+  if (VALS && (!GRP || values)) e_l = row_lane ? row_ptr[mw + rl] : 0;
   // GRP: lane p's value is that of stage column p of row r (zero when the bit
   // is clear), so the walk reads it by column, not by rank; tbase[r] is the
   // group-table tile index of row r's word 0
@@ -336,7 +337,7 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
     const int64_t row = mw + r < M ? mw + r : M - 1;
     tbase[r] = GRP ? (row / gt.T) * wpr : 0;
   }
-  auto grp_values = [&](float (&dst)[GRP ? RPW : 1], uint32_t words, int64_t st, int64_t e_row) {
+  auto grp_values = [&](float (&dst)[VALS ? RPW : 1], uint32_t words, int64_t st, int64_t e_row) {
     const uint64_t sm = stage_mask(st);
     const int p = lane;
     const int64_t wp = WPS * st + (p >> 5);
@@ -363,16 +364,25 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
           v = 1.0f;
         }
       }
-      dst[GRP ? r : 0] = v;
+      dst[VALS ? r : 0] = v;
     }
   };
 
   issue(0, base0);
   uint32_t wcur = load_words(0);
   uint32_t wnext = load_words(1);
-  if (GRP) {
+  if (VALS) {
     cnt_cur = __popcll(lane_row_mask(wcur, stage_mask(0)));
-    grp_values(vv, wcur, 0, e_l);
+    if (GRP) {
+      grp_values(vv, wcur, 0, e_l);
+    } else {
+#pragma unroll
+      for (int r = 0; r < RPW; ++r) {
+        const int64_t e = readlane_i64(e_l, r);
+        const int c = __builtin_amdgcn_readlane(cnt_cur, r);
+        vv[r] = lane < c ? values[e + lane] : 0.0f;
+      }
+    }
   }
 
   auto stage = [&](int64_t st, float4 (*cur)[64], uint32_t nxt_base) {
@@ -381,21 +391,30 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
     // re-defining them through an empty asm statement tells the compiler so,
     // which keeps it from waiting (vmcnt(0)) on the prefetch issued next.
     asm volatile("" : "+v"(wcur), "+v"(wnext));
-    if (GRP) {
+    if (VALS) {
 #pragma unroll
-      for (int r = 0; r < RPW; ++r) asm volatile("" : "+v"(vv[GRP ? r : 0]));
+      for (int r = 0; r < RPW; ++r) asm volatile("" : "+v"(vv[VALS ? r : 0]));
     }
     __syncthreads(); // everyone's; the other buffer is no longer being read
     const bool more = st + 1 < nst;
     if (more) issue(st + 1, nxt_base);
     const uint32_t wn2 = load_words(st + 2);
     const uint64_t smask = stage_mask(st);
-    float vn[GRP ? RPW : 1];
+    float vn[VALS ? RPW : 1];
     int cnt_next = 0;
-    if (GRP) {
+    if (VALS) {
       const int64_t e_next = e_l + cnt_cur;
       cnt_next = more ? __popcll(lane_row_mask(wnext, stage_mask(st + 1))) : 0;
-      grp_values(vn, wnext, st + 1, e_next);
+      if (GRP) {
+        grp_values(vn, wnext, st + 1, e_next);
+      } else {
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
+          const int64_t e = readlane_i64(e_next, r);
+          const int c = __builtin_amdgcn_readlane(cnt_next, r);
+          vn[r] = lane < c ? values[e + lane] : 0.0f;
+        }
+      }
     }
 
     // every row's stage mask, masked and bit-reversed once in VALU (lane r
@@ -409,6 +428,7 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
       uint64_t m = (((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)rev_hi, r)) << 32) |
                    (uint32_t)__builtin_amdgcn_readlane((int)rev_lo, r);
       int n = __builtin_amdgcn_readlane(cnt_v, r);
+      int j = 0;
       while (n >= 4) {
         int k0, k1, k2, k3;
         take_bit(m, k0);
@@ -417,11 +437,11 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
         take_bit(m, k3);
         const float4 b0 = cur[k0][lane], b1 = cur[k1][lane], b2 = cur[k2][lane],
                      b3 = cur[k3][lane];
-        if (GRP) {
-          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k0), b0);
-          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k1), b1);
-          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k2), b2);
-          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k3), b3);
+        if (VALS) {
+          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k0 : j), b0);
+          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k1 : j + 1), b1);
+          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k2 : j + 2), b2);
+          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k3 : j + 3), b3);
         } else {
           add4(acc[r], b0);
           add4(acc[r], b1);
@@ -429,30 +449,32 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
           add4(acc[r], b3);
         }
         n -= 4;
+        j += 4;
       }
       if (n >= 2) {
         int k0, k1;
         take_bit(m, k0);
         take_bit(m, k1);
         const float4 b0 = cur[k0][lane], b1 = cur[k1][lane];
-        if (GRP) {
-          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k0), b0);
-          fma4(acc[r], readlane_f(vv[GRP ? r : 0], k1), b1);
+        if (VALS) {
+          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k0 : j), b0);
+          fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k1 : j + 1), b1);
         } else {
           add4(acc[r], b0);
           add4(acc[r], b1);
         }
         n -= 2;
+        j += 2;
       }
       if (n) {
         int k0;
         take_bit(m, k0);
         const float4 b0 = cur[k0][lane];
-        if (GRP) fma4(acc[r], readlane_f(vv[GRP ? r : 0], k0), b0);
+        if (VALS) fma4(acc[r], readlane_f(vv[VALS ? r : 0], GRP ? k0 : j), b0);
         else add4(acc[r], b0);
       }
     }
-    if (GRP) {
+    if (VALS) {
       e_l += cnt_cur;
       cnt_cur = cnt_next;
 #pragma unroll
@@ -490,7 +512,7 @@ __device__ __forceinline__ void rows2_tile(const uint32_t* __restrict__ W, int64
   }
 }
 
-template <int WAVES, int RPW, int KS>
+template <int WAVES, int RPW, int KS, bool VALS>
 __global__ void __launch_bounds__(WAVES * 64)
 k_spmm_rows2(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
              const int64_t* __restrict__ row_ptr, const float* __restrict__ values,
@@ -499,7 +521,7 @@ k_spmm_rows2(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
              int64_t per_xcd) {
   const int64_t tile = xcd_tile(blockIdx.x, per_xcd);
   if (tile >= row_blocks * col_blocks) return;
-  rows2_tile<WAVES, RPW, KS>(W, M, K, ldw, row_ptr, values, B, ldb, N, C, ldc, alpha, beta,
+  rows2_tile<WAVES, RPW, KS, VALS>(W, M, K, ldw, row_ptr, values, B, ldb, N, C, ldc, alpha, beta,
                                    tile, row_blocks);
 }
 
@@ -513,7 +535,7 @@ k_spmm_rows2_groups(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_
                     int64_t per_xcd) {
   const int64_t tile = xcd_tile(blockIdx.x, per_xcd);
   if (tile >= row_blocks * col_blocks) return;
-  rows2_tile<WAVES, RPW, KS, true>(W, M, K, ldw, row_ptr, values, B, ldb, N, C, ldc, 1.0f,
+  rows2_tile<WAVES, RPW, KS, true, true>(W, M, K, ldw, row_ptr, values, B, ldb, N, C, ldc, 1.0f,
                                          0.0f, tile, row_blocks, gt);
 }
 
@@ -526,7 +548,7 @@ k_spmm_rows2_batch(const BatchEntry* __restrict__ entries, const int64_t* __rest
   int64_t tile;
   if (!batch_tile(entries, off, count, range, lo, tile)) return;
   const BatchEntry& e = entries[lo];
-  rows2_tile<WAVES, RPW, KS>(e.W, e.M, e.K, e.ldw, e.row_ptr, e.values,
+  rows2_tile<WAVES, RPW, KS, false>(e.W, e.M, e.K, e.ldw, e.row_ptr, e.values,
                                    static_cast<const float*>(e.B), e.ldb, e.N, e.C, e.ldc, 1.0f,
                                    0.0f, tile, e.row_blocks);
 }
@@ -637,7 +659,7 @@ k_sddmm_f32(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
   }
 }
 
-template <int WAVES, int RPW, int KS>
+template <int WAVES, int RPW, int KS, bool VALS>
 bws_status launch_rows2(const bws_bitmap* A, const float* B, int64_t ldb, int64_t N, float* C,
                         int64_t ldc, float alpha, float beta, hipStream_t s) {
   const int64_t row_blocks = ceil_div(A->rows, WAVES * RPW);
@@ -645,7 +667,7 @@ bws_status launch_rows2(const bws_bitmap* A, const float* B, int64_t ldb, int64_
   const int64_t tiles = row_blocks * col_blocks;
   const int64_t per_xcd = ceil_div(tiles, 8);
   if (8 * per_xcd > kMaxGrid) return BWS_ECAPACITY;
-  hipLaunchKernelGGL((k_spmm_rows2<WAVES, RPW, KS>), dim3((unsigned)(8 * per_xcd)),
+  hipLaunchKernelGGL((k_spmm_rows2<WAVES, RPW, KS, VALS>), dim3((unsigned)(8 * per_xcd)),
                      dim3(WAVES * 64), 0, s, A->words, A->rows, A->cols, A->ldw, A->row_ptr,
                      A->values, B, ldb, N, C, ldc, alpha, beta, row_blocks, col_blocks, per_xcd);
   return launch_check();
@@ -735,12 +757,23 @@ bws_status spmm_valu(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_
                    (reinterpret_cast<uintptr_t>(B) % (4 * esz) == 0) &&
                    (reinterpret_cast<uintptr_t>(C) % 16 == 0);
   const float* Bf = static_cast<const float*>(B);
-  if (b_dtype == BWS_DTYPE_F32 && A->values && spmm_vals_ok(A->cols))
+  // Values: the tile of spmm_vals.hip takes 1.7 us more to start than a stage of this
+  // file's kernels, which therefore keep the short K.  us, this file | that, 1% and
+  // 20% density: 1024 x 32 x 1024 5.0 | 6.8, 6.7 | 7.9, x 48 6.1 | 6.8, 8.7 | 8.4, x 64
+  // 6.1 | 6.5, 9.3 | 8.5; rows off 16 bytes 300 x 16 x 301 7.8 | 9.5, 9.4 | 9.6, x 32
+  // 8.8 | 9.4, 11.6 | 10.0; 500 x 32 x 1 4.8 | 6.9, 7.7 | 7.8.  The sums are the same
+  // bits.
+  const bool rows16 = vec && N % 4 == 0 && N >= 4;
+  if (b_dtype == BWS_DTYPE_F32 && A->values && rows16 && A->cols <= 48)
+    return cfg.rows >= 128 ? launch_rows2<16, 8, 64, true>(A, Bf, ldb, N, C, ldc, alpha, beta, s)
+                           : launch_rows2<16, 4, 32, true>(A, Bf, ldb, N, C, ldc, alpha, beta, s);
+  if (b_dtype == BWS_DTYPE_F32 && A->values && (rows16 || A->cols > (N <= 64 ? 32 : 16)) &&
+      spmm_vals_ok(A->cols))
     return spmm_vals_f32(A, Bf, ldb, N, C, ldc, alpha, beta, cfg.rows, s);
-  if (b_dtype == BWS_DTYPE_F32 && vec && N % 4 == 0 && N >= 4 && !A->values) {
+  if (b_dtype == BWS_DTYPE_F32 && rows16 && !A->values) {
 #define BWS_V2(WV, RP, KS)                                        \
   if (cfg.waves == WV && cfg.rows == WV * RP && cfg.kstage == KS) \
-    return launch_rows2<WV, RP, KS>(A, Bf, ldb, N, C, ldc, alpha, beta, s);
+    return launch_rows2<WV, RP, KS, false>(A, Bf, ldb, N, C, ldc, alpha, beta, s);
     BWS_V2(8, 32, 64)
     BWS_V2(16, 16, 64)
     BWS_V2(16, 16, 32)
