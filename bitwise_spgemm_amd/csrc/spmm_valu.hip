@@ -767,7 +767,7 @@ bws_status spmm_valu(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_
   if (b_dtype == BWS_DTYPE_F32 && A->values && rows16 && A->cols <= 48)
     return cfg.rows >= 128 ? launch_rows2<16, 8, 64, true>(A, Bf, ldb, N, C, ldc, alpha, beta, s)
                            : launch_rows2<16, 4, 32, true>(A, Bf, ldb, N, C, ldc, alpha, beta, s);
-  if (b_dtype == BWS_DTYPE_F32 && A->values && (rows16 || A->cols > (N <= 64 ? 32 : 16)) &&
+  if (b_dtype == BWS_DTYPE_F32 && A->values && (rows16 || A->cols > (N <= 256 ? 32 : 16)) &&
       spmm_vals_ok(A->cols))
     return spmm_vals_f32(A, Bf, ldb, N, C, ldc, alpha, beta, cfg.rows, s);
   if (b_dtype == BWS_DTYPE_F32 && rows16 && !A->values) {
