@@ -61,7 +61,7 @@ bool valu_direct_ok(int32_t b_dtype, const void* B, int64_t ldb, int64_t N, cons
 bws_status spmm_mfma(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb, int64_t N,
                      float* C, int64_t ldc, float alpha, float beta, int32_t precision,
                      const bws_plan* plan, int64_t nb, hipStream_t s);
-size_t spmm_pad_workspace(int64_t K, int64_t N, int32_t precision);
+size_t spmm_pad_workspace(int64_t M, int64_t K, int64_t N, int32_t precision);
 bws_status spmm_mfma_padded(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t ldb,
                             int64_t N, float* C, int64_t ldc, float alpha, float beta,
                             int32_t precision, void* workspace, hipStream_t s);
@@ -245,7 +245,7 @@ size_t bws_spmm_best_workspace_size(const bws_bitmap* A, int64_t N, int32_t prec
   if (precision != BWS_PREC_FP32) {
     if (!plan && spmm_direct16_ok(A, precision, N, N)) return 0;
     return plan || N % 8 == 0 ? bws_spmm_workspace_size(A, N, precision, plan)
-                              : spmm_pad_workspace(A->cols, N, precision);
+                              : spmm_pad_workspace(A->rows, A->cols, N, precision);
   }
   if (plan && (plan->kernel != 0 || plan->rows_per_wg != 0))  // (min_bits alone: 16 bits only)
     return bws_spmm_workspace_size(A, N, precision, plan);
@@ -366,7 +366,8 @@ bws_status bws_spmm(const bws_bitmap* A, const void* B, int32_t b_dtype, int64_t
   // them: with room, B once more in 16 bits with padded rows
   if (!A->values && A->cols > 0 && !plan && precision != BWS_PREC_FP32 &&
       (b_dtype == BWS_DTYPE_F32 ? N % 8 != 0 : !dma_ok(precision, b_dtype, B, ldb, N)) &&
-      ws_ok(workspace, workspace_bytes, spmm_pad_workspace(A->cols, N, precision)))
+      spmm_pad_workspace(A->rows, A->cols, N, precision) > 0 &&
+      ws_ok(workspace, workspace_bytes, spmm_pad_workspace(A->rows, A->cols, N, precision)))
     return spmm_mfma_padded(A, B, b_dtype, ldb, N, C, ldc, alpha, beta, precision, workspace,
                             stream);
   // Split-BF16 on a 0/1 A: with room for B's two BF16 planes, split B once and

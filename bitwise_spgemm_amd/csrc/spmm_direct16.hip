@@ -287,12 +287,19 @@ bws_status launch_direct16(const bws_bitmap* A, const void* B, int64_t ldb, int6
 // 6 and 9 us besides.  BF16X2 of up to 512: the other side is a pass that splits B
 // and two products; us, that | this: 200 x 16 x 100 10.4 | 6.6, 500 x 1000 x 300 19.8 |
 // 11.5, 1999 x 3100 x 1000 60.6 | 42.1; at 1024 tiles, 2048 x 256 x 2048, 23.0 | 28.2.
+// Where N is no multiple of 8 a short K goes to the kernel that splits B in
+// registers, one launch too: 1359 x 32 x 1351 (484 tiles) 12.5 | 22.2, K 128 17.3 |
+// 23.0, K 256 27.0 | 24.5; 32000 x 128 x 60 (500) 12.7 | 15.6, K 256 17.0 | 17.0;
+// 1000 x 32 x 1001 (256) 11.9 | 12.7, K 64 13.2 | 12.7, 1000 x 32 x 1004 12.0 | 8.7.
 bool spmm_direct16_ok(const bws_bitmap* A, int32_t precision, int64_t ldb, int64_t N) {
   const int64_t rows = ceil_div(A->rows, 64), cols = ceil_div(N, 64);
-  const int64_t most = precision == BWS_PREC_BF16X2 ? 512
-                       : A->cols < 1280            ? 0
-                       : A->cols < 2048            ? 256
-                                                   : 512;
+  const int64_t most = precision == BWS_PREC_BF16X2
+                           ? (N % 8 == 0 || A->cols >= 256      ? 512
+                              : N % 4 == 0 || A->cols >= 64 ? 256
+                                                            : 128)
+                       : A->cols < 1280 ? 0
+                       : A->cols < 2048 ? 256
+                                        : 512;
   return rows <= most && cols <= most && rows * cols <= most &&
          A->cols < ((int64_t)1 << 31) && ldb < (1 << 24);  // 32-bit steps and offsets
 }

@@ -999,8 +999,20 @@ k_pad_b16(const void* __restrict__ B, int64_t K, int64_t N, int64_t ldb, int64_t
 
 }  // namespace
 
-size_t spmm_pad_workspace(int64_t K, int64_t N, int32_t precision) {
-  return (precision == BWS_PREC_BF16X2 ? 2 : 1) * split_plane_bytes(K, (N + 7) / 8 * 8);
+// Room for B with padded rows, 0 where they do not pay: at BF16X2 a short K, since
+// the second of the two products reads and writes C once more, which the kernel that
+// splits B in registers does not.  us, in registers | padded: 2000 x 1452, K 256
+// 20.7 | 25.0, K 512 31.7 | 30.6; 6000 x 3004, K 128 50 | 121, K 512 113 | 150, K 1024
+// 196 | 188; rows off 16 bytes 3000 x 1351, K 128 34 | 37, K 256 54 | 42; 8191 x 8191,
+// K 256 258 | 371, K 512 448 | 436.  (BF16 and FP16 have one product: faster from
+// K = 8 on, 1500 x 8 x 1451 12.5 | 10.4.)
+size_t spmm_pad_workspace(int64_t M, int64_t K, int64_t N, int32_t precision) {
+  const size_t plane = split_plane_bytes(K, (N + 7) / 8 * 8);
+  if (precision != BWS_PREC_BF16X2) return plane;
+  const int64_t least = N % 4 == 0                                   ? 1024
+                        : ceil_div(M, 64) * ceil_div(N, 64) <= 2304 ? 256
+                                                                    : 512;
+  return K >= least ? 2 * plane : 0;
 }
 
 // The 16-bit precisions for a B whose rows the direct copies cannot take (N or

@@ -383,7 +383,8 @@ typedef struct {
  * of at least 1280, and of up to 512 with 2048, share K out over the waves of a
  * workgroup (the partial sums are added at the end: another summation order than
  * the other MFMA kernels', which a plan selects) and need no workspace; so do
- * BF16X2 outputs of up to 512 such tiles.
+ * BF16X2 outputs of up to 512 such tiles (N % 8 != 0: 256 below K = 256, and 128
+ * below K = 64 where N % 4 != 0).
  * precision/b_dtype combinations: FP32 with F32 (or exact BF16/F16 input);
  * BF16 with BF16 or F32 (rounded to nearest even); FP16 with F16 or F32;
  * BF16X2 with F32.
@@ -418,7 +419,7 @@ size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision
  * and more: for BF16 / FP16 / BF16X2 with N % 8 != 0, room for B in 16 bits with
  * rows of a multiple of 8 columns (also used for a 16-bit B whose rows are off 16
  * bytes; the same bits as without it at BF16 / FP16, at BF16X2 as with the split
- * of N % 8 == 0); at FP32, for outputs of at least 192 tiles of 256 x 256 (N % 4 ==
+ * of N % 8 == 0, from K = 256 to 1024 on by size); at FP32, for outputs of at least 192 tiles of 256 x 256 (N % 4 ==
  * 0) and K of at least 96: room for B split exactly into three BF16 parts (6 bytes
  * per element), so that masks with more than one bit in eight run on the matrix
  * cores (at 4096³ a third of the vector kernel's time at 50% density).  The density

@@ -8,8 +8,8 @@ from _helpers import to_dev
 
 pytestmark = pytest.mark.gpu
 
-# ragged M, K and N; N off 8: the planes' rows are padded
-SHAPES = [(2100, 97, 1352), (2100, 97, 1355), (1990, 300, 1100), (4200, 33, 643), (2049, 130, 1021)]
+# ragged M, K and N; N off 8: the planes' rows are padded (from K = 256, 512 and 1024)
+SHAPES = [(2100, 97, 1352), (2100, 297, 1355), (1990, 1024, 1100), (4200, 257, 643), (4099, 513, 2501)]
 
 
 def _product(bws, A, B, C, alpha, beta, ws):
@@ -59,3 +59,17 @@ def test_two_passes_round_once(bws, dev, M, K, N):
     R = bws.unpack_bitmap(A).double() @ B
     C = torch.empty((M, N), device=dev)
     assert torch.equal(_product(bws, A, B.float(), C, 1.0, 0.0, _room(bws, A, N, dev)), R.float())
+
+
+@pytest.mark.parametrize("M,K,N", [(1359, 128, 1351), (2000, 512, 1452), (6000, 640, 1004), (3000, 130, 1351),
+                                   (4099, 300, 2501), (1000, 32, 1001)])
+def test_short_k_in_registers(bws, dev, M, K, N):
+    """N off 8 with a short K: no workspace is asked for, and one given is not used
+    (the bits of the kernel that splits in registers, which a plan selects)."""
+    A = bws.Bitmap(to_dev(bws.gen_bitmap_iid(M, M, K, 0.4), dev), M, K)
+    B = torch.randn((K, N), device=dev, generator=torch.Generator(device=dev).manual_seed(N))
+    s = A.struct()
+    assert bws.lib().bws_spmm_best_workspace_size(bws.C.byref(s), N, bws.PRECISION["bf16x2"], None) == 0
+    room = torch.empty(4 * K * (N + 8) + 4096, dtype=torch.uint8, device=dev)
+    C = _product(bws, A, B, torch.empty((M, N), device=dev), 1.0, 0.0, room)
+    assert torch.equal(C, bws.spmm(A, B, "bf16x2", plan=bws.make_plan(2)))
