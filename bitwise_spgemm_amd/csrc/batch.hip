@@ -200,15 +200,14 @@ bws_status bws_batch_prepare(const bws_problem* problems, int32_t count, int32_t
 
   std::vector<Choice> choice((size_t)count);
   std::vector<int> order;
-  int64_t t64 = 0, t128 = 0, t256 = 0;  // 64 x 64, 64 x 128 and 128 x 256 tiles of the whole batch
+  int64_t t64 = 0, t256 = 0;  // 64 x 64 and 128 x 256 tiles of the whole batch
   for (int32_t i = 0; i < count; ++i) {
     BWS_TRY(validate_problem(problems[i], b_dtype));
     t64 += ceil_div(problems[i].A.rows, 64) * ceil_div(problems[i].N, 64);
-    t128 += ceil_div(problems[i].A.rows, 64) * ceil_div(problems[i].N, 128);
     t256 += ceil_div(problems[i].A.rows, 128) * ceil_div(problems[i].N, 256);
   }
   MfmaTile together;
-  mfma_auto_tile(together, t64, t128, t256);
+  mfma_auto_tile(together, t64, t256, t64 <= 1280);
   for (int32_t i = 0; i < count; ++i) {
     if (problems[i].A.rows == 0 || problems[i].N == 0) continue;
     choice[(size_t)i] = classify(problems[i], b_dtype, precision, plan, together);

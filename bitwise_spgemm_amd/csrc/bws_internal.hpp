@@ -73,7 +73,7 @@ struct MfmaTile {
 bool dma_ok(int32_t precision, int32_t b_dtype, const void* B, int64_t ldb, int64_t N);
 MfmaTile mfma_tile_for(const bws_plan* plan, int32_t precision, int32_t b_dtype, int64_t M,
                        int64_t N);
-void mfma_auto_tile(MfmaTile& t, int64_t t64, int64_t t128, int64_t t256);
+void mfma_auto_tile(MfmaTile& t, int64_t t64, int64_t t256, bool mid);
 bool mfma_tile_valid(int bm, int bn);
 
 // One problem of a grouped launch, as the kernels read it from the workspace.
@@ -222,7 +222,7 @@ __device__ __forceinline__ T wave_incl_scan(T v) {
 
 // Grouped launches: workgroup b runs on XCD b % 8.
 //
-// Shares (range == 0): the workgroup takes
+// Shares (RANGE false): the workgroup takes
 // slot b / 8 of its XCD.  Every problem gives each XCD an eighth of its tiles (a
 // contiguous range of the column-block-major order, so an XCD's L2 holds few
 // panels of B); off[i] is the first slot of problem i, off[i + 1] - off[i] the
@@ -238,11 +238,13 @@ __device__ __forceinline__ T wave_incl_scan(T v) {
 // N = 100 114 | 93, 8 of 256 to 4096, N = 64 (70) 127 | 96; BF16, 64 of 64 to 512,
 // N = 1000 (504) 31 | 26.  Beyond that shares win: 16 of 100 to 1000, N = 1000 (440)
 // 45 | 56, split BF16, 32 of 256 to 4096, N = 8 (430) 138 | 218.
+// (Two kernels: one that decides at run time starts 0.3 us later.)
+template <bool RANGE>
 __device__ __forceinline__ bool batch_tile(const BatchEntry* __restrict__ entries,
                                            const int64_t* __restrict__ off, int count,
                                            int64_t range, int& problem, int64_t& tile) {
   const int64_t slot = blockIdx.x >> 3;
-  const int64_t at = range ? (blockIdx.x & 7) * range + slot : slot;
+  const int64_t at = RANGE ? (blockIdx.x & 7) * range + slot : slot;
   if (at >= off[count]) return false;
   int lo = 0, hi = count;
   while (hi - lo > 1) {
@@ -251,7 +253,7 @@ __device__ __forceinline__ bool batch_tile(const BatchEntry* __restrict__ entrie
     else hi = mid;
   }
   problem = lo;
-  if (range) {
+  if constexpr (RANGE) {
     tile = at - off[lo];
     return true;
   }

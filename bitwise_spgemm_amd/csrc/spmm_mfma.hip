@@ -454,13 +454,13 @@ k_spmm_mfma4(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
                                      row_blocks, nb);
 }
 
-template <int PREC, int WM, int WN, int NBUF, int KS>
+template <int PREC, int WM, int WN, int NBUF, int KS, bool RANGE>
 __global__ void __launch_bounds__(256, 2)
 k_spmm_mfma4_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ off,
                    int count, int64_t range) {
   int lo;
   int64_t tile;
-  if (!batch_tile(entries, off, count, range, lo, tile)) return;
+  if (!batch_tile<RANGE>(entries, off, count, range, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   mfma4_tile<PREC, WM, WN, NBUF, KS>(e.W, e.M, e.K, e.ldw, static_cast<const uint16_t*>(e.B),
                                      e.ldb, e.N, e.C, e.ldc, 1.0f, 0.0f, tile,
@@ -479,13 +479,13 @@ k_spmm_mfma3(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
                                vec);
 }
 
-template <int PREC, int TB, int WM, int WN>
+template <int PREC, int TB, int WM, int WN, bool RANGE>
 __global__ void __launch_bounds__(256, 2)
 k_spmm_mfma3_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ off,
                    int count, int64_t range, int vec) {
   int lo;
   int64_t tile;
-  if (!batch_tile(entries, off, count, range, lo, tile)) return;
+  if (!batch_tile<RANGE>(entries, off, count, range, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   mfma3_tile<PREC, TB, WM, WN>(e.W, e.M, e.K, e.ldw, e.B, e.ldb, e.N, e.C, e.ldc, 1.0f, 0.0f,
                                tile, e.row_blocks, vec);
@@ -602,8 +602,12 @@ bws_status launch_mfma_cfg(const MfmaTile& t, const bws_bitmap* A, const void* B
 template <int PREC, int TB, int WM, int WN>
 void launch_mfma3_batch(dim3 grid, const BatchEntry* entries, const int64_t* off, int count,
                         int64_t range, int vec, hipStream_t s) {
-  hipLaunchKernelGGL((k_spmm_mfma3_batch<PREC, TB, WM, WN>), grid, dim3(256), 0, s, entries,
-                     off, count, range, vec);
+  if (range)
+    hipLaunchKernelGGL((k_spmm_mfma3_batch<PREC, TB, WM, WN, true>), grid, dim3(256), 0, s,
+                       entries, off, count, range, vec);
+  else
+    hipLaunchKernelGGL((k_spmm_mfma3_batch<PREC, TB, WM, WN, false>), grid, dim3(256), 0, s,
+                       entries, off, count, range, vec);
 }
 
 template <int PREC, int TB>
@@ -617,24 +621,22 @@ bws_status launch_mfma_batch(const BatchEntry* entries, const int64_t* off, int 
   bool done = false;
   if constexpr (TB != 0 && PREC != 3) {
     if (t.dma) {
-      if (t.bm == 32)
-        hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 16, 32, 2, 128>), grid, dim3(256), 0, s,
-                           entries, off, count, range);
-      else if (t.bm == 64 && t.bn == 64)
-        hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 32, 32, 2, 128>), grid, dim3(256), 0, s,
-                           entries, off, count, range);
-      else if (t.bm == 64)
-        hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 32, 64, 2, 128>), grid, dim3(256), 0, s,
-                           entries, off, count, range);
-      else if (t.bn == 256)
-        hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 64, 128, 2, 64>), grid, dim3(256), 0, s,
-                           entries, off, count, range);
-      else if (t.bm == 256)
-        hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 128, 64, 2, 64>), grid, dim3(256), 0, s,
-                           entries, off, count, range);
-      else
-        hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, 64, 64, 2, 64>), grid, dim3(256), 0, s,
-                           entries, off, count, range);
+#define BWS_B4(WM, WN, KS)                                                                       \
+  do {                                                                                           \
+    if (range)                                                                                   \
+      hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, WM, WN, 2, KS, true>), grid, dim3(256), 0, s, \
+                         entries, off, count, range);                                            \
+    else                                                                                         \
+      hipLaunchKernelGGL((k_spmm_mfma4_batch<PREC, WM, WN, 2, KS, false>), grid, dim3(256), 0,   \
+                         s, entries, off, count, range);                                         \
+  } while (0)
+      if (t.bm == 32) BWS_B4(16, 32, 128);
+      else if (t.bm == 64 && t.bn == 64) BWS_B4(32, 32, 128);
+      else if (t.bm == 64) BWS_B4(32, 64, 128);
+      else if (t.bn == 256) BWS_B4(64, 128, 64);
+      else if (t.bm == 256) BWS_B4(128, 64, 64);
+      else BWS_B4(64, 64, 64);
+#undef BWS_B4
       return launch_check();
     }
   }
@@ -665,7 +667,7 @@ bool dma_ok(int32_t precision, int32_t b_dtype, const void* B, int64_t ldb, int6
 }
 
 // The direct-to-LDS tile for an output (or a grouped launch's outputs together)
-// of t64 tiles of 64 x 64, t128 of 64 x 128 and t256 of 128 x 256: the larger tile when it still
+// of t64 tiles of 64 x 64 and t256 of 128 x 256: the larger tile when it still
 // gives about 1.5 workgroups per CU (two fit on a CU), and below that the one that
 // keeps every CU's waves busy.  A K stage is a barrier and a copy's latency
 // whatever the tile, so small outputs want many small workgroups and 128-row
@@ -682,15 +684,18 @@ bool dma_ok(int32_t precision, int32_t b_dtype, const void* B, int64_t ldb, int6
 //   2048 x 2048 x 2112   (t64 1056)             42 |  37
 //   3000 x 700 x 2000    (t64 1504)  29 |  22 |  24 |  19
 //   4096² x 2048         (t64 2048) 119 |  88 |  80 |  66
-// 64 x 128 up to the 512 tiles that run at once, two on a CU: one more is a second
-// round (1024 to 1280 tiles of 64 x 64: 8 to 20% over 128 x 128 at K 16 to 4096).
+// mid: 64 x 128 is still small enough.  For one output that is up to the 512 tiles
+// that run at once, two on a CU: one more is a second round (1024 to 1280 tiles of
+// 64 x 64: 8 to 20% over 128 x 128 at K 16 to 4096).  In a grouped launch the tiles'
+// lengths differ and fill it: up to 1280 tiles of 64 x 64 (17 problems of 256 to 4096
+// rows and columns, N = 128: 43 us against 57 with 128 x 128).
 // All take the K steps in the same order: the results are the same bits.
-void mfma_auto_tile(MfmaTile& t, int64_t t64, int64_t t128, int64_t t256) {
+void mfma_auto_tile(MfmaTile& t, int64_t t64, int64_t t256, bool mid) {
   t.bm = t.bn = 128;
   t.ks = 64;
   if (t256 >= 384) {
     t.bn = 256;
-  } else if (t64 <= 768 || t128 <= 512) {
+  } else if (t64 <= 768 || mid) {
     t.ks = 128;
     t.bm = t64 <= 256 ? 32 : 64;
     t.bn = t64 <= 768 ? 64 : 128;
@@ -715,8 +720,8 @@ MfmaTile mfma_tile_for(const bws_plan* plan, int32_t precision, int32_t b_dtype,
   int bn = plan && plan->kernel == 2 ? plan->cols_per_wg : 0;
   if (bm == 0 || bn == 0) {
     MfmaTile best;
-    mfma_auto_tile(best, ceil_div(M, 64) * ceil_div(N, 64), ceil_div(M, 64) * ceil_div(N, 128),
-                   ceil_div(M, 128) * ceil_div(N, 256));
+    mfma_auto_tile(best, ceil_div(M, 64) * ceil_div(N, 64), ceil_div(M, 128) * ceil_div(N, 256),
+                   ceil_div(M, 64) * ceil_div(N, 128) <= 512);
     // the small tiles exist with direct-to-LDS staging in two stages only
     if (best.bm < 128 && (!t.dma || t.nbuf != 2)) best.bm = best.bn = 128;
     if (best.bm < 128) t.ks = best.ks;

@@ -20,14 +20,14 @@ k_spmm_vals(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
 }
 
 // Grouped launch: a workgroup finds its problem and tile with batch_tile.
-template <int VR>
+template <int VR, bool RANGE>
 __global__ void __launch_bounds__(kVW * 64)
 k_spmm_vals_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ off,
                   int count, int64_t range) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kValsLds];
   int lo;
   int64_t tile;
-  if (!batch_tile(entries, off, count, range, lo, tile)) return;
+  if (!batch_tile<RANGE>(entries, off, count, range, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   vals_tile<VR>(e.W, e.M, e.K, e.ldw, e.row_ptr, e.values, static_cast<const float*>(e.B), e.ldb,
                 e.N, e.C, e.ldc, 1.0f, 0.0f, tile, e.row_blocks, smem);
@@ -83,11 +83,14 @@ bws_status spmm_vals_f32_batch(const BatchEntry* entries, const int64_t* off, in
   const int64_t grid = batch_grid(total_tiles, count, range);
   if (grid > kMaxGrid) return BWS_ECAPACITY;
   if (total_tiles == 0) return BWS_OK;
-  const dim3 g((unsigned)grid), b(kVW * 64);
+  auto launch = [&](auto ranges, auto shares) {
+    hipLaunchKernelGGL(range ? ranges : shares, dim3((unsigned)grid), dim3(kVW * 64), 0, s, entries,
+                       off, count, range);
+  };
   switch (rows) {
-    case 256: hipLaunchKernelGGL(k_spmm_vals_batch<16>, g, b, 0, s, entries, off, count, range); break;
-    case 128: hipLaunchKernelGGL(k_spmm_vals_batch<8>, g, b, 0, s, entries, off, count, range); break;
-    case 64: hipLaunchKernelGGL(k_spmm_vals_batch<4>, g, b, 0, s, entries, off, count, range); break;
+    case 256: launch(k_spmm_vals_batch<16, true>, k_spmm_vals_batch<16, false>); break;
+    case 128: launch(k_spmm_vals_batch<8, true>, k_spmm_vals_batch<8, false>); break;
+    case 64: launch(k_spmm_vals_batch<4, true>, k_spmm_vals_batch<4, false>); break;
     default: return BWS_EINVAL;
   }
   return launch_check();

@@ -540,13 +540,13 @@ k_spmm_rows2_groups(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_
 }
 
 // Grouped launch: a workgroup finds its problem and tile with batch_tile.
-template <int WAVES, int RPW, int KS>
+template <int WAVES, int RPW, int KS, bool RANGE>
 __global__ void __launch_bounds__(WAVES * 64)
 k_spmm_rows2_batch(const BatchEntry* __restrict__ entries, const int64_t* __restrict__ off,
                    int count, int64_t range) {
   int lo;
   int64_t tile;
-  if (!batch_tile(entries, off, count, range, lo, tile)) return;
+  if (!batch_tile<RANGE>(entries, off, count, range, lo, tile)) return;
   const BatchEntry& e = entries[lo];
   rows2_tile<WAVES, RPW, KS, false>(e.W, e.M, e.K, e.ldw, e.row_ptr, e.values,
                                    static_cast<const float*>(e.B), e.ldb, e.N, e.C, e.ldc, 1.0f,
@@ -714,8 +714,9 @@ bws_status launch_rows2_batch(const BatchEntry* entries, const int64_t* off, int
   const int64_t grid = batch_grid(total_tiles, count, range);
   if (grid > kMaxGrid) return BWS_ECAPACITY;
   if (total_tiles == 0) return BWS_OK;
-  hipLaunchKernelGGL((k_spmm_rows2_batch<WAVES, RPW, KS>), dim3((unsigned)grid),
-                     dim3(WAVES * 64), 0, s, entries, off, count, range);
+  hipLaunchKernelGGL((range ? k_spmm_rows2_batch<WAVES, RPW, KS, true>
+                            : k_spmm_rows2_batch<WAVES, RPW, KS, false>),
+                     dim3((unsigned)grid), dim3(WAVES * 64), 0, s, entries, off, count, range);
   return launch_check();
 }
 
