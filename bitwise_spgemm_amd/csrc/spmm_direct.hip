@@ -65,91 +65,95 @@ __device__ __forceinline__ bool not_exact(float x, bool any_tiny) {
   return !(m < __builtin_inff()) || (any_tiny && m < kSmallOut);
 }
 
-// The tile's outputs once more as FP32 sums over the set bits, ascending k, as the
-// vector-add kernels form them: sums[x][i] of row 16a + j, a the wave's x-th row
-// tile, column n0 + 8q + i.  112 DW rows of B at a time go through lds (room for
-// 16 KiB DW), a lane walks its row's bits, four in flight.  us with ordinary values
-// in B | an infinity in every column | the vector-add kernels: 1024³, 10%
-// 12 | 41 | 41, 50% 12 | 78 | 94; 2048 x 1024 x 2048, 5% 30 | 104 | 36, 50%
-// 31 | 262 | 96 (two waves for four row tiles each); 3001 x 2053 x 516, 5%
-// 29 | 96 | 63.  Output by output and bit by bit from global memory the second
-// column was 305, 885, 780 and, in the last row, 735.
+// A wave's outputs once more as FP32 sums over the set bits, ascending k, as the
+// vector-add kernels form them: sums[x][i] of row row0 + 16x + j, column n0 + 8q + i.
+// 128 rows of B at a time go through the LDS that held the partial tiles of these
+// rows, which no other wave reads (16 KiB in DW pieces, part_bytes apart; 16-byte
+// units swizzled by the row); a lane walks its row's bits, four in flight.  The waves
+// do it by themselves: a barrier at the kernel's end, good or bad outputs, kept the
+// next workgroup off the CU (703 x 3181 x 3984, 750 tiles, 61 us then 66).  Bound by
+// LDS reads, a row of B per set bit.  Us for ordinary B, for B with an Inf in every
+// column and for the vector-add kernel on that B (output by output it was 305, 885 and
+// 735 at the first, second and fourth):
+//   1024 x 1024 x 1024, 10% of A   12.5   54  41     (50%  12.4  112   94)
+//   2048 x 1024 x 2048,  5%        30    116  36     (50%  31    336   96)
+//   4095 x 2000 x 2047, 10%       115    577 253
+//   256 x 512 x 192,     5%         8.8   25  18
+// Loading the next 128 rows ahead of the sums gave nothing (55 and 113 at the first).
 template <int DW>
 __device__ __forceinline__ void vector_sums(const uint32_t* __restrict__ W, int64_t M, int64_t K,
                                             int64_t ldw, const float* __restrict__ B, int64_t ldb,
-                                            int64_t N, int64_t m0, int64_t n0, float* lds,
-                                            float (&sums)[kDA / DW][8]) {
-  constexpr int kRW = 7 * DW / 2;  // bitmap words of a row at once
-  constexpr int kPitch = kDN + 4;  // floats: B rows start in different banks
-  static_assert(kRW * 32 * kPitch * 4 <= DW * 16384 && kRW * 32 * (kDN / 4) == 14 * DW * 64, "");
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+                                            int64_t N, int64_t row0, int64_t n0, uint8_t* own,
+                                            uint32_t part_bytes, float (&sums)[kDA / DW][8]) {
+  constexpr int NX = kDA / DW;
+  constexpr uint32_t kPieceRows = 16 * NX;
+  static_assert(kPieceRows * DW == 128 && kDN * 4 == 128, "four bitmap words, 128 bytes a row");
+  const int lane = threadIdx.x & 63;
   const int j = lane & 15, q = lane >> 4;
   const int64_t nks = ceil_div(K, 32);
+  auto at = [&](uint32_t k, uint32_t unit) {
+    return reinterpret_cast<f32x4*>(own + (k / kPieceRows) * part_bytes + (k % kPieceRows) * 128u +
+                                    ((unit ^ (k & 7u)) << 4));
+  };
 #pragma unroll
-  for (int x = 0; x < kDA / DW; ++x)
+  for (int x = 0; x < NX; ++x)
 #pragma unroll
     for (int i = 0; i < 8; ++i) sums[x][i] = 0.0f;
-  for (int64_t w0 = 0; w0 < nks; w0 += kRW) {
-    __syncthreads();  // what was there has been read
-    for (int u0 = 0; u0 < 14; u0 += 7) {  // a thread's pieces, seven loads in flight
-      f32x4 v[7];
+  for (int64_t w0 = 0; w0 < nks; w0 += 4) {
+    f32x4 v[16];
+    uint32_t wd[NX][4];
+    const int64_t c = n0 + 4 * (lane & 7);
 #pragma unroll
-      for (int u = 0; u < 7; ++u) {
-        const int i = (u0 + u) * (DW * 64) + threadIdx.x;
-        const int64_t k = 32 * w0 + i / (kDN / 4), c = n0 + i % (kDN / 4) * 4;
-        const float* p = B + (k < K ? k : K - 1) * ldb;
-        if (c + 4 <= N) {
-          v[u] = *reinterpret_cast<const f32x4_u*>(p + c);
-        } else {
+    for (int u = 0; u < 16; ++u) {
+      const int64_t k = 32 * w0 + 8 * u + (lane >> 3);
+      const float* p = B + (k < K ? k : K - 1) * ldb;
+      if (c + 4 <= N) {
+        v[u] = *reinterpret_cast<const f32x4_u*>(p + c);
+      } else {
 #pragma unroll
-          for (int t = 0; t < 4; ++t) v[u][t] = p[c + t < N ? c + t : N - 1];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 7; ++u) {
-        const int i = (u0 + u) * (DW * 64) + threadIdx.x;
-        *reinterpret_cast<f32x4*>(lds + i / (kDN / 4) * kPitch + i % (kDN / 4) * 4) = v[u];
+        for (int t = 0; t < 4; ++t) v[u][t] = p[c + t < N ? c + t : N - 1];
       }
     }
-    __syncthreads();
-    const int nw = (int)(nks - w0 < kRW ? nks - w0 : kRW);
 #pragma unroll
-    for (int x = 0; x < kDA / DW; ++x) {
-      const int64_t row = m0 + 16 * (wave * (kDA / DW) + x) + j;
+    for (int x = 0; x < NX; ++x) {
+      const int64_t row = row0 + 16 * x + j;
       const uint32_t* wp = W + (row < M ? row : M - 1) * ldw + w0;
-      for (int i0 = 0; i0 < nw; i0 += 8) {
-        uint32_t wd[8];
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
-          wd[t] = i0 + t < nw ? wp[i0 + t] & valid_bits(w0 + i0 + t, K) : 0u;
+      for (int t = 0; t < 4; ++t) wd[x][t] = w0 + t < nks ? wp[t] & valid_bits(w0 + t, K) : 0u;
+    }
+    asm volatile("" ::: "memory");  // (a wave's LDS accesses stay in order)
 #pragma unroll
-        for (int t = 0; t < 8; t += 2) {
-          uint64_t m = ((uint64_t)wd[t] << 32) | wd[t + 1];
-          const float* b = lds + 32 * (i0 + t) * kPitch + 8 * q;
-          while (m) {
-            f32x4 v[4][2];
-            bool on[4];
-            int k = 0;
+    for (int u = 0; u < 16; ++u) *at(8 * u + (lane >> 3), lane & 7) = v[u];
+    asm volatile("" ::: "memory");
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {  // past the last bit: its row again, not added
-              on[e] = m != 0ull;
-              if (on[e]) {
-                k = __clzll((long long)m);
-                m &= ~(1ull << (63 - k));
-              }
-              v[e][0] = *reinterpret_cast<const f32x4*>(b + k * kPitch);
-              v[e][1] = *reinterpret_cast<const f32x4*>(b + k * kPitch + 4);
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+      for (int t = 0; t < 4; t += 2) {
+        uint64_t m = ((uint64_t)wd[x][t] << 32) | wd[x][t + 1];
+        while (m) {
+          f32x4 b[4][2];
+          bool on[4];
+          uint32_t k = 0;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {  // past the last bit: its row again, not added
+            on[e] = m != 0ull;
+            if (on[e]) {
+              const int z = __clzll((long long)m);
+              m &= ~(1ull << (63 - z));
+              k = 32u * t + (uint32_t)z;
             }
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (on[e]) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) sums[x][i] += v[e][i >> 2][i & 3];
-              }
+            b[e][0] = *at(k, 2 * q);
+            b[e][1] = *at(k, 2 * q + 1);
           }
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (on[e]) {
+#pragma unroll
+              for (int i = 0; i < 8; ++i) sums[x][i] += b[e][i >> 2][i & 3];
+            }
         }
       }
-    }
+    asm volatile("" ::: "memory");
   }
 }
 
@@ -162,7 +166,7 @@ k_spmm_direct(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
   constexpr int kDW = 32 * DW;  // bitmap words of a row in LDS at once,
   __shared__ f32x4 part[DW][kDA * kDB][64];  // in the room of the partial tiles
   static_assert(kDW * kDM * 4 == sizeof(part), "");
-  __shared__ uint32_t tiny[DW], redo[DW];
+  __shared__ uint32_t tiny[DW];
   uint32_t(*const words)[kDM] = reinterpret_cast<uint32_t(*)[kDM]>(&part[0][0][0]);
   const int64_t tile = xcd_tile(blockIdx.x, per_xcd);
   if (tile >= row_blocks * col_blocks) return;
@@ -355,15 +359,10 @@ k_spmm_direct(const uint32_t* __restrict__ W, int64_t M, int64_t K, int64_t ldw,
     }
     any_bad |= bad[x];
   }
-  const uint64_t waiting = __ballot(any_bad != 0u);
-  if (lane == 0) redo[wave] = waiting != 0ull ? 1u : 0u;
-  __syncthreads();
-  any_bad = 0u;
-#pragma unroll
-  for (int w = 0; w < DW; ++w) any_bad |= redo[w];
-  if (any_bad == 0u) return;  // the same for the whole workgroup
+  if (__ballot(any_bad != 0u) == 0ull) return;  // (of this wave)
   float again[NX][8];
-  vector_sums<DW>(W, M, K, ldw, B, ldb, N, m0, n0, reinterpret_cast<float*>(&part[0][0][0]), again);
+  vector_sums<DW>(W, M, K, ldw, B, ldb, N, m0 + 16 * NX * wave, n0,
+                  reinterpret_cast<uint8_t*>(&part[0][wave * NX * kDB][0]), sizeof(part[0]), again);
 #pragma unroll
   for (int x = 0; x < NX; ++x) {
     float* c = C + (m0 + 16 * (wave * NX + x) + j) * ldc + n0 + 8 * q;

@@ -378,7 +378,8 @@ typedef struct {
  * exactly into three BF16 parts and every product and sum in FP32.
  * Outputs that meet an infinity or a NaN, overflow, or are below 2^-80 beside
  * b below 2^-100, are summed by vector adds in ascending k instead: the tiles of
- * 128 x 32 that hold one take up to about three times the vector kernel's time.
+ * 128 x 32 that hold one take up to about three and a half times the vector
+ * kernel's time.
  * BF16 / FP16 with a 0/1 A and no plan: outputs of up to 256 tiles of 64 x 64 with K
  * of at least 1280, and of up to 512 with 2048, share K out over the waves of a
  * workgroup (the partial sums are added at the end: another summation order than
