@@ -52,7 +52,9 @@ bool spmm_vals_ok(int64_t K) { return K <= kValsMaxK; }
 // Rows per workgroup of the value product's tile.  A workgroup has a CU to itself,
 // so the time is the number of rounds over 256 CUs times a tile's: 143, 242 and
 // 421 us for 64, 128 and 256 rows at K = 4096 and 10% density (80, 120, 189 at 1%;
-// 394, 735, 1412 at 50%), of which 100 us do not depend on the rows.
+// 394, 735, 1412 at 50%), of which 100 us do not depend on the rows.  The 256-row
+// form keeps 28 bytes a lane in scratch (16 waves leave a lane 128 registers, 64 of
+// them sums); the other two keep none.
 int32_t spmm_vals_rows(int64_t M, int64_t N) {
   static const int32_t rows[3] = {256, 128, 64}, cost[3] = {26, 15, 9};
   int32_t best = 0;

@@ -373,9 +373,10 @@ typedef struct {
 /* C = alpha * (A · B) + beta * C, A M x K bitmap, B K x N dense (dtype b_dtype,
  * leading dimension ldb), C M x N FP32.  beta == 0 never reads C.
  * FP32 with a 0/1 A, an F32 B and no plan: outputs of up to 256, 512 and 1024 tiles
- * of 64 x 64 with K of at least 160, 256 and 1024 (larger ones and K from 128 too
- * where rows of B or C are off 16 bytes) run on the matrix cores without a workspace, each b split
- * exactly into three BF16 parts and every product and sum in FP32.
+ * of 64 x 64 with K of at least 160, 256 and 1024 (where rows of B or C are
+ * off 16 bytes: up to 256 with 128, 2304 with 192 and any number with 1024) run on
+ * the matrix cores without a workspace, each b split exactly into three BF16 parts
+ * and every product and sum in FP32.
  * Outputs that meet an infinity or a NaN, overflow, or are below 2^-80 beside
  * b below 2^-100, are summed by vector adds in ascending k instead: the tiles of
  * 128 x 32 that hold one take up to about three and a half times the vector
@@ -420,9 +421,9 @@ size_t bws_spmm_workspace_size(const bws_bitmap* A, int64_t N, int32_t precision
  * and more: for BF16 / FP16 / BF16X2 with N % 8 != 0, room for B in 16 bits with
  * rows of a multiple of 8 columns (also used for a 16-bit B whose rows are off 16
  * bytes; the same bits as without it at BF16 / FP16, at BF16X2 as with the split
- * of N % 8 == 0, from K = 256 to 1024 on by size); at FP32, for outputs of at least 192 tiles of 256 x 256 (N % 4 ==
- * 0) and K of at least 96: room for B split exactly into three BF16 parts (6 bytes
- * per element), so that masks with more than one bit in eight run on the matrix
+ * of N % 8 == 0, from K = 256 to 1024 on by size); at FP32, for outputs of at least
+ * 192 tiles of 256 x 256 (N % 4 == 0) and K of at least 96: room for B split exactly
+ * into three BF16 parts (6 bytes per element), so that masks with more than one bit in eight run on the matrix
  * cores (at 4096³ a third of the vector kernel's time at 50% density).  The density
  * is estimated from a fixed sample of A's words on the device: the same A always
  * takes the same kernel.  256-column blocks of B that hold an infinity, a NaN, a
